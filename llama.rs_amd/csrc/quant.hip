@@ -178,42 +178,140 @@ hipError_t launch_generate(WeightView w, uint8_t *q, uint64_t seed, int mode, fl
 // ---------------------------------------------------------------------------
 // dequant (bit-exact with dequant.rs)
 // ---------------------------------------------------------------------------
-__global__ void k_dequant(WeightView w, float *__restrict__ out) {
-    const uint32_t be = (uint32_t)block_elems(w.type);
-    const uint64_t n = (uint64_t)w.n_out * w.n_in;
-    for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n;
-         i += (uint64_t)gridDim.x * blockDim.x)
-        out[i] = deq_elem(w, i / be, (uint32_t)(i % be));
+// One wavefront turns 256 consecutive elements of a row (a super-block, or four
+// Q8_0 units) into one contiguous KB of f32: lane l makes elements 4 l .. 4 l + 3
+// from one word of quants (two for Q5_K / Q6_K) and the run's scale bytes, which
+// the lanes of a run share.  Bound by the f32 written; a thread per element that
+// looked every byte up through toff took 640 us for a 5120 x 5120 Q5_K weight,
+// this 29.4 us (123 MB moved, 4.2 TB/s; a
+// large copy reaches 4.9 TB/s).
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+
+__device__ __forceinline__ uint32_t ld32(const uint8_t *p) { return *reinterpret_cast<const uint32_t *>(p); }
+__device__ __forceinline__ uint32_t ld16(const uint8_t *p) { return *reinterpret_cast<const uint16_t *>(p); }
+
+// elements 4 l .. 4 l + 3 of super-block u (Q8_0: of the 256 elements from 256 u) of row `row`
+template <uint32_t T>
+__device__ __forceinline__ f32x4 deq4(const WeightView &w, uint32_t row, uint32_t u, uint32_t l) {
+    const uint32_t r = row % TILE_ROWS, e = 4 * l;
+    const uint8_t *tile = w.q + (size_t)(row / TILE_ROWS) * tunits(T, w.n_in) * tchunk_bytes(T);
+    f32x4 v;
+    if constexpr (T == T_Q8_0) {
+        const uint8_t *c = tile + (size_t)(4 * u + (e >> 6)) * tchunk_bytes(T);
+        const uint32_t b = (e >> 5) & 1, q = ld32(c + 16 * (16 * (2 * b + ((e >> 4) & 1)) + r) + (e & 15));
+        const float d = h2f((uint16_t)ld16(c + 1024 + 4 * r + 2 * b));
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[i] = __fmul_rn((float)(int8_t)((q >> (8 * i)) & 0xFF), d);
+    } else if constexpr (T == T_Q4_K || T == T_Q5_K) {
+        constexpr uint32_t QS = T == T_Q4_K ? 256 : 768;
+        const uint8_t *c = tile + (size_t)u * tchunk_bytes(T);
+        const uint32_t j = e >> 6, hi = (e >> 5) & 1, sub = 2 * j + hi, x = e & 31;
+        uint32_t q = (ld32(c + QS + 1024 * (j >> 1) + 16 * (16 * (2 * (j & 1) + (x >> 4)) + r) + (x & 15)) >> (4 * hi)) &
+                     0x0F0F0F0Fu;
+        if constexpr (T == T_Q5_K)
+            q |= ((ld32(c + 256 + 16 * (16 * (x >> 4) + r) + (x & 15)) >> sub) & 0x01010101u) << 4;
+        const uint32_t h = ld32(c + 16 * r), s0 = ld32(c + 16 * r + 4), s1 = ld32(c + 16 * r + 8),
+                       s2 = ld32(c + 16 * r + 12), sh = 8 * (sub & 3);
+        const uint32_t a = (s0 >> sh) & 0xFF, m = (s1 >> sh) & 0xFF, x2 = (s2 >> sh) & 0xFF;
+        const uint32_t sc = sub < 4 ? a & 63 : (x2 & 0xF) | ((a >> 6) << 4);
+        const uint32_t mn = sub < 4 ? m & 63 : (x2 >> 4) | ((m >> 6) << 4);
+        const float d1 = __fmul_rn(h2f((uint16_t)(h & 0xFFFF)), (float)sc);
+        const float m1 = __fmul_rn(h2f((uint16_t)(h >> 16)), (float)mn);
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[i] = __fsub_rn(__fmul_rn(d1, (float)((q >> (8 * i)) & 0xFF)), m1);
+    } else {  // T_Q6_K
+        const uint8_t *c = tile + (size_t)u * tchunk_bytes(T);
+        const uint32_t half = e >> 7, quarter = (e >> 5) & 3, x = e & 31, pc = 16 * (16 * (2 * half + (x >> 4)) + r) + (x & 15);
+        const uint32_t lo = (ld32(c + 256 + 1024 * (quarter & 1) + pc) >> (4 * (quarter >> 1))) & 0x0F0F0F0Fu;
+        const uint32_t q = lo | (((ld32(c + 2304 + pc) >> (2 * quarter)) & 0x03030303u) << 4);
+        const float s = (float)(int8_t)c[16 * r + 8 * half + (x >> 4) + 2 * quarter];
+        const float ds = __fmul_rn(h2f((uint16_t)ld16(c + 3328 + 2 * r)), s);
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[i] = __fmul_rn(ds, (float)((int)((q >> (8 * i)) & 0xFF) - 32));
+    }
+    return v;
 }
 
-// rows_dev[r] selects a row; out is [n_rows * n_in] (embedding lookup,
-// ops.rs:11-26 on the dequantized table, done one row at a time)
-__global__ void k_dequant_rows(WeightView w, const uint32_t *__restrict__ rows, uint32_t n_rows,
-                               float *__restrict__ out) {
+// VEC: `out` is 16-byte aligned (rows are whole blocks, so every store is)
+template <bool VEC>
+__device__ __forceinline__ void put4(float *__restrict__ o, f32x4 v) {
+    if constexpr (VEC)
+        *reinterpret_cast<f32x4 *>(o) = v;
+    else
+        for (int i = 0; i < 4; i++) o[i] = v[i];
+}
+
+// workgroup = 256 elements of the 16 rows of a tile, a wavefront every fourth row
+template <uint32_t T, bool VEC>
+__global__ __launch_bounds__(256) void k_dequant(WeightView w, uint32_t nu, float *__restrict__ out) {
+    const uint32_t u = blockIdx.x % nu, row0 = blockIdx.x / nu * TILE_ROWS, l = threadIdx.x & 63;
+    if (256 * u + 4 * l >= w.n_in) return;  // Q8_0: the row's last, partial 256 elements
+#pragma unroll
+    for (uint32_t i = 0; i < TILE_ROWS / 4; i++) {
+        const uint32_t row = row0 + 4 * i + (threadIdx.x >> 6);
+        if (row < w.n_out) put4<VEC>(out + (size_t)row * w.n_in + 256 * u + 4 * l, deq4<T>(w, row, u, l));
+    }
+}
+
+// rows[r] selects a row; out is [n_rows][n_in] (embedding lookup, ops.rs:11-26
+// on the dequantized table); workgroup = 1024 elements of one row
+template <uint32_t T, bool VEC>
+__global__ __launch_bounds__(256) void k_dequant_rows(WeightView w, const uint32_t *__restrict__ rows, uint32_t n_rows,
+                                                      uint32_t nq, float *__restrict__ out) {
+    const uint32_t r = blockIdx.x / nq, u = 4 * (blockIdx.x % nq) + (threadIdx.x >> 6), l = threadIdx.x & 63;
+    const uint32_t row = min(rows[r], w.n_out - 1);  // ids are validated on the host
+    if (256 * u + 4 * l < w.n_in) put4<VEC>(out + (size_t)r * w.n_in + 256 * u + 4 * l, deq4<T>(w, row, u, l));
+}
+
+// the types that are kept as GGUF bytes (F32, F16, Q4_0): one element per thread
+__global__ void k_dequant_raw(WeightView w, const uint32_t *__restrict__ rows, uint32_t n_rows,
+                              float *__restrict__ out) {
     const uint32_t be = (uint32_t)block_elems(w.type);
     const uint64_t n = (uint64_t)n_rows * w.n_in;
     for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n;
          i += (uint64_t)gridDim.x * blockDim.x) {
-        uint32_t r = (uint32_t)(i / w.n_in), c = (uint32_t)(i % w.n_in);
-        uint32_t row = rows[r];
-        if (row >= w.n_out) row = w.n_out - 1;  // ids are validated on the host
-        uint64_t e = (uint64_t)row * w.n_in + c;
+        uint64_t e = i;
+        if (rows) e = (uint64_t)min(rows[i / w.n_in], w.n_out - 1) * w.n_in + i % w.n_in;
         out[i] = deq_elem(w, e / be, (uint32_t)(e % be));
     }
 }
 
-hipError_t launch_dequant(WeightView w, float *out, hipStream_t s) {
-    uint64_t n = (uint64_t)w.n_out * w.n_in;
-    hipLaunchKernelGGL(k_dequant, dim3(grid_for(n, 256)), dim3(256), 0, s, w, out);
+// rows null: every row of w
+template <uint32_t T, bool VEC>
+static void start_dequant(const WeightView &w, const uint32_t *rows, uint32_t n_rows, float *out, hipStream_t s) {
+    const uint32_t nu = (w.n_in + 255) / 256;
+    if (rows)
+        hipLaunchKernelGGL((k_dequant_rows<T, VEC>), dim3(n_rows * ((nu + 3) / 4)), dim3(256), 0, s, w, rows, n_rows,
+                           (nu + 3) / 4, out);
+    else
+        hipLaunchKernelGGL((k_dequant<T, VEC>), dim3(ttiles(w.n_out) * nu), dim3(256), 0, s, w, nu, out);
+}
+
+static hipError_t dequant(const WeightView &w, const uint32_t *rows, uint32_t n_rows, float *out, hipStream_t s) {
+    const bool vec = ((uintptr_t)out & 15) == 0;
+#define LRS_DEQ(T)                                                 \
+    case T:                                                        \
+        if (vec) start_dequant<T, true>(w, rows, n_rows, out, s);  \
+        else start_dequant<T, false>(w, rows, n_rows, out, s);     \
+        break;
+    switch (w.type) {
+        LRS_DEQ(T_Q8_0)
+        LRS_DEQ(T_Q4_K)
+        LRS_DEQ(T_Q5_K)
+        LRS_DEQ(T_Q6_K)
+    default:
+        hipLaunchKernelGGL(k_dequant_raw, dim3(grid_for((uint64_t)n_rows * w.n_in, 256)), dim3(256), 0, s, w, rows,
+                           n_rows, out);
+    }
+#undef LRS_DEQ
     return hipGetLastError();
 }
 
+hipError_t launch_dequant(WeightView w, float *out, hipStream_t s) { return dequant(w, nullptr, w.n_out, out, s); }
+
 hipError_t launch_dequant_rows(WeightView w, const uint32_t *rows_dev, uint32_t n_rows, float *out,
                                hipStream_t s) {
-    uint64_t n = (uint64_t)n_rows * w.n_in;
-    hipLaunchKernelGGL(k_dequant_rows, dim3(grid_for(n, 256)), dim3(256), 0, s, w, rows_dev,
-                       n_rows, out);
-    return hipGetLastError();
+    return dequant(w, rows_dev, n_rows, out, s);
 }
 
 }  // namespace lrs

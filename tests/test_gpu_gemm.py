@@ -113,3 +113,47 @@ def test_gemm_group_rejects_bad_groups(lrs, orc, ctx):
     for group in ([w6, w4], [w4, w6, w4], [w4, w8], [w4, w4k], [w4, w4, w4, w4]):
         with pytest.raises(lrs.ModelError):
             lrs.gemm_group(ctx, group, a)
+
+
+def quantizer_like(t, n, k, seed):
+    """GGUF blocks with every scale a quantizer can leave: Q6_K scales of -128
+    (products above 2048), Q8_0 scales that differ by 2^12 inside a row, K-quant
+    super-blocks with d = 0 (only the minimum counts) and with dmin = 0."""
+    rng = np.random.default_rng(seed)
+    be, bb = {Q8_0: (32, 34), Q4_K: (256, 144), Q5_K: (256, 176), Q6_K: (256, 210)}[t]
+    b = rng.integers(0, 256, (n * k // be, bb), dtype=np.uint8)
+    nb = b.shape[0]
+    f16 = lambda v: np.ascontiguousarray(v, np.float16).view(np.uint8).reshape(nb, 2)
+    if t == Q8_0:
+        b[:, 0:2] = f16(2.0 ** rng.uniform(-16, -4, nb))
+        b[rng.integers(0, nb, max(1, nb // 16)), 0:2] = 0
+    elif t == Q6_K:
+        b[:, 192] = 128
+        b[:, 200] = 127
+        b[:, 208:210] = f16(rng.uniform(0.7, 1.3, nb) * 1e-5)
+    else:
+        d = rng.uniform(0.5, 2.0, nb) * 1e-4
+        d[rng.integers(0, nb, max(1, nb // 8))] = 0
+        m = rng.uniform(0.5, 2.0, nb) * 1e-3
+        m[rng.integers(0, nb, max(1, nb // 8))] = 0
+        b[:, 0:2], b[:, 2:4] = f16(d), f16(m)
+    return b.reshape(-1)
+
+
+@pytest.mark.parametrize("t", [Q8_0, Q4_K, Q5_K, Q6_K])
+@pytest.mark.parametrize("n,k,shift", [(1, 256, 0), (17, 768, 0), (5, 512, 1)])
+def test_dequant_into_any_float_address_is_exact(lrs, orc, ctx, t, n, k, shift):
+    """lrs_weight_dequant_dev at whole and odd row tiles; Q8_0 rows that end
+    inside 256 elements; an output that is not 16-byte aligned; nothing written
+    past the end."""
+    k += 32 if t == Q8_0 else 0
+    w = quantizer_like(t, n, k, n)
+    W = lrs.Weight.upload(ctx, t, w, k, n)
+    out = ctx.alloc(4 * (n * k + 8))
+    out.upload(np.full(n * k + 8, 7.0, np.float32))
+    lrs.check(lrs.lib.lrs_weight_dequant_dev(ctx.h, W.h, out.ptr + 4 * shift))
+    ctx.sync()
+    got = out.download(np.float32, n * k + 8)
+    ref = orc.dequant(t, w)
+    assert np.array_equal(got[shift:shift + n * k].view(np.uint32), ref.view(np.uint32))
+    assert np.all(got[:shift] == 7.0) and np.all(got[shift + n * k:] == 7.0)
