@@ -158,10 +158,10 @@ int lrs_matvec_q8_0_actq_dev(lrs_ctx *ctx, const lrs_weight *w, const float *x_d
  * device f32 buffers, enqueued on the context stream (async).  Replaces the
  * prefill matmul matmul::dispatch_mul_mm_q4k / shaders/mul_mm.comp
  * (crates/llama-vulkan/src/matmul.rs:433-465), which quantizes a to int8:
- * here a and dequant(W) go to v_mfma_f32_32x32x16_bf16 as bf16 with f32
- * accumulation.  precision 1: each operand rounded to bf16 once;
- * precision 3: each split into bf16 hi + lo and three products summed
- * (~2^-16 relative, for prefill that must match the f32 forward).
+ * here both operands keep more bits, with f32 accumulation on the matrix cores.
+ * precision 1: each operand rounded to bf16 once; precision 3: the weights as
+ * exact f16 whole numbers and the activations as f16 hi + lo (22 bits), for
+ * prefill that must match the f32 forward (observed 2e-7 to 5e-7 relative L2).
  * Weights: Q4_K, Q5_K, Q6_K, Q8_0; n_in a multiple of 256. */
 int lrs_gemm_dev(lrs_ctx *ctx, const lrs_weight *w, const float *a_dev, float *y_dev, uint32_t m,
                  int precision);
@@ -171,7 +171,7 @@ int lrs_gemm_dev(lrs_ctx *ctx, const lrs_weight *w, const float *a_dev, float *y
  * is the form a prompt block uses for q / k / v.  The weights share n_in;
  * at most two types, the first type's weights first, and the mixes Q4_K or
  * Q5_K followed by Q6_K (else LRS_E_UNSUPPORTED).  Each output equals the
- * single-weight GEMM without a split over K. */
+ * single-weight GEMM up to the f32 summation order (either may split K). */
 int lrs_gemm_group_dev(lrs_ctx *ctx, const lrs_weight *const *w, uint32_t n_w, const float *a_dev,
                        float *const *y_dev, uint32_t m, int precision);
 

@@ -419,6 +419,20 @@ int lrs_matvec_f32(lrs_ctx *ctx, const lrs_weight *w, const float *x, float *y, 
     return LRS_OK;
 }
 
+// the input packed into context scratch, then the GEMM (its K-slice partials
+// behind the packed input)
+static int gemm_run(lrs_ctx *ctx, const WeightView *wv, float *const *y, const uint32_t *ldy, uint32_t n_w,
+                    const float *a_dev, uint32_t m, int precision) {
+    const size_t ab = gemm_planes_bytes(m, wv[0].n_in, precision);
+    const size_t wb = gemm_work_bytes(m, ldy, n_w, wv[0].n_in, wv[0].type, precision);
+    void *buf = nullptr;
+    if (int rc_ = ctx_scratch(ctx, ab + wb, &buf)) return rc_;
+    LRS_HIP(launch_gemm_pack(a_dev, m, wv[0].n_in, precision, (uint8_t *)buf, ctx->stream));
+    LRS_HIP(launch_gemm_segs(wv, y, ldy, n_w, (const uint8_t *)buf, m, precision, ctx->stream, false,
+                             wb ? (float *)((char *)buf + ab) : nullptr, wb));
+    return LRS_OK;
+}
+
 int lrs_gemm_dev(lrs_ctx *ctx, const lrs_weight *w, const float *a_dev, float *y_dev, uint32_t m,
                  int precision) {
     if (!ctx || !w || !a_dev || !y_dev) return fail(LRS_E_ARG, "null argument");
@@ -429,17 +443,8 @@ int lrs_gemm_dev(lrs_ctx *ctx, const lrs_weight *w, const float *a_dev, float *y
     if (w->v.n_in % 256)
         return fail(LRS_E_ARG, "the GEMM needs n_in to be a multiple of 256");
     SETDEV(ctx);
-    // the activation as bf16 planes (hi, and lo for precision 3) in context scratch
-    // (and the K-slice partials when the GEMM is split over K)
-    const size_t n = (size_t)m * w->v.n_in, ab = (n * 2 * (precision == 3 ? 2 : 1) + 255) & ~(size_t)255;
-    const size_t wb = gemm_work_bytes(m, w->v.n_out, w->v.n_in, precision);
-    void *buf = nullptr;
-    if (int rc_ = ctx_scratch(ctx, ab + wb, &buf)) return rc_;
-    __bf16 *hi = (__bf16 *)buf, *lo = precision == 3 ? hi + n : nullptr;
-    LRS_HIP(launch_split_bf16(a_dev, n, hi, lo, ctx->stream));
-    LRS_HIP(launch_gemm(w->v, hi, lo, y_dev, m, w->v.n_out, precision, ctx->stream, false,
-                        wb ? (float *)((char *)buf + ab) : nullptr));
-    return LRS_OK;
+    const uint32_t ldy = w->v.n_out;
+    return gemm_run(ctx, &w->v, &y_dev, &ldy, 1, a_dev, m, precision);
 }
 
 int lrs_gemm_group_dev(lrs_ctx *ctx, const lrs_weight *const *w, uint32_t n_w, const float *a_dev,
@@ -460,13 +465,7 @@ int lrs_gemm_group_dev(lrs_ctx *ctx, const lrs_weight *const *w, uint32_t n_w, c
     if (!gemm_segs_supported(wv, n_w))
         return fail(LRS_E_UNSUPPORTED, "group types: one type, or Q4_K / Q5_K weights then Q6_K");
     SETDEV(ctx);
-    const size_t n = (size_t)m * wv[0].n_in, ab = n * 2 * (precision == 3 ? 2 : 1);
-    void *buf = nullptr;
-    if (int rc_ = ctx_scratch(ctx, ab, &buf)) return rc_;
-    __bf16 *hi = (__bf16 *)buf, *lo = precision == 3 ? hi + n : nullptr;
-    LRS_HIP(launch_split_bf16(a_dev, n, hi, lo, ctx->stream));
-    LRS_HIP(launch_gemm_segs(wv, y_dev, ldy, n_w, hi, lo, m, precision, ctx->stream));
-    return LRS_OK;
+    return gemm_run(ctx, wv, y_dev, ldy, n_w, a_dev, m, precision);
 }
 
 int lrs_matvec_set_geom(int tiles_per_wave, int tile_groups, int k_slices) {

@@ -1,569 +1,810 @@
 // gemm.hip — dequantize x GEMM for batched prefill on the gfx950 matrix cores.
 //
-// Y[m][n] = sum_k A[m][k] * W[n][k]: A = M tokens x K activations (f32 in
-// HBM), W = a resident N x K GGUF weight (Q4_K, Q5_K, Q6_K or Q8_0).  Replaces the
-// reference's prefill GEMM (shaders/mul_mm.comp, dispatched by
-// matmul::dispatch_mul_mm_q4k, crates/llama-vulkan/src/matmul.rs:433-465),
-// which quantizes A to int8; here both operands go to the MFMA units as bf16
-// (v_mfma_f32_32x32x16_bf16, f32 accumulate):
-//   PREC 1  A and dequant(W) rounded to bf16 once
-//   PREC 3  both split into bf16 hi + lo, three products (hi*hi + hi*lo +
-//           lo*hi): ~2^-16 relative per product, for prefill whose logits must
-//           match the f32 reference
+// Y[m][n] = sum_k A[m][k] * W[n][k]: A = M tokens x K activations (f32, packed
+// by the producing kernel or launch_gemm_pack, gemm_pack.h), W = a resident
+// N x K GGUF weight (Q4_K, Q5_K, Q6_K or Q8_0).  Replaces the reference's
+// prefill GEMM (shaders/mul_mm.comp, dispatched by matmul::dispatch_mul_mm_q4k,
+// crates/llama-vulkan/src/matmul.rs:433-465), which quantizes A to int8.
+//   precision 1  A and dequant(W) rounded to bf16 once, f32 accumulation
+//   precision 3  f32-grade, for prefill whose logits must match the f32
+//                forward: the weights go to the matrix cores as exact whole
+//                numbers in f16 (sub-block scale times quant: at most 1953 for
+//                Q4_K / Q5_K; Q6_K products above 2048 and Q8_0's f16 scale
+//                times quant as f16 hi + lo), the activations as f16 hi + lo
+//                (22 bits under their super-block's own power of two).  Two
+//                products a weight (three for Q6_K / Q8_0) accumulate in f32
+//                over a super-block of 256; its f16 scale and the activations'
+//                power of two multiply the sum once (fold).  The K-quant
+//                minima are one more K-step: minima x sub-block sums.
+// With both operands split into bf16 hi + lo and three products this took 1.7
+// times as long (32B gate / up at 512 tokens 978 -> 575 us; bf16 hi + lo is
+// 4e-6 from the 64-bit result, this 2e-7 to 3e-7).
 //
-// Tiling.  A 512-thread workgroup owns a BM (tokens) x 128 (weight rows)
-// output tile: BM = 256 for bf16 operands at M >= 512 (each wavefront a
-// 64 x 64 part = 4 MFMA tiles of 32 x 32), else 128 (64 x 32 parts, 2
-// tiles).  K advances 64 at a time: every thread stages BM / 8 activations
-// (bf16, split from f32 once per GEMM input) and dequantizes 16 weights of
-// one row (f32 dequant as in dequant.rs, the K-quant min term in the same
-// fused multiply-add as the scale, then bf16) into a double-buffered LDS
-// tile, and each wavefront issues 4 K16 steps of MFMA over its tiles.  LDS
-// rows are padded to 72 bf16 so the 32 lanes that read 32 different rows at
-// one K offset hit distinct banks.
-#include "lrs_internal.h"
+// Tiling.  A 256-thread workgroup owns 32 MT tokens x 256 weight rows, each of
+// its four wavefronts MT x 2 tiles of 32 x 32.  A wavefront unpacks its own 64
+// rows' weights from registers straight into matrix operands, so weights never
+// go through LDS and no wavefront waits for another's dequant; the activations
+// are copied to LDS by global_load_lds in the order in which they are read (no
+// padding, no address arithmetic, no bank conflicts).  A stage is half a
+// super-block: the next stage's copies and weight loads are issued, then the
+// current one computes, then one barrier.  Two independent workgroups per CU
+// fill each other's waits (one workgroup of eight wavefronts in lockstep took
+// 98 against 63 us at 512 x 5120 x 5120).
+//
+// What bounds it: the matrix pipe and the vector pipe both near full (132
+// matrix operations of 32 clocks and about 610 vector operations of 4.8 clocks
+// per wavefront and super-block; up to four vector operations hide behind a
+// matrix one), and at 512 tokens the card's power: 1.85-1.95 GHz during the
+// gate / up launch, whose 1.1 PFLOP/s of products compare with 1.27 (bf16) and
+// 1.37 (f16) of a large library product.
+#include "gemm_pack.h"
 #include "quant_dev.h"
+
+#include <algorithm>
 
 namespace lrs {
 
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
+typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
+typedef __attribute__((address_space(3))) void lds_void;
 
-constexpr int GM_BN = 128, GM_BK = 64;
-constexpr int GM_LD = GM_BK + 8;  // padded LDS row (bf16 elements)
-
-// one weight of a launch: weights that share the input (a prompt block's q,
-// k and v projections) run as one launch over their concatenated output
-// tiles, segment s owning tiles [nt0, next segment's nt0) along N
-constexpr int GM_MAX_SEG = 3;
-struct GemmSeg {
+constexpr int PG_WAVES = 4;
+constexpr int PG_MAX_SEG = 3;
+struct PgSeg {
     const uint8_t *q;  // weight, tiled layout (tiled.h)
     float *y;          // [M][ldy]
-    uint32_t N, ldy, nt0;
+    uint32_t N, ldy, nt0, noff;
 };
-
-struct GemmArgs {
-    const __bf16 *ahi, *alo;  // A [M][K] as bf16 (hi, and lo = bf16(a - hi) for PREC 3)
-    GemmSeg seg[GM_MAX_SEG];
-    uint32_t nseg, nseg0;     // segments; the first nseg0 have the kernel's type T0, the rest T1
-    uint32_t M, K;
-    uint32_t accum;           // 1: y += A W^T (residual add), 0: y = A W^T
-    uint32_t nm, nn;          // output tiles along M and N (all segments)
-    uint32_t ks;              // K slices (one segment): slice z writes part + z*M*N (then a reduce)
+struct PgArgs {
+    const uint8_t *a;  // planes (gemm_pack.h)
+    PgSeg seg[PG_MAX_SEG];
+    uint32_t nseg, nseg0, M, nsb, accum, nm, nn, ks, ntot;
     float *part;
 };
 
-__device__ __forceinline__ u32x4 ldq16(const uint8_t *p) { return *reinterpret_cast<const u32x4 *>(p); }
+__device__ __forceinline__ f16x2 as_h2(uint32_t v) { return __builtin_bit_cast(f16x2, v); }
+// Raw bytes of one lane for 128 elements (half a super-block) of its weight
+// row: lane group hf holds the pieces of 16 elements whose index is odd / even.
+// A stage loads only the words it uses: a register that a load in flight will
+// write and nobody reads would be handed out again, and its next use would wait
+// for that load.  Q4_K / Q5_K: h0 = f16 d and dmin, sc and mn the packed scales
+// and minima of the half (raw words); Q6_K: sc the half's two scale words.
+template <uint32_t T> struct WHalf;
+template <> struct WHalf<T_Q4_K> { uint32_t h0, h1, h2, h3; u32x4 q[2]; };
+template <> struct WHalf<T_Q5_K> { uint32_t h0, h1, h2, h3; u32x4 qh, q[2]; };
+template <> struct WHalf<T_Q6_K> { u32x2 sc; u32x4 la, lb, qh; uint32_t d; };
+template <> struct WHalf<T_Q8_0> { u32x4 q[4]; uint32_t d[4]; };  // d: the f16 scales of the whole super-block
 
-// Raw GGUF bytes a thread needs for 16 consecutive weights of row n starting
-// at element e (e % 16 == 0), loaded three K-steps ahead and dequantized
-// after the current step's matrix-core work has been issued
-template <uint32_t T> struct WRaw;
-template <> struct WRaw<T_Q4_K> { u32x4 hd, qs; };
-template <> struct WRaw<T_Q6_K> { u32x4 ql, qh; uint32_t sc, d; };
-template <> struct WRaw<T_Q5_K> { u32x4 hd, qh, qs; };
-template <> struct WRaw<T_Q8_0> { u32x4 qs; uint32_t d; };
+// Addresses: c is uniform (the chunk of the wavefront's first row tile, in
+// scalar registers), o the lane's 32-bit offset to its own row tile, so that a
+// load needs no 64-bit address arithmetic per lane.
+__device__ __forceinline__ u32x4 ldo(const uint8_t *c, uint32_t o) { return *reinterpret_cast<const u32x4 *>(c + o); }
 
-// rowq = the first chunk of the row's 16-row tile (hoisted out of the K
-// loop: per step only the 32-bit unit offset changes); r = row in the tile
-template <uint32_t T>
-__device__ __forceinline__ void wload(const uint8_t *rowq, uint32_t r, uint32_t e, WRaw<T> &w) {
-    const uint32_t o = e & 255;  // offset inside the super-block
-    const uint32_t l0 = o & 16;  // first or second 16 of a 32-element run
-    const uint8_t *c = rowq + (e / tunit_elems(T)) * tchunk_bytes(T);
-    if constexpr (T == T_Q8_0) {
-        // 64-element units of two blocks: piece g = 2 block + 16-byte half,
-        // then the 16 rows' f16 d of both blocks (tiled.h)
-        const uint32_t o6 = e & 63, b = o6 >> 5, pg = 2 * b + ((o6 >> 4) & 1);
-        w.qs = ldq16(c + 16 * (16 * pg + r));
-        w.d = *reinterpret_cast<const uint16_t *>(c + 1024 + 4 * r + 2 * b);
+// Q8_0: 16-byte piece k (K-steps 2 k, 2 k + 1 of the half) of the lane's row
+__device__ __forceinline__ u32x4 q8_piece(const uint8_t *c, uint32_t o, uint32_t r, uint32_t hf, int half, int k) {
+    return ldo(c + (2 * half + (k >> 1)) * 1088 + 512 * (k & 1), o + 256 * hf + 16 * r);
+}
+
+// c + o = the super-block's chunk (Q8_0: its first 64-element unit's chunk) of the row's tile
+template <uint32_t T, int PREC>
+__device__ __forceinline__ void wload(const uint8_t *c, uint32_t o, uint32_t r, uint32_t hf, int half, WHalf<T> &w) {
+    const uint32_t o0 = o + 16 * r, o1 = o0 + 256 * hf;
+    if constexpr (T == T_Q4_K || T == T_Q5_K) {
+        // precision 3 takes d, dmin and the minima once, with the second half
+        if (half == 1) {
+            const u32x4 h = ldo(c, o0);
+            w.h0 = h.x, w.h1 = h.y, w.h2 = h.z, w.h3 = h.w;
+        } else if (PREC == 3) {
+            w.h1 = *reinterpret_cast<const uint32_t *>(c + 4 + o0);
+        } else {
+            w.h0 = *reinterpret_cast<const uint32_t *>(c + o0);
+            const u32x2 h = *reinterpret_cast<const u32x2 *>(c + 4 + o0);
+            w.h1 = h.x, w.h2 = h.y;
+        }
+    }
+    if constexpr (T == T_Q4_K) {
+        w.q[0] = ldo(c + 256 + 1024 * half, o1);
+        w.q[1] = ldo(c + 768 + 1024 * half, o1);
     } else if constexpr (T == T_Q5_K) {
-        // as Q4_K with qs after the qh halves; qh[l0 .. l0 + 16) of row r is
-        // half l0 / 16 of the row's qh (dequant.rs:157-203)
-        const uint32_t j = o >> 6, pg = 2 * (j & 1) + (l0 >> 4);
-        w.hd = ldq16(c + 16 * r);
-        w.qh = ldq16(c + 256 + 16 * (16 * (l0 >> 4) + r));
-        w.qs = ldq16(c + 768 + 1024 * (j >> 1) + 16 * (16 * pg + r));
-    } else if constexpr (T == T_Q4_K) {
-        // qs[32j + l0 ..+16), j = o / 64: piece (g, r), g = 2(j&1) + l0/16, of half j>>1
-        const uint32_t j = o >> 6, pg = 2 * (j & 1) + (l0 >> 4);
-        w.hd = ldq16(c + 16 * r);
-        w.qs = ldq16(c + 256 + 1024 * (j >> 1) + 16 * (16 * pg + r));
-    } else {  // T_Q6_K
-        // elements 128h + 32 quarter + l: ql[64h + 32(quarter&1) + l], qh[32h + l],
-        // pieces g = 2h + l0/16; scale byte 8h + l0/16 + 2 quarter
-        const uint32_t h = o >> 7, quarter = (o >> 5) & 3, pg = 2 * h + (l0 >> 4);
-        w.ql = ldq16(c + 256 + 1024 * (quarter & 1) + 16 * (16 * pg + r));
-        w.qh = ldq16(c + 2304 + 16 * (16 * pg + r));
-        w.sc = c[16 * r + 8 * h + (l0 >> 4) + 2 * quarter];
-        w.d = *reinterpret_cast<const uint16_t *>(c + 3328 + 2 * r);
+        w.qh = ldo(c + 256, o1);
+        w.q[0] = ldo(c + 768 + 1024 * half, o1);
+        w.q[1] = ldo(c + 1280 + 1024 * half, o1);
+    } else if constexpr (T == T_Q6_K) {
+        w.sc = *reinterpret_cast<const u32x2 *>(c + 8 * half + o0);
+        w.la = ldo(c + 256 + 512 * half, o1);
+        w.lb = ldo(c + 1280 + 512 * half, o1);
+        w.qh = ldo(c + 2304 + 512 * half, o1);
+        if (PREC == 1 || half == 1) w.d = *reinterpret_cast<const uint16_t *>(c + 3328 + (o + 2 * r));
+    } else {
+#pragma unroll
+        for (int k = 0; k < 4; k++) w.q[k] = q8_piece(c, o, r, hf, half, k);
+#pragma unroll
+        for (int u = 0; u < 4; u++) w.d[u] = *reinterpret_cast<const uint32_t *>(c + u * 1088 + 1024 + (o + 4 * r));
     }
 }
 
-// the 16 weights in f32 as ggml_cpu::dequant (dequant.rs:101-258) computes
-// them with one fused multiply-add each: Q6_K a*q - 32a is a*(q - 32)
-// rounded once, bit-exact; Q4_K / Q5_K a*q - b skips the reference's
-// rounding of a*q (half an ulp of the product), which the bf16 rounding
-// that follows absorbs:
-// wprep decodes the run's scale (and min), wdeq4 the weights 4c..4c+3, so the
-// dequant can be spread between the matrix-core ops of a pipeline step
-struct DeqPrep {
-    float a, b;    // Q4_K / Q5_K: d * sc, dmin * m; Q6_K: d * scale; Q8_0: d
-    uint32_t sel;  // Q4_K / Q5_K: high nibbles; Q6_K: quarter of the half
-    uint32_t sub;  // Q5_K: sub-block (its bit of qh)
+// the 6-bit scales (minima) of sub-blocks 4 half .. 4 half + 3 as bytes of a
+// word, from header words h1 (h2) and h3
+template <class W>
+__device__ __forceinline__ uint32_t k4_scales(const W &w, int half) {
+    return half == 0 ? w.h1 & 0x3F3F3F3Fu : (w.h3 & 0x0F0F0F0Fu) | ((w.h1 >> 2) & 0x30303030u);
+}
+template <class W>
+__device__ __forceinline__ uint32_t k4_mins(const W &w, int half) {
+    return half == 0 ? w.h2 & 0x3F3F3F3Fu : ((w.h3 >> 4) & 0x0F0F0F0Fu) | ((w.h2 >> 2) & 0x30303030u);
+}
+
+// words 2 pair, 2 pair + 1 of a piece
+__device__ __forceinline__ uint32_t pw(const u32x4 &v, int pair, int i) { return v[2 * pair + i]; }
+
+// Q8_0: the f16 scales of a super-block share a power of two 2^ex > max |d|
+// (an f16 scale over it is a fraction, exact in f16 but for scales 2^14 below
+// the largest, whose last bits fall under 2^-24 of it)
+__device__ __forceinline__ int q8_exp(const uint32_t (&d)[4]) {
+    uint32_t m = 0;
+#pragma unroll
+    for (int u = 0; u < 4; u++) m = max(m, max(d[u] & 0x7FFFu, (d[u] >> 16) & 0x7FFFu));
+    int ex;
+    (void)frexpf(h2f((uint16_t)m), &ex);
+    return m ? ex : 0;
+}
+
+// (v & M) | 0x64006400 (two f16 of 1024 + the masked bits) as one instruction:
+// the constants are hidden from the compiler, which would fold them into two
+// instructions with a literal each
+template <uint32_t M>
+__device__ __forceinline__ uint32_t and_1024(uint32_t v) {
+    uint32_t m = M, k = 0x64006400u;
+    asm("" : "+s"(m));
+    asm("" : "+v"(k));
+    return (v & m) | k;
+}
+// the bytes (b0, b2) or (b1, b3) of a word as a pair of f16 whole numbers + 1024
+__device__ __forceinline__ f16x2 pair02(uint32_t v) { return as_h2((v & 0x00FF00FFu) | 0x64006400u); }
+__device__ __forceinline__ f16x2 pair13(uint32_t v) { return pair02(v >> 8); }
+__device__ __forceinline__ f16x2 both(_Float16 v) { return f16x2{v, v}; }
+__device__ __forceinline__ f16x2 both(float v) { return both((_Float16)v); }
+
+// the f16 scales of half a super-block's K-steps 2 s, 2 s + 1 (s = 0..3)
+template <uint32_t T> struct SHalf { f16x2 a, b; };  // (s = 0, 2), (s = 1, 3); Q6_K: (0, 1), (2, 3)
+template <uint32_t T>
+__device__ __forceinline__ SHalf<T> scales(const WHalf<T> &w, int half, uint32_t hf, int ex) {
+    SHalf<T> s;
+    if constexpr (T == T_Q4_K || T == T_Q5_K) {
+        // the odd sub-blocks are the high nibbles, unpacked times 16
+        const uint32_t v = k4_scales(w, half);
+        s.a = pair02(v) - both(1024.0f);
+        s.b = (pair13(v) - both(1024.0f)) * both(0.0625f);
+    } else if constexpr (T == T_Q6_K) {
+        // int8 scales 8 half + 2 quarter + hf
+        s.a = pair02((w.sc.x >> (8 * hf)) ^ 0x00800080u) - both(1152.0f);
+        s.b = pair02((w.sc.y >> (8 * hf)) ^ 0x00800080u) - both(1152.0f);
+    } else {
+        float d[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) d[i] = ldexpf(h2f((uint16_t)(w.d[2 * half + (i >> 1)] >> (16 * (i & 1)))), -ex);
+        s.a = f16x2{(_Float16)d[0], (_Float16)d[2]};
+        s.b = f16x2{(_Float16)d[1], (_Float16)d[3]};
+    }
+    return s;
+}
+
+// B operand of K-step t (0..7 of the half) for precision 3: bh + bl is the
+// weight without the super-block's factor (fold), exact
+template <uint32_t T>
+__device__ __forceinline__ void bfrag_int(const WHalf<T> &w, const SHalf<T> &sc, int half, int t, f16x8 &bh, f16x8 &bl) {
+    const int s = t >> 1, pair = t & 1;
+    const f16x2 sv = T == T_Q6_K ? both(s < 2 ? sc.a[s & 1] : sc.b[s & 1]) : both(s & 1 ? sc.b[s >> 1] : sc.a[s >> 1]);
+    // the constants that take the unpacking offset off: -1024 sc (K-quants)
+    const f16x2 cv = sv * both(-1024.0f);
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        f16x2 f[2];
+        if constexpr (T == T_Q4_K || T == T_Q5_K) {
+            // (1024 + q) sc - 1024 sc, or with the nibble in bits 4..7
+            // (1024 + 16 q) sc / 16 - 64 sc: whole numbers up to 1953, exact
+            const int hi = s & 1;
+            const uint32_t v = pw(w.q[s >> 1], pair, i);
+            uint32_t e0 = hi ? and_1024<0x00F000F0u>(v) : and_1024<0x000F000Fu>(v);
+            uint32_t e1 = hi ? and_1024<0x00F000F0u>(v >> 8) : and_1024<0x000F000Fu>(v >> 8);
+            if constexpr (T == T_Q5_K) {
+                const uint32_t h = pw(w.qh, pair, i) >> (4 * half + s);
+                e0 |= (h & 0x00010001u) << (hi ? 8 : 4);
+                e1 |= ((h >> 8) & 0x00010001u) << (hi ? 8 : 4);
+            }
+            f[0] = __builtin_elementwise_fma(as_h2(e0), sv, cv);
+            f[1] = __builtin_elementwise_fma(as_h2(e1), sv, cv);
+        } else {
+            // whole numbers q times the scale, rounded to f16, and the exact
+            // remainder of that rounding (Q6_K: of products above 2048)
+            f16x2 q0, q1;
+            if constexpr (T == T_Q6_K) {
+                const uint32_t l = pw((s & 1) ? w.lb : w.la, pair, i) >> (4 * (s >> 1));
+                const uint32_t hb = pw(w.qh, pair, i);
+                const uint32_t h = s == 0 ? hb << 4 : s == 1 ? hb << 2 : s == 2 ? hb : hb >> 2;
+                q0 = as_h2(and_1024<0x000F000Fu>(l) | (h & 0x00300030u)) - both(1056.0f);
+                q1 = as_h2(and_1024<0x000F000Fu>(l >> 8) | ((h >> 8) & 0x00300030u)) - both(1056.0f);
+            } else {
+                const uint32_t v = pw(w.q[s], pair, i) ^ 0x80808080u;
+                q0 = pair02(v) - both(1152.0f);
+                q1 = pair13(v) - both(1152.0f);
+            }
+            f[0] = q0 * sv;
+            f[1] = q1 * sv;
+            const f16x2 g0 = __builtin_elementwise_fma(q0, sv, -f[0]), g1 = __builtin_elementwise_fma(q1, sv, -f[1]);
+            bl[4 * i] = g0[0];
+            bl[4 * i + 1] = g0[1];
+            bl[4 * i + 2] = g1[0];
+            bl[4 * i + 3] = g1[1];
+        }
+        bh[4 * i] = f[0][0];
+        bh[4 * i + 1] = f[0][1];
+        bh[4 * i + 2] = f[1][0];
+        bh[4 * i + 3] = f[1][1];
+    }
+}
+
+// precision 1: the f32 scale and offset of K-steps 2 s, 2 s + 1 of a half
+template <uint32_t T> struct AHalf { float a[4], o[4]; };
+template <uint32_t T>
+__device__ __forceinline__ AHalf<T> affine(const WHalf<T> &w, int half, uint32_t hf) {
+    AHalf<T> r;
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+        if constexpr (T == T_Q4_K || T == T_Q5_K) {
+            const uint32_t sc = (k4_scales(w, half) >> (8 * s)) & 0xFF, m = (k4_mins(w, half) >> (8 * s)) & 0xFF;
+            r.a[s] = __fmul_rn(h2f((uint16_t)(w.h0 & 0xFFFF)), (float)sc);
+            r.o[s] = -__fmul_rn(h2f((uint16_t)(w.h0 >> 16)), (float)m);
+        } else if constexpr (T == T_Q6_K) {
+            const uint32_t sw = w.sc[s >> 1] >> (16 * (s & 1));
+            r.a[s] = __fmul_rn(h2f((uint16_t)w.d), (float)(int8_t)((sw >> (8 * hf)) & 0xFF));
+        } else {
+            r.a[s] = h2f((uint16_t)(w.d[2 * half + (s >> 1)] >> (16 * (s & 1))));
+        }
+    }
+    return r;
+}
+
+// B operand of K-step t, precision 1: the weights in f32 (one fused
+// multiply-add each: dequant.rs's value for Q6_K and Q8_0; Q4_K / Q5_K without
+// the rounding of d sc q), rounded to bf16
+template <uint32_t T>
+__device__ __forceinline__ bf16x8 bfrag_bf16(const WHalf<T> &w, const AHalf<T> &af, int half, int t) {
+    const int s = t >> 1, pair = t & 1;
+    const float o = T == T_Q6_K ? -32.0f * af.a[s] : T == T_Q8_0 ? -128.0f * af.a[s] : af.o[s];  // exact products
+    u32x4 b;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        uint32_t q;
+        if constexpr (T == T_Q8_0) {
+            q = pw(w.q[s], pair, i) ^ 0x80808080u;
+        } else if constexpr (T == T_Q6_K) {
+            const uint32_t hb = pw(w.qh, pair, i);
+            q = ((pw((s & 1) ? w.lb : w.la, pair, i) >> (4 * (s >> 1))) & 0x0F0F0F0Fu) |
+                ((s == 0 ? hb << 4 : s == 1 ? hb << 2 : s == 2 ? hb : hb >> 2) & 0x30303030u);
+        } else {
+            q = (pw(w.q[s >> 1], pair, i) >> (4 * (s & 1))) & 0x0F0F0F0Fu;
+            if constexpr (T == T_Q5_K) q |= ((pw(w.qh, pair, i) >> (4 * half + s)) & 0x01010101u) << 4;
+        }
+        // hidden: the compiler would turn the byte conversions into shifts,
+        // knowing which bits of the bytes are set
+        asm("" : "+v"(q));
+        float v[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[k] = fmaf(af.a[s], (float)((q >> (8 * k)) & 0xFF), o);
+        typedef __attribute__((ext_vector_type(2))) float f32x2;
+        b[2 * i] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{v[0], v[2]}), bf16x2));
+        b[2 * i + 1] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{v[1], v[3]}), bf16x2));
+    }
+    return __builtin_bit_cast(bf16x8, b);
+}
+
+// the eight minima as f16, in the order of the sub-block sums
+template <class W>
+__device__ __forceinline__ f16x8 min_frag(const W &w) {
+    f16x8 m;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const uint32_t v = k4_mins(w, i);
+        const f16x2 f0 = pair02(v) - both(1024.0f), f1 = pair13(v) - both(1024.0f);
+        m[4 * i] = f0[0];
+        m[4 * i + 1] = f0[1];
+        m[4 * i + 2] = f1[0];
+        m[4 * i + 3] = f1[1];
+    }
+    return m;
+}
+
+template <int PREC, int MT> struct PgLds {
+    static constexpr int STEP = PREC == 3 ? 2048 : 1024;  // bytes of a K-step of a row tile
+    static constexpr int STAGE = MT * 8 * STEP;
+    static constexpr int SUMS = PREC == 3 ? MT * 2048 : 16;
 };
-template <uint32_t T>
-__device__ __forceinline__ DeqPrep wprep(const WRaw<T> &w, uint32_t e) {
-    const uint32_t o = e & 255;
-    DeqPrep p;
-    p.sub = 0;
-    if constexpr (T == T_Q8_0) {
-        p.a = h2f((uint16_t)w.d);
-        p.b = 0.f;
-        p.sel = 0;
-    } else if constexpr (T == T_Q4_K || T == T_Q5_K) {
-        const uint32_t j = o >> 6, hi = (o >> 5) & 1;  // qs group, high nibbles
-        // get_scale_min_k4 (dequant.rs:101-110): scale bytes 0-3, 4-7, 8-11 are
-        // header words y, z, w; sub-block jj reads byte jj & 3 of each
-        const uint32_t jj = 2 * j + hi, sh = 8 * (jj & 3);
-        const uint32_t by = (w.hd.y >> sh) & 0xFF, bz = (w.hd.z >> sh) & 0xFF,
-                       bw = (w.hd.w >> sh) & 0xFF;
-        // both forms, then a mask select: a conditional here compiles to a
-        // divergent branch, which splits the step's MFMA / VALU interleaving
-        const uint32_t lowm = 0u - (uint32_t)(jj < 4);
-        const uint32_t sc = ((by & 63) & lowm) | (((bw & 0xF) | ((by >> 6) << 4)) & ~lowm);
-        const uint32_t m = ((bz & 63) & lowm) | (((bw >> 4) | ((bz >> 6) << 4)) & ~lowm);
-        const float dv = h2f((uint16_t)(w.hd.x & 0xFFFF)), mv = h2f((uint16_t)(w.hd.x >> 16));
-        p.a = __fmul_rn(dv, (float)sc);
-        p.b = __fmul_rn(mv, (float)m);
-        p.sel = hi;
-        p.sub = jj;
-    } else {  // T_Q6_K
-        p.a = __fmul_rn(h2f((uint16_t)w.d), (float)(int8_t)(w.sc & 0xFF));
-        p.b = 0.f;
-        p.sel = (o >> 5) & 3;
-    }
-    return p;
-}
-template <uint32_t T>
-__device__ __forceinline__ void wdeq4(const WRaw<T> &w, const DeqPrep &p, int c, float (&v)[16]) {
-    if constexpr (T == T_Q8_0) {
-        // dequant.rs:58-76: q * d
-        const uint32_t qw = c == 0 ? w.qs.x : c == 1 ? w.qs.y : c == 2 ? w.qs.z : w.qs.w;
+
+template <uint32_t T, int PREC, int MT, int NT> struct PgTile {
+static __device__ __forceinline__ void run(const PgArgs &g, const PgSeg &sg, uint32_t kz, uint32_t mb, uint32_t n0,
+                                           uint8_t *As0, uint8_t *As1, uint8_t *Ss) {
+    using L = PgLds<PREC, MT>;
+    constexpr uint32_t BB = gemm_block_bytes(PREC);
+    constexpr bool MINS = T == T_Q4_K || T == T_Q5_K;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, hf = lane >> 5;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t s0 = kz * g.nsb / g.ks, s1 = (kz + 1) * g.nsb / g.ks;  // super-blocks of the K slice
+    const uint32_t nw0 = n0 + 32 * NT * wave;  // this wavefront's rows
+    const uint32_t nmt = (g.M + 31) / 32;
+
+    constexpr uint32_t CH = T == T_Q8_0 ? 4 * tchunk_bytes(T) : tchunk_bytes(T);  // bytes per super-block
+    const uint32_t r = lane & 15, last = (sg.N + 15) / 16 - 1;
+    const uint32_t tile0 = min(nw0 / 16, last);
+    const uint8_t *const wp = sg.q + (size_t)tile0 * g.nsb * CH;
+    uint32_t wo[NT];
 #pragma unroll
-        for (int i = 0; i < 4; i++)
-            v[4 * c + i] = __fmul_rn((float)(int8_t)((qw >> (8 * i)) & 0xFF), p.a);
-    } else if constexpr (T == T_Q4_K || T == T_Q5_K) {
-        // the four quants as bytes of one word (nibble select and, for Q5_K,
-        // the fifth bits: a few ops per 4 weights), then per weight one byte
-        // conversion and one fused a * q - b
-        const uint32_t qw = c == 0 ? w.qs.x : c == 1 ? w.qs.y : c == 2 ? w.qs.z : w.qs.w;
-        uint32_t q4 = (qw >> (4 * p.sel)) & 0x0F0F0F0Fu;
-        if constexpr (T == T_Q5_K) {
-            const uint32_t hw = c == 0 ? w.qh.x : c == 1 ? w.qh.y : c == 2 ? w.qh.z : w.qh.w;
-            q4 |= ((hw >> p.sub) & 0x01010101u) << 4;
+    for (int i = 0; i < NT; i++) wo[i] = (min(nw0 / 16 + 2 * i + ((lane >> 4) & 1), last) - tile0) * g.nsb * CH;
+    // activation blocks of the row tiles (past the last one: a copy of it)
+    const uint8_t *ap[MT];
+#pragma unroll
+    for (int i = 0; i < MT; i++) ap[i] = g.a + (size_t)min(mb * MT + i, nmt - 1) * g.nsb * BB;
+
+    auto dma = [&](uint32_t sb, int half, uint8_t *dst) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < MT; i++)
+#pragma unroll
+            for (int u = 0; u < 8 * L::STEP / 1024 / PG_WAVES; u++) {
+                const uint32_t un = wave + PG_WAVES * u;
+                __builtin_amdgcn_global_load_lds(ap[i] + ((size_t)sb * BB + half * 8 * L::STEP + 1024 * un) + 16 * lane,
+                                                 (lds_void *)(dst + i * 8 * L::STEP + 1024 * un), 16, 0, 0);
+            }
+    };
+    auto dma_sums = [&](uint32_t sb) __attribute__((always_inline)) {
+        if constexpr (PREC == 3) {
+            if (wave < 2)
+#pragma unroll
+                for (int i = 0; i < MT; i++)
+                    __builtin_amdgcn_global_load_lds(ap[i] + (size_t)sb * BB + GP_SUMS + 1024 * wave + 16 * lane,
+                                                     (lds_void *)(Ss + (sb & 1) * L::SUMS + i * 2048 + 1024 * wave),
+                                                     16, 0, 0);
         }
-#pragma unroll
-        for (int i = 0; i < 4; i++) v[4 * c + i] = fmaf(p.a, (float)((q4 >> (8 * i)) & 0xFF), -p.b);
-    } else {  // T_Q6_K: q = (ql nibble | qh 2 bits << 4) - 32
-        const uint32_t lw = c == 0 ? w.ql.x : c == 1 ? w.ql.y : c == 2 ? w.ql.z : w.ql.w;
-        const uint32_t hw = c == 0 ? w.qh.x : c == 1 ? w.qh.y : c == 2 ? w.qh.z : w.qh.w;
-        const uint32_t q4 = ((lw >> (4 * (p.sel >> 1))) & 0x0F0F0F0Fu) |
-                            (((hw >> (2 * p.sel)) & 0x03030303u) << 4);
-        const float o = -32.0f * p.a;  // exact: a power-of-two multiple
-#pragma unroll
-        for (int i = 0; i < 4; i++) v[4 * c + i] = fmaf(p.a, (float)((q4 >> (8 * i)) & 0xFF), o);
-    }
-}
+    };
 
-__device__ __forceinline__ __bf16 to_bf16(float v) { return (__bf16)v; }
-
-// stores 16 values as bf16 (hi) and, for PREC 3, the bf16 remainders (lo)
-template <int PREC>
-__device__ __forceinline__ void put16(__bf16 *hi, __bf16 *lo, const float (&v)[16]) {
-#pragma unroll
-    for (int c = 0; c < 2; c++) {
-        bf16x8 h, l;
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const float x = v[8 * c + i];
-            h[i] = to_bf16(x);
-            if constexpr (PREC == 3) l[i] = to_bf16(x - (float)h[i]);
-        }
-        *reinterpret_cast<bf16x8 *>(hi + 8 * c) = h;
-        if constexpr (PREC == 3) *reinterpret_cast<bf16x8 *>(lo + 8 * c) = l;
-    }
-}
-
-// 512 threads = 8 wavefronts, each a 64 (tokens) x 32 (rows) part of the
-// 128 x 128 tile (2 MFMA tiles of 32 x 32).  Software pipeline over K: step
-// k's operands sit in LDS buffer k & 1; the activations (already bf16, split
-// once per GEMM input by k_split_bf16) and raw weight bytes of steps k+1..k+3
-// are in flight to four rotating register sets; each step the wavefronts
-// load step k+3, issue step k's MFMAs, then dequantize step k+1 into the
-// other buffer (VALU work that overlaps the matrix cores), then one barrier.
-// K-quant rows are whole super-blocks (K % 256 == 0), so the loop runs four
-// steps per trip with no tail.  One call computes the output tile (m0, n0
-// of segment sg) of K slice kz with the weight of type T, over the
-// workgroup's LDS stages As / Ws.
-template <uint32_t T, int PREC, int BM>
-__device__ __forceinline__ void gemm_tile(const GemmArgs &g, const GemmSeg &sg, uint32_t kz,
-                                          uint32_t m0, uint32_t n0,
-                                          __bf16 (*As)[PREC == 3 ? 2 : 1][BM * GM_LD],
-                                          __bf16 (*Ws)[PREC == 3 ? 2 : 1][GM_BN * GM_LD]) {
-    constexpr int NS = PREC == 3 ? 2 : 1;  // hi (+ lo) planes
-    // wavefront grid: WM x WN = 8 wavefronts, each (BM / WM) x (128 / WN) of
-    // the tile in MT x NT MFMA tiles of 32 x 32 (the 256-token tile uses 4 x 2
-    // wavefronts of 64 x 64: fewer LDS operand reads per matrix-core op)
-    constexpr int WM = BM == 256 ? 4 : 2, WN = 8 / WM;
-    constexpr int MT = BM / WM / 32, NT = GM_BN / WN / 32;
-    constexpr int AR = BM / 128;           // activation rows staged per thread
-    const uint32_t kspan = g.K / g.ks;     // a multiple of 256
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const uint32_t wm = wave / WN, wn = wave % WN;
-    // staging roles: thread t handles row t/4, K quarter t%4 (16 of the 64)
-    const uint32_t sr = tid >> 2, sq = (tid & 3) * 16;
-    const uint32_t wr = min(n0 + sr, sg.N - 1);
-    size_t aoff[AR];  // activation rows sr, sr + 128, ...
-#pragma unroll
-    for (int j = 0; j < AR; j++)
-        aoff[j] = (size_t)min(m0 + sr + 128 * j, g.M - 1) * g.K + sq + (size_t)kz * kspan;
-    const uint32_t kbase = kz * kspan;  // weight element offset of the slice
-    const uint8_t *rowq = sg.q + (size_t)(wr >> 4) * tunits(T, g.K) * tchunk_bytes(T);
-
-    f32x16 acc[MT][NT];
+    f32x16 tot[MT][NT], acc[MT][NT];
 #pragma unroll
     for (int i = 0; i < MT; i++)
 #pragma unroll
-        for (int jn = 0; jn < NT; jn++)
+        for (int j = 0; j < NT; j++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][jn][r] = 0.f;
+            for (int e = 0; e < 16; e++) tot[i][j][e] = 0.f;
 
-    u32x4 a0[NS][AR][2], a1[NS][AR][2], a2[NS][AR][2], a3[NS][AR][2];
-    WRaw<T> w0, w1, w2, w3;
-#define LRS_GFETCH(A, W, K0)                                                                  \
-    do {                                                                                      \
-        _Pragma("unroll") for (int p = 0; p < NS; p++)                                         \
-            _Pragma("unroll") for (int j = 0; j < AR; j++) {                                   \
-                const u32x4 *ap = reinterpret_cast<const u32x4 *>((p == 0 ? g.ahi : g.alo) + aoff[j] + (K0)); \
-                A[p][j][0] = ap[0];                                                           \
-                A[p][j][1] = ap[1];                                                           \
-            }                                                                                 \
-        wload<T>(rowq, wr & 15, kbase + (K0) + sq, W);                                       \
-    } while (0)
-#define LRS_GSTAGE(BUF, A, W, K0)                                                             \
-    do {                                                                                      \
-        _Pragma("unroll") for (int p = 0; p < NS; p++)                                         \
-            _Pragma("unroll") for (int j = 0; j < AR; j++) {                                   \
-                *reinterpret_cast<u32x4 *>(&As[BUF][p][(sr + 128 * j) * GM_LD + sq]) = A[p][j][0];     \
-                *reinterpret_cast<u32x4 *>(&As[BUF][p][(sr + 128 * j) * GM_LD + sq + 8]) = A[p][j][1]; \
-            }                                                                                 \
-        float v_[16];                                                                         \
-        const DeqPrep dp_ = wprep<T>(W, kbase + (K0) + sq);                                   \
-        _Pragma("unroll") for (int c = 0; c < 4; c++) wdeq4<T>(W, dp_, c, v_);                \
-        put16<PREC>(&Ws[BUF][0][sr * GM_LD + sq], &Ws[BUF][NS - 1][sr * GM_LD + sq], v_);     \
-    } while (0)
-    // operand fragments of sub-step ks (K16) from LDS buffer buf
-    auto frag = [&](int buf, int ks, bf16x8 (&a)[NS][MT], bf16x8 (&b)[NS][NT]) __attribute__((always_inline)) {
-        const uint32_t kk = 16 * ks + 8 * (lane >> 5);
+    auto scale4 = [&](uint32_t sb, int i, int q) __attribute__((always_inline)) {
+        return *reinterpret_cast<const float4 *>(Ss + (sb & 1) * L::SUMS + i * 2048 + 1024 + 4 * (8 * q + 4 * hf));
+    };
+    // one half of a super-block from its LDS stage
+    // operands of a K-step: the activations' hi (and lo) parts, the weights'
+    // hi (and for Q6_K and Q8_0 lo) parts; precision 1 uses the hi members
+    constexpr bool LO = PREC == 3 && (T == T_Q6_K || T == T_Q8_0);
+    struct FragA { u32x4 h[MT], l[PREC == 3 ? MT : 1]; };
+    struct FragB { u32x4 h[NT], l[LO ? NT : 1]; };
+    // Half a super-block from its LDS stage.  The operands of K-step t + 1 are
+    // read and unpacked while step t's matrix operations run: the scheduling
+    // groups put about as many vector operations behind each matrix operation
+    // as there are.
+    auto compute = [&](int half, const uint8_t *As, WHalf<T> (&w)[NT], const uint8_t *nxt, int nhalf)
+                       __attribute__((always_inline)) {
+        SHalf<T> sc[NT];
+        AHalf<T> af[NT];
 #pragma unroll
-        for (int p = 0; p < NS; p++) {
+        for (int j = 0; j < NT; j++) {
+            if constexpr (PREC == 3) {
+                int ex = 0;
+                if constexpr (T == T_Q8_0) ex = q8_exp(w[j].d);
+                sc[j] = scales<T>(w[j], half, hf, ex);
+            } else {
+                af[j] = affine<T>(w[j], half, hf);
+            }
+        }
+        FragA fa[2];
+        FragB fb[2];
+        auto lfrag = [&](int t, FragA &A, FragB &B) __attribute__((always_inline)) {
 #pragma unroll
-            for (int u = 0; u < MT; u++)
-                a[p][u] = *reinterpret_cast<const bf16x8 *>(&As[buf][p][((BM / WM) * wm + 32 * u + (lane & 31)) * GM_LD + kk]);
+            for (int i = 0; i < MT; i++) {
+                A.h[i] = *reinterpret_cast<const u32x4 *>(As + (i * 8 + t) * L::STEP + 16 * lane);
+                if constexpr (PREC == 3)
+                    A.l[i] = *reinterpret_cast<const u32x4 *>(As + (i * 8 + t) * L::STEP + 1024 + 16 * lane);
+            }
 #pragma unroll
-            for (int u = 0; u < NT; u++)
-                b[p][u] = *reinterpret_cast<const bf16x8 *>(&Ws[buf][p][((GM_BN / WN) * wn + 32 * u + (lane & 31)) * GM_LD + kk]);
+            for (int j = 0; j < NT; j++) {
+                if constexpr (PREC == 3) {
+                    f16x8 bh, bl;
+                    bfrag_int<T>(w[j], sc[j], half, t, bh, bl);
+                    B.h[j] = __builtin_bit_cast(u32x4, bh);
+                    if constexpr (LO) B.l[j] = __builtin_bit_cast(u32x4, bl);
+                } else {
+                    B.h[j] = __builtin_bit_cast(u32x4, bfrag_bf16<T>(w[j], af[j], half, t));
+                }
+            }
+        };
+        auto mma = [&](const u32x4 &a, const u32x4 &b, f32x16 &c) __attribute__((always_inline)) {
+            if constexpr (PREC == 3)
+                c = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b),
+                                                           c, 0, 0, 0);
+            else
+                c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
+                                                            __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+        };
+        if (PREC == 3 && half == 0) {
+#pragma unroll
+            for (int i = 0; i < MT; i++)
+#pragma unroll
+                for (int j = 0; j < NT; j++)
+#pragma unroll
+                    for (int e = 0; e < 16; e++) acc[i][j][e] = 0.f;
+        }
+        lfrag(0, fa[0], fb[0]);
+#pragma unroll
+        for (int t = 0; t < 8; t++) {
+            if (t < 7) lfrag(t + 1, fa[(t + 1) & 1], fb[(t + 1) & 1]);
+            const FragA &A = fa[t & 1];
+            const FragB &B = fb[t & 1];
+            if constexpr (LO) {
+#pragma unroll
+                for (int j = 0; j < NT; j++)
+#pragma unroll
+                    for (int i = 0; i < MT; i++) mma(A.h[i], B.l[j], acc[i][j]);
+            }
+            if constexpr (PREC == 3) {
+#pragma unroll
+                for (int j = 0; j < NT; j++)
+#pragma unroll
+                    for (int i = 0; i < MT; i++) mma(A.l[i], B.h[j], acc[i][j]);
+            }
+#pragma unroll
+            for (int j = 0; j < NT; j++)
+#pragma unroll
+                for (int i = 0; i < MT; i++) mma(A.h[i], B.h[j], PREC == 3 ? acc[i][j] : tot[i][j]);
+            constexpr int NM = MT * NT * (LO ? 3 : PREC == 3 ? 2 : 1);  // matrix operations of a step
+            constexpr int NV = PREC == 1 ? (NT * 25 + NM - 1) / NM : LO ? 6 : 5;
+#pragma unroll
+            for (int z = 0; z < NM; z++) {
+                __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);   // a matrix operation
+                __builtin_amdgcn_sched_group_barrier(0x2, NV, 0);  // vector operations
+                if (z < (PREC == 3 ? 2 : 1) * MT) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // an LDS read
+            }
+            if constexpr (T == T_Q8_0) {
+                if (t & 1)
+#pragma unroll
+                    for (int j = 0; j < NT; j++) w[j].q[t >> 1] = q8_piece(nxt, wo[j], r, hf, nhalf, t >> 1);
+            }
         }
     };
-    auto mfma = [&](const bf16x8 (&a)[NS][MT], const bf16x8 (&b)[NS][NT]) __attribute__((always_inline)) {
+    // the super-block's whole-number sums times its scales, into the totals
+    auto fold = [&](uint32_t sb, const WHalf<T> (&w)[NT]) __attribute__((always_inline)) {
+        if constexpr (PREC == 3) {
 #pragma unroll
-        for (int i = 0; i < MT; i++)
-#pragma unroll
-            for (int jn = 0; jn < NT; jn++) {
-                if constexpr (PREC == 3) {
-                    acc[i][jn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1][i], b[0][jn], acc[i][jn], 0, 0, 0);
-                    acc[i][jn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0][i], b[1][jn], acc[i][jn], 0, 0, 0);
+            for (int j = 0; j < NT; j++) {
+                float d, dm = 0.f;
+                f16x8 mf;
+                if constexpr (T == T_Q6_K) {
+                    d = h2f((uint16_t)w[j].d);
+                } else if constexpr (T == T_Q8_0) {
+                    d = ldexpf(1.0f, q8_exp(w[j].d));
+                } else {
+                    d = h2f((uint16_t)(w[j].h0 & 0xFFFF));
+                    dm = h2f((uint16_t)(w[j].h0 >> 16));
+                    mf = min_frag(w[j]);
                 }
-                acc[i][jn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0][i], b[0][jn], acc[i][jn], 0, 0, 0);
-            }
-    };
-    // one pipeline step: step k's four K16 sub-steps from buffer buf (the
-    // fragments of sub-step ks+1 read while sub-step ks's matrix-core ops
-    // run), step k+1's activations copied into the other buffer first and
-    // its weights dequantized a quarter after each sub-step, so the VALU
-    // work overlaps the matrix cores
-#define LRS_GSTEP(BUF, A, W, K0)                                                              \
-    do {                                                                                      \
-        _Pragma("unroll") for (int p = 0; p < NS; p++)                                         \
-            _Pragma("unroll") for (int j = 0; j < AR; j++) {                                   \
-                *reinterpret_cast<u32x4 *>(&As[1 - (BUF)][p][(sr + 128 * j) * GM_LD + sq]) = A[p][j][0];     \
-                *reinterpret_cast<u32x4 *>(&As[1 - (BUF)][p][(sr + 128 * j) * GM_LD + sq + 8]) = A[p][j][1]; \
-            }                                                                                 \
-        const DeqPrep dp_ = wprep<T>(W, kbase + (K0) + sq);                                   \
-        float v_[16];                                                                         \
-        bf16x8 fa0[NS][MT], fb0[NS][NT], fa1[NS][MT], fb1[NS][NT];                            \
-        frag(BUF, 0, fa0, fb0);                                                               \
-        frag(BUF, 1, fa1, fb1);                                                               \
-        mfma(fa0, fb0);                                                                       \
-        wdeq4<T>(W, dp_, 0, v_);                                                              \
-        frag(BUF, 2, fa0, fb0);                                                               \
-        mfma(fa1, fb1);                                                                       \
-        wdeq4<T>(W, dp_, 1, v_);                                                              \
-        frag(BUF, 3, fa1, fb1);                                                               \
-        mfma(fa0, fb0);                                                                       \
-        wdeq4<T>(W, dp_, 2, v_);                                                              \
-        mfma(fa1, fb1);                                                                       \
-        wdeq4<T>(W, dp_, 3, v_);                                                              \
-        put16<PREC>(&Ws[1 - (BUF)][0][sr * GM_LD + sq], &Ws[1 - (BUF)][NS - 1][sr * GM_LD + sq], v_); \
-    } while (0)
-
-    const uint32_t nk = kspan / GM_BK;  // a multiple of 4
-    auto kc = [&](uint32_t k) { return min(k, nk - 1) * GM_BK; };  // look-ahead past the end repeats the last step (unused)
-    LRS_GFETCH(a0, w0, 0);
-    LRS_GFETCH(a1, w1, kc(1));
-    LRS_GFETCH(a2, w2, kc(2));
-    LRS_GSTAGE(0, a0, w0, 0);
-    __syncthreads();
-    for (uint32_t k = 0; k < nk; k += 4) {
-        LRS_GFETCH(a3, w3, kc(k + 3));
-        LRS_GSTEP(0, a1, w1, kc(k + 1));
-        __syncthreads();
-        LRS_GFETCH(a0, w0, kc(k + 4));
-        LRS_GSTEP(1, a2, w2, kc(k + 2));
-        __syncthreads();
-        LRS_GFETCH(a1, w1, kc(k + 5));
-        LRS_GSTEP(0, a3, w3, kc(k + 3));
-        __syncthreads();
-        LRS_GFETCH(a2, w2, kc(k + 6));
-        LRS_GSTEP(1, a0, w0, kc(k + 4));
-        __syncthreads();
-    }
-#undef LRS_GFETCH
-#undef LRS_GSTAGE
-#undef LRS_GSTEP
-    // D layout: lane l, register r -> row 8(r/4) + 4(l/32) + r%4, column l%32
 #pragma unroll
-    for (int jn = 0; jn < NT; jn++) {
-        const uint32_t n = n0 + (GM_BN / WN) * wn + 32 * jn + (lane & 31);
+                for (int i = 0; i < MT; i++) {
+                    f32x16 q;
+                    if constexpr (MINS) {
+                        const f16x8 sf =
+                            *reinterpret_cast<const f16x8 *>(Ss + (sb & 1) * L::SUMS + i * 2048 + 16 * lane);
+#pragma unroll
+                        for (int e = 0; e < 16; e++) q[e] = 0.f;
+                        q = __builtin_amdgcn_mfma_f32_32x32x16_f16(sf, mf, q, 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const float4 s = scale4(sb, i, e);
+                        const float sv[4] = {s.x, s.y, s.z, s.w};
+#pragma unroll
+                        for (int k = 0; k < 4; k++) {
+                            const int x = 4 * e + k;
+                            const float v = MINS ? fmaf(acc[i][j][x], d, -(q[x] * dm)) : acc[i][j][x] * d;
+                            tot[i][j][x] = fmaf(v, sv[k], tot[i][j][x]);
+                        }
+                    }
+                }
+            }
+        }
+    };
+    auto sync = [&]() __attribute__((always_inline)) {
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wavefront's copies and loads have arrived
+        __syncthreads();
+    };
+
+    // Stages of half a super-block: the next stage's copy and weight loads are
+    // issued first, then the current one computes from the other LDS array.
+    // Q8_0 holds one set of weight registers (its pieces are the widest) and
+    // refills each piece once its K-steps are done.
+    WHalf<T> w0[NT], w1[NT];
+    const uint8_t *cw = wp + (size_t)s0 * CH;
+    dma(s0, 0, As0);
+    dma_sums(s0);
+#pragma unroll
+    for (int j = 0; j < NT; j++) wload<T, PREC>(cw, wo[j], r, hf, 0, w0[j]);
+    sync();
+    for (uint32_t sb = s0; sb < s1; sb++) {
+        const uint32_t nx = min(sb + 1, s1 - 1);  // past the end: the last block again, unused
+        const uint8_t *nw = wp + (size_t)nx * CH;
+        dma(sb, 1, As1);
+        if constexpr (T != T_Q8_0)
+#pragma unroll
+            for (int j = 0; j < NT; j++) wload<T, PREC>(cw, wo[j], r, hf, 1, w1[j]);
+        __builtin_amdgcn_sched_barrier(0);
+        compute(0, As0, w0, cw, 1);
+        sync();
+        dma(nx, 0, As0);
+        if (sb + 1 < s1) dma_sums(nx);
+        if constexpr (T != T_Q8_0)
+#pragma unroll
+            for (int j = 0; j < NT; j++) wload<T, PREC>(nw, wo[j], r, hf, 0, w0[j]);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (T == T_Q8_0) {
+            compute(1, As1, w0, nw, 0);
+            fold(sb, w0);
+#pragma unroll
+            for (int j = 0; j < NT; j++)
+#pragma unroll
+                for (int u = 0; u < 4; u++)
+                    w0[j].d[u] = *reinterpret_cast<const uint32_t *>(nw + u * 1088 + 1024 + (wo[j] + 4 * r));
+        } else {
+            compute(1, As1, w1, nw, 0);
+            fold(sb, w1);
+        }
+        cw = nw;
+        sync();
+    }
+    // D layout: lane l, register e -> row 8(e/4) + 4(l/32) + e%4, column l%32
+#pragma unroll
+    for (int j = 0; j < NT; j++) {
+        const uint32_t n = nw0 + 32 * j + (lane & 31);
+        if (n >= sg.N) continue;
 #pragma unroll
         for (int i = 0; i < MT; i++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const uint32_t m = m0 + (BM / WM) * wm + 32 * i + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                if (m < g.M && n < sg.N) {
+            for (int e = 0; e < 16; e++) {
+                const uint32_t m = 32 * (mb * MT + i) + 8 * (e >> 2) + 4 * hf + (e & 3);
+                if (m < g.M) {
                     if (g.ks > 1) {
-                        g.part[((size_t)kz * g.M + m) * sg.N + n] = acc[i][jn][r];
+                        g.part[((size_t)kz * g.M + m) * g.ntot + sg.noff + n] = tot[i][j][e];
                     } else {
                         float *o = sg.y + (size_t)m * sg.ldy + n;
-                        *o = g.accum ? *o + acc[i][jn][r] : acc[i][jn][r];
+                        *o = g.accum ? *o + tot[i][j][e] : tot[i][j][e];
                     }
                 }
             }
     }
 }
+};
 
-// workgroup b takes output tile t0 of the (K slice, M block, N tile) order;
-// the segment of its N tile picks the weight and the type (T0 for the first
-// nseg0 segments, T1 after them); MS = the most segments the instance takes
-// (1: single-weight launches).  Tile order: workgroup b runs on XCD b % 8
-// (round-robin dispatch); the tiles are numbered M-block-major and XCD x
-// takes the x-th contiguous run of them, so the workgroups of one XCD share
-// one or two activation blocks, which stay in that XCD's L2.
-template <uint32_t T0, uint32_t T1, int PREC, int BM, int MS>
-__global__ __launch_bounds__(512) void k_gemm(GemmArgs g) {
-    constexpr int NS = PREC == 3 ? 2 : 1;
-    __shared__ __attribute__((aligned(16))) __bf16 As[2][NS][BM * GM_LD];
-    __shared__ __attribute__((aligned(16))) __bf16 Ws[2][NS][GM_BN * GM_LD];
+template <uint32_t T0, uint32_t T1, int PREC, int MT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_pgemm(PgArgs g) {
+    using L = PgLds<PREC, MT>;
+    constexpr int NT = 2;  // weight-row tiles of 32 per wavefront
+    __shared__ __attribute__((aligned(16))) uint8_t As0[L::STAGE];
+    __shared__ __attribute__((aligned(16))) uint8_t As1[L::STAGE];
+    __shared__ __attribute__((aligned(16))) uint8_t Ss[2 * L::SUMS];
     const uint32_t ntile = g.nm * g.nn * g.ks, per = (ntile + 7) / 8;
     const uint32_t t0 = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-    if (t0 >= ntile) return;
-    const uint32_t kz = t0 / (g.nm * g.nn), t = t0 % (g.nm * g.nn);  // K slice, output tile
-    const uint32_t nt = t % g.nn;
+    if ((blockIdx.x >> 3) >= per || t0 >= ntile) return;
+    const uint32_t mb = t0 % g.nm, t = t0 / g.nm, nt = t % g.nn, kz = t / g.nn;
     uint32_t si = 0;
 #pragma unroll
-    for (int i = 1; i < MS; i++)
+    for (int i = 1; i < PG_MAX_SEG; i++)
         if ((uint32_t)i < g.nseg && nt >= g.seg[i].nt0) si = i;
-    const GemmSeg sg = g.seg[si];
-    const uint32_t m0 = (t / g.nn) * BM, n0 = (nt - sg.nt0) * GM_BN;
+    const PgSeg sg = g.seg[si];
+    const uint32_t n0 = (nt - sg.nt0) * 32 * NT * PG_WAVES;
     if (T0 == T1 || si < g.nseg0)
-        gemm_tile<T0, PREC, BM>(g, sg, kz, m0, n0, As, Ws);
+        PgTile<T0, PREC, MT, NT>::run(g, sg, kz, mb, n0, As0, As1, Ss);
     else
-        gemm_tile<T1, PREC, BM>(g, sg, kz, m0, n0, As, Ws);
+        PgTile<T1, PREC, MT, NT>::run(g, sg, kz, mb, n0, As0, As1, Ss);
 }
 
-// y[m][n] (+)= sum over the K slices of part[z][m][n], slices in order
-__global__ __launch_bounds__(256) void k_reduce_ks(const float *__restrict__ part, float *__restrict__ y,
-                                                   uint32_t M, uint32_t N, uint32_t ldy, uint32_t ks,
-                                                   uint32_t accum) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= (size_t)M * N) return;
-    const uint32_t m = (uint32_t)(i / N), n = (uint32_t)(i % N);
-    float v = part[i];
-    for (uint32_t z = 1; z < ks; z++) v += part[(size_t)z * M * N + i];
-    float *o = y + (size_t)m * ldy + n;
-    *o = accum ? *o + v : v;
+
+
+// y[m][n] (+)= sum over the K slices of part[z][m][noff + n], slices in order,
+// four outputs per thread (N % 4 == 0, else one)
+template <int V>
+__global__ __launch_bounds__(256) void k_reduce_ks(PgArgs g) {
+    const PgSeg sg = g.seg[blockIdx.z];
+    const uint32_t n = V * (blockIdx.x * 256 + threadIdx.x), m = blockIdx.y;
+    if (n >= sg.N) return;
+    typedef __attribute__((ext_vector_type(V))) float fv;
+    const float *p = g.part + (size_t)m * g.ntot + sg.noff + n;
+    const size_t st = (size_t)g.M * g.ntot;
+    fv v = *reinterpret_cast<const fv *>(p);
+    for (uint32_t z = 1; z < g.ks; z++) v += *reinterpret_cast<const fv *>(p + z * st);
+    fv *o = reinterpret_cast<fv *>(sg.y + (size_t)m * sg.ldy + n);
+    *o = g.accum ? *o + v : v;
 }
 
-// a -> bf16 hi (round to nearest even) and, if lo, bf16(a - hi): the
-// activation planes of the GEMM, 4 elements per thread
-__global__ __launch_bounds__(256) void k_split_bf16(const float *__restrict__ a, size_t n4,
-                                                    __bf16 *__restrict__ hi, __bf16 *__restrict__ lo) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n4) return;
-    const float4 v = reinterpret_cast<const float4 *>(a)[i];
-    typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
-    bf16x4 h, l;
-    h[0] = to_bf16(v.x);
-    h[1] = to_bf16(v.y);
-    h[2] = to_bf16(v.z);
-    h[3] = to_bf16(v.w);
-    reinterpret_cast<bf16x4 *>(hi)[i] = h;
-    if (lo) {
-        l[0] = to_bf16(v.x - (float)h[0]);
-        l[1] = to_bf16(v.y - (float)h[1]);
-        l[2] = to_bf16(v.z - (float)h[2]);
-        l[3] = to_bf16(v.w - (float)h[3]);
-        reinterpret_cast<bf16x4 *>(lo)[i] = l;
+// rows of f32 into the GEMM's input layout: workgroup = 32 rows x one super-block
+template <int PREC>
+__global__ __launch_bounds__(256) void k_gemm_pack(const float *__restrict__ a, uint32_t M, uint32_t nsb,
+                                                   uint8_t *__restrict__ p) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const uint32_t row = 32 * (blockIdx.x / nsb) + 8 * i + (threadIdx.x >> 5);
+        const uint32_t c = 32 * (blockIdx.x % nsb) + (threadIdx.x & 31);
+        if (row >= M) return;
+        const float *x = a + ((size_t)row * nsb) * 256 + 8 * c;
+        const float4 u = *reinterpret_cast<const float4 *>(x), w = *reinterpret_cast<const float4 *>(x + 4);
+        const float v[8] = {u.x, u.y, u.z, u.w, w.x, w.y, w.z, w.w};
+        gp_store8<PREC>(v, row, c, nsb, p);
     }
 }
 
-hipError_t launch_split_bf16(const float *a, size_t n, __bf16 *hi, __bf16 *lo, hipStream_t s) {
-    if (n % 4) return hipErrorInvalidValue;
-    const size_t n4 = n / 4;
-    hipLaunchKernelGGL(k_split_bf16, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, a, n4, hi, lo);
+hipError_t launch_gemm_pack(const float *a, uint32_t M, uint32_t K, int prec, uint8_t *planes, hipStream_t s) {
+    if (M == 0 || K == 0 || K % 256) return hipErrorInvalidValue;
+    const dim3 grid((M + 31) / 32 * (K / 256));
+    if (prec == 3)
+        hipLaunchKernelGGL((k_gemm_pack<3>), grid, dim3(256), 0, s, a, M, K / 256, planes);
+    else
+        hipLaunchKernelGGL((k_gemm_pack<1>), grid, dim3(256), 0, s, a, M, K / 256, planes);
     return hipGetLastError();
 }
 
-// K slices for a GEMM with fewer output tiles than CUs (the long-K o / down
-// projections): the slice count ks divides K into whole super-blocks and
-// minimises the rounds of 256 workgroups (one per CU) each slice-sized unit
-// of work takes, ceil(tiles * ks / 256) / ks, plus a small charge for the
-// reduction pass; ties keep fewer slices
-// token tile: 256 for bf16 operands at M >= 512 (twice the MFMA work per
-// dequantized weight: the dequant, not the matrix cores, bounds the 128-row
-// tile), else 128; the hi/lo form keeps 128 (its LDS would not fit)
-static uint32_t gemm_bm(uint32_t M, int prec) { return prec == 1 && M >= 512 ? 256u : 128u; }
+size_t gemm_planes_bytes(uint32_t M, uint32_t K, int prec) {
+    return (size_t)((M + 31) / 32) * (K / 256) * gemm_block_bytes(prec);
+}
 
-static uint32_t ksplit_for(uint32_t tiles, uint32_t K) {
-    const uint32_t units = K / 256;
-    uint32_t best = 1;
-    if (tiles >= 256) return 1;  // a full round already; partial traffic would cost more
-    double best_cost = 1.0;
-    for (uint32_t ks = 2; ks <= 8; ks++) {
-        if (units % ks || units / ks < 4) continue;
-        const double cost = (double)((tiles * ks + 255) / 256) / ks + 0.05;
-        if (cost < best_cost - 1e-9) {
-            best_cost = cost;
-            best = ks;
+constexpr uint32_t PG_ROWS = 64 * PG_WAVES;  // weight rows of a workgroup
+
+// Launch shape of a GEMM: row tiles of 32 tokens per workgroup, K slices.
+struct PgPlan {
+    uint32_t mt, ks;
+};
+
+static uint32_t pg_tiles(uint32_t M, const uint32_t *N, uint32_t nseg, uint32_t mt) {
+    uint32_t nn = 0;
+    for (uint32_t i = 0; i < nseg; i++) nn += (N[i] + PG_ROWS - 1) / PG_ROWS;
+    return (M + 32 * mt - 1) / (32 * mt) * nn;
+}
+
+// us per super-block of n workgroups that share a CU, measured with Q4_K
+// weights at K = 5120: the first workgroups of a CU hide each other's waits
+static double pg_unit(int prec, uint32_t mt, uint32_t n) {
+    static const double p3m1[3] = {2.4, 3.3, 6.2}, p3m2[2] = {3.6, 6.4};
+    static const double p1m1[3] = {2.0, 3.0, 4.2}, p1m2[3] = {2.7, 4.8, 6.4}, p1m4[2] = {4.4, 7.8};
+    const double *c = prec == 3 ? (mt == 1 ? p3m1 : p3m2) : mt == 1 ? p1m1 : mt == 2 ? p1m2 : p1m4;
+    const uint32_t full = mt == (prec == 3 ? 2u : 4u) ? 2 : 3;
+    return n / full * c[full - 1] + (n % full ? c[n % full - 1] : 0.0);
+}
+
+// The shape with the least expected time: the workgroups that a CU gets, and
+// for K slices the partial sums written and read back (at about 8 TB/s, most
+// of them in the memory-side cache) and the launch that adds them.
+// have_work: K slices may be used
+static PgPlan pg_plan(uint32_t M, const uint32_t *N, uint32_t nseg, uint32_t nsb, uint32_t type, int prec,
+                      bool have_work) {
+    // precision 3: Q6_K and Q8_0 take a third product, Q5_K more unpacking
+    const double rel = prec == 1 || type == T_Q4_K ? 1.0 : type == T_Q5_K ? 1.2 : 1.5;
+    uint32_t ntot = 0;
+    for (uint32_t i = 0; i < nseg; i++) ntot += N[i];
+    PgPlan best = {1, 1};
+    double best_cost = 1e30;
+    for (uint32_t mt = 1; mt <= (prec == 3 ? 2u : 4u); mt *= 2) {
+        if (mt > 1 && M <= 16 * mt) break;
+        const uint32_t tiles = pg_tiles(M, N, nseg, mt);
+        for (uint32_t ks = 1; ks <= nsb && ks <= 32; ks++) {
+            if (ks > 1 && (!have_work || tiles >= 2048)) break;
+            const uint32_t len = (nsb + ks - 1) / ks;
+            double cost = (len + 0.5) * rel * pg_unit(prec, mt, (tiles * ks + 255) / 256);
+            if (ks > 1) cost += 4.0 + (2.0 * ks + 1) * M * ntot * 4.0 / 8e6;
+            if (cost < best_cost * 0.999) {
+                best_cost = cost;
+                best = {mt, ks};
+            }
         }
     }
     return best;
 }
 
-uint32_t gemm_out_tiles(uint32_t M, uint32_t N, int prec) {
-    const uint32_t bm = gemm_bm(M, prec);
-    return ((M + bm - 1) / bm) * ((N + GM_BN - 1) / GM_BN);
+// scratch of the K-sliced form for any row count up to M (a smaller one may
+// split over more slices): a caller that made its largest call first never
+// needs more
+size_t gemm_work_bytes(uint32_t M, const uint32_t *N, uint32_t nseg, uint32_t K, uint32_t type, int prec) {
+    uint32_t ntot = 0;
+    for (uint32_t i = 0; i < nseg; i++) ntot += N[i];
+    size_t most = 0;
+    for (uint32_t m = M;; m = (m - 1) / 32 * 32) {
+        const uint32_t ks = pg_plan(m, N, nseg, K / 256, type, prec, true).ks;
+        if (ks > 1) most = std::max(most, (size_t)ks * m * ntot * sizeof(float));
+        if (m <= 32) break;
+    }
+    return most;
 }
 
-uint32_t gemm_ksplit(uint32_t M, uint32_t N, uint32_t K, int prec) {
-    const uint32_t bm = gemm_bm(M, prec);
-    return ksplit_for(((M + bm - 1) / bm) * ((N + GM_BN - 1) / GM_BN), K);
-}
+using GemmFn = void (*)(PgArgs);
 
-// scratch of the K-sliced form (at most 8 * M * N floats)
-size_t gemm_work_bytes(uint32_t M, uint32_t N, uint32_t K, int prec) {
-    const uint32_t ks = gemm_ksplit(M, N, K, prec);
-    return ks > 1 ? (size_t)ks * M * N * sizeof(float) : 0;
+template <uint32_t T0, uint32_t T1>
+static GemmFn pick_gemm_shape(int prec, uint32_t mt) {
+    if (prec == 3) return mt == 1 ? k_pgemm<T0, T1, 3, 1> : k_pgemm<T0, T1, 3, 2>;
+    return mt == 1 ? k_pgemm<T0, T1, 1, 1> : mt == 2 ? k_pgemm<T0, T1, 1, 2> : k_pgemm<T0, T1, 1, 4>;
 }
-
-using GemmFn = void (*)(GemmArgs);
 
 // the kernel for weight types t0 (the first segments) and t1 (the rest)
-template <uint32_t T0>
-static GemmFn pick_gemm_t0(uint32_t t1, uint32_t nseg, int prec, uint32_t bm) {
-#define LRS_GEMM_PICK(T1, MS)                                                             \
-    return prec == 3 ? k_gemm<T0, T1, 3, 128, MS>                                         \
-                     : bm == 256 ? k_gemm<T0, T1, 1, 256, MS> : k_gemm<T0, T1, 1, 128, MS>
-    if (t1 == T0 && nseg == 1) { LRS_GEMM_PICK(T0, 1); }
-    if (t1 == T0) { LRS_GEMM_PICK(T0, GM_MAX_SEG); }
+static GemmFn pick_gemm(uint32_t t0, uint32_t t1, int prec, uint32_t mt) {
+    if (t0 == T_Q4_K && t1 == T_Q4_K) return pick_gemm_shape<T_Q4_K, T_Q4_K>(prec, mt);
+    if (t0 == T_Q5_K && t1 == T_Q5_K) return pick_gemm_shape<T_Q5_K, T_Q5_K>(prec, mt);
+    if (t0 == T_Q6_K && t1 == T_Q6_K) return pick_gemm_shape<T_Q6_K, T_Q6_K>(prec, mt);
+    if (t0 == T_Q8_0 && t1 == T_Q8_0) return pick_gemm_shape<T_Q8_0, T_Q8_0>(prec, mt);
     // a prompt block's q / k with a Q6_K v (the K-quant mixes)
-    if constexpr (T0 == T_Q4_K || T0 == T_Q5_K)
-        if (t1 == T_Q6_K) { LRS_GEMM_PICK(T_Q6_K, GM_MAX_SEG); }
-#undef LRS_GEMM_PICK
+    if (t0 == T_Q4_K && t1 == T_Q6_K) return pick_gemm_shape<T_Q4_K, T_Q6_K>(prec, mt);
+    if (t0 == T_Q5_K && t1 == T_Q6_K) return pick_gemm_shape<T_Q5_K, T_Q6_K>(prec, mt);
     return nullptr;
-}
-static GemmFn pick_gemm(uint32_t t0, uint32_t t1, uint32_t nseg, int prec, uint32_t bm) {
-    switch (t0) {
-    case T_Q4_K: return pick_gemm_t0<T_Q4_K>(t1, nseg, prec, bm);
-    case T_Q5_K: return pick_gemm_t0<T_Q5_K>(t1, nseg, prec, bm);
-    case T_Q6_K: return pick_gemm_t0<T_Q6_K>(t1, nseg, prec, bm);
-    case T_Q8_0: return pick_gemm_t0<T_Q8_0>(t1, nseg, prec, bm);
-    default: return nullptr;
-    }
 }
 
 bool gemm_segs_supported(const WeightView *w, uint32_t nseg) {
-    if (nseg == 0 || nseg > (uint32_t)GM_MAX_SEG) return false;
+    if (nseg == 0 || nseg > (uint32_t)PG_MAX_SEG) return false;
     uint32_t nseg0 = 1;
     while (nseg0 < nseg && w[nseg0].type == w[0].type) nseg0++;
     for (uint32_t i = 0; i < nseg; i++) {
         if (w[i].n_in != w[0].n_in || !is_tiled(w[i].type)) return false;
         if (i >= nseg0 && w[i].type != w[nseg0].type) return false;  // at most two types, in two runs
     }
-    return pick_gemm(w[0].type, w[nseg - 1].type, nseg, 3, 128) != nullptr;
+    return pick_gemm(w[0].type, w[nseg - 1].type, 3, 1) != nullptr;
 }
 
 hipError_t launch_gemm_segs(const WeightView *w, float *const *y, const uint32_t *ldy, uint32_t nseg,
-                            const __bf16 *ahi, const __bf16 *alo, uint32_t M, int prec,
-                            hipStream_t s, bool accum, float *work, uint32_t *ks_out) {
-    if (M == 0 || nseg == 0 || nseg > (uint32_t)GM_MAX_SEG || (prec == 3 && !alo))
+                            const uint8_t *planes, uint32_t M, int prec, hipStream_t s, bool accum, float *work,
+                            size_t work_bytes, uint32_t *ks_out) {
+    if (M == 0 || !planes || !gemm_segs_supported(w, nseg) || w[0].n_in == 0 || w[0].n_in % 256)
         return hipErrorInvalidValue;
-    if (!gemm_segs_supported(w, nseg) || w[0].n_in % (4 * GM_BK)) return hipErrorInvalidValue;
-    const uint32_t bm = gemm_bm(M, prec);
-    GemmArgs g = {};
-    g.ahi = ahi;
-    g.alo = alo;
+    uint32_t Ns[PG_MAX_SEG];
+    for (uint32_t i = 0; i < nseg; i++) Ns[i] = w[i].n_out;
+    PgPlan p = pg_plan(M, Ns, nseg, w[0].n_in / 256, w[0].type, prec, work != nullptr);
+    PgArgs g = {};
+    g.a = planes;
     g.nseg = nseg;
     g.nseg0 = 1;
     while (g.nseg0 < nseg && w[g.nseg0].type == w[0].type) g.nseg0++;
-    uint32_t nt = 0;
+    uint32_t nt = 0, ntot = 0, nmax = 0;
+    bool v4 = true;
     for (uint32_t i = 0; i < nseg; i++) {
-        g.seg[i].q = w[i].q;
-        g.seg[i].y = y[i];
-        g.seg[i].N = w[i].n_out;
-        g.seg[i].ldy = ldy[i];
-        g.seg[i].nt0 = nt;
-        nt += (w[i].n_out + GM_BN - 1) / GM_BN;
+        const uint32_t N = w[i].n_out;
+        g.seg[i] = {w[i].q, y[i], N, ldy[i], nt, ntot};
+        nt += (N + PG_ROWS - 1) / PG_ROWS;
+        ntot += N;
+        nmax = std::max(nmax, N);
+        v4 = v4 && N % 4 == 0 && ldy[i] % 4 == 0 && ((uintptr_t)y[i] & 15) == 0;
     }
     g.M = M;
-    g.K = w[0].n_in;
+    g.nsb = w[0].n_in / 256;
     g.accum = accum ? 1u : 0u;
-    g.nm = (M + bm - 1) / bm;
+    if (p.ks > 1 && (size_t)p.ks * M * ntot * sizeof(float) > work_bytes)
+        p = pg_plan(M, Ns, nseg, g.nsb, w[0].type, prec, false);
+    g.nm = (M + 32 * p.mt - 1) / (32 * p.mt);
     g.nn = nt;
-    // K slices write [M][N] partials of one weight: one-segment launches only
-    g.ks = work && nseg == 1 ? ksplit_for(g.nm * g.nn, g.K) : 1;
+    g.ntot = ntot;
+    g.ks = p.ks;
     g.part = work;
-    const GemmFn fn = pick_gemm(w[0].type, w[nseg - 1].type, nseg, prec, bm);
-    if (!fn) return hipErrorNotSupported;
+    const GemmFn fn = pick_gemm(w[0].type, w[nseg - 1].type, prec, p.mt);
     const uint32_t grid = 8 * ((g.nm * g.nn * g.ks + 7) / 8);
-    hipLaunchKernelGGL(fn, dim3(grid), dim3(512), 0, s, g);
+    hipLaunchKernelGGL(fn, dim3(grid), dim3(64 * PG_WAVES), 0, s, g);
     if (ks_out) {
         *ks_out = g.ks;  // the caller reduces the slices (launch_reduce_norm_rows)
     } else if (g.ks > 1) {
-        const size_t n = (size_t)M * g.seg[0].N;
-        hipLaunchKernelGGL(k_reduce_ks, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, work,
-                           y[0], M, g.seg[0].N, ldy[0], g.ks, g.accum);
+        if (v4)
+            hipLaunchKernelGGL((k_reduce_ks<4>), dim3((nmax + 1023) / 1024, M, nseg), dim3(256), 0, s, g);
+        else
+            hipLaunchKernelGGL((k_reduce_ks<1>), dim3((nmax + 255) / 256, M, nseg), dim3(256), 0, s, g);
     }
     return hipGetLastError();
-}
-
-hipError_t launch_gemm(WeightView w, const __bf16 *ahi, const __bf16 *alo, float *y, uint32_t M,
-                       uint32_t ldy, int prec, hipStream_t s, bool accum, float *work,
-                       uint32_t *ks_out) {
-    if (!is_tiled(w.type)) return hipErrorNotSupported;
-    return launch_gemm_segs(&w, &y, &ldy, 1, ahi, alo, M, prec, s, accum, work, ks_out);
 }
 
 }  // namespace lrs

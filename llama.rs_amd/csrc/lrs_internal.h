@@ -70,6 +70,9 @@ inline size_t weight_dev_bytes(uint32_t t, uint32_t n_in, uint32_t n_out) {
     return (size_t)(n_in / block_elems(t)) * n_out * block_bytes(t);
 }
 
+// bytes of one (32 rows, 256 elements) block of a GEMM input (gemm_pack.h)
+__host__ __device__ constexpr uint32_t gemm_block_bytes(int prec) { return prec == 3 ? 34816u : 16384u; }
+
 // launch wrappers implemented in the .hip files (all enqueue on `s`)
 hipError_t launch_repack_from_gguf(const uint8_t *gguf_dev, WeightView w, uint8_t *q,
                                    hipStream_t s);
@@ -135,38 +138,32 @@ hipError_t launch_q8norm(const float *x, const float *w, uint32_t n, float eps, 
 // launch_matvec with each column rounded to Q8_0 first (Q8_0 weights only)
 hipError_t launch_matvec_actq(WeightView w, const float *x, float *y, uint32_t cols, void *pack,
                               int half_even, hipStream_t s);
-// Y[M][ldy] = A[M][K] W^T on the matrix cores; A given as bf16 planes
-// (prec 1: hi only; 3: hi + lo, three products) from launch_split_bf16
-// work: gemm_work_bytes(M, N, K, prec) of scratch for the K-sliced form (null: one slice)
-// ks_out: when given, a K split leaves its ks_out slices of [M][N] partials in
-// work for the caller to reduce (ks_out 1: y written directly)
-hipError_t launch_gemm(WeightView w, const __bf16 *ahi, const __bf16 *alo, float *y, uint32_t M,
-                       uint32_t ldy, int prec, hipStream_t s, bool accum = false,
-                       float *work = nullptr, uint32_t *ks_out = nullptr);
-size_t gemm_work_bytes(uint32_t M, uint32_t N, uint32_t K, int prec);
-// several weights over the same A in one launch (their output tiles side by
-// side; y[i] [M][ldy[i]]): at most 3, the same n_in, at most two types with
-// the first type's weights first and only the pairs the kernel is built for
-// (one type; Q4_K or Q5_K then Q6_K); no K split
+// Prompt GEMM (gemm.hip).  Its input is packed (gemm_pack.h) by
+// launch_gemm_pack or by the kernel that makes the rows, K a multiple of 256.
+hipError_t launch_gemm_pack(const float *a, uint32_t M, uint32_t K, int prec, uint8_t *planes, hipStream_t s);
+size_t gemm_planes_bytes(uint32_t M, uint32_t K, int prec);
+// y[i][M][ldy[i]] (+)= A[M][K] W[i]^T for up to 3 weights over the same A in
+// one launch (their output tiles side by side): the same n_in, at most two
+// types with the first type's weights first and only the pairs the kernel is
+// built for (one type; Q4_K or Q5_K then Q6_K).
+// work (gemm_work_bytes): scratch of the K-sliced form (null or too small: one slice)
+// ks_out: when given, a K split leaves its ks_out slices of [M][sum of N]
+// partials in work for the caller to reduce (ks_out 1: y written directly)
 bool gemm_segs_supported(const WeightView *w, uint32_t nseg);
-// output tiles (workgroups without a K split) of an M x N GEMM
-uint32_t gemm_out_tiles(uint32_t M, uint32_t N, int prec);
+size_t gemm_work_bytes(uint32_t M, const uint32_t *N, uint32_t nseg, uint32_t K, uint32_t type, int prec);
 hipError_t launch_gemm_segs(const WeightView *w, float *const *y, const uint32_t *ldy, uint32_t nseg,
-                            const __bf16 *ahi, const __bf16 *alo, uint32_t M, int prec,
-                            hipStream_t s, bool accum = false, float *work = nullptr,
-                            uint32_t *ks_out = nullptr);
-// hi = bf16(a), lo = bf16(a - hi) (lo may be null); n a multiple of 4
-hipError_t launch_split_bf16(const float *a, size_t n, __bf16 *hi, __bf16 *lo, hipStream_t s);
+                            const uint8_t *planes, uint32_t M, int prec, hipStream_t s, bool accum = false,
+                            float *work = nullptr, size_t work_bytes = 0, uint32_t *ks_out = nullptr);
 // batched prompt block (prefill.hip)
-// Y = RMSNorm rows of X times w (Y may be null), and, when hi is given, the
-// same values as the bf16 planes of launch_split_bf16 ([n][E] hi, then lo)
+// RMSNorm rows of X times w as a GEMM input of precision 3 (planes), and in
+// f32 when Y is given; E a multiple of 256
 hipError_t launch_rmsnorm_rows(const float *X, const float *w, float eps, uint32_t E, uint32_t n,
-                               float *Y, hipStream_t s, __bf16 *hi = nullptr);
+                               float *Y, uint8_t *planes, hipStream_t s);
 // X += the ks K-slice partials part[z][n][E] (slices in order, as
 // k_reduce_ks), then the RMSNorm rows of the new X times w as
-// launch_rmsnorm_rows writes them (Y may be null; hi planes)
+// launch_rmsnorm_rows writes them
 hipError_t launch_reduce_norm_rows(const float *part, uint32_t ks, float *X, const float *w,
-                                   float eps, uint32_t E, uint32_t n, float *Y, __bf16 *hi,
+                                   float eps, uint32_t E, uint32_t n, float *Y, uint8_t *planes,
                                    hipStream_t s);
 hipError_t launch_qkv_post(const float *qt, const float *kt, const float *vt, const float *bq,
                            const float *bk, const float *bv, const float *freq, float *q,
@@ -176,10 +173,9 @@ hipError_t launch_qkv_post(const float *qt, const float *kt, const float *vt, co
 hipError_t launch_attn_prefill(const float *q, const _Float16 *kc, const _Float16 *vc, float *out,
                                uint32_t n, uint32_t pos0, uint32_t n_head, uint32_t n_kv,
                                uint32_t hd, uint32_t ctx, hipStream_t s);
-// silu(G) * U written straight to the bf16 planes of launch_split_bf16 (hi,
-// then lo = hi + n); n a multiple of 4
-hipError_t launch_swiglu_split(const float *G, const float *U, size_t n, __bf16 *hi,
-                               hipStream_t s);
+// silu(G) * U [n][F] as a GEMM input of precision 3; F a multiple of 256
+hipError_t launch_swiglu_pack(const float *G, const float *U, uint32_t F, uint32_t n, uint8_t *planes,
+                              hipStream_t s);
 // hybrid (qwen35) mixers (dn.hip)
 // QK-norm + RoPE of the hybrid's gated attention run by the split kernel
 // (attention.hip, QP): query rows from the projection's q + gate rows, the

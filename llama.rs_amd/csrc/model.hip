@@ -173,7 +173,7 @@ struct lrs_model {
     // gate / up, token ids
     uint32_t pb_cap = 0;
     float *pX = nullptr, *pXN, *pQt, *pKt, *pVt, *pQ, *pATT, *pG, *pU;
-    __bf16 *pA16 = nullptr;  // bf16 hi / lo planes of the current GEMM input
+    uint8_t *pA = nullptr;  // the current GEMM input (gemm_pack.h)
     // hybrid blocks: Q + gate rows, conv in / out, output gate, rule output,
     // gated norm, per-(token, head) gates
     float *pQG = nullptr, *pCI = nullptr, *pCO = nullptr, *pZ = nullptr, *pO = nullptr,
@@ -1249,6 +1249,32 @@ static bool prefill_capable(const lrs_model *m) {
     return true;
 }
 
+// scratch of the K-sliced GEMMs of a prompt block
+static size_t prefill_work_bytes(const lrs_model *m) {
+    size_t most = 0;
+    auto need = [&](std::initializer_list<const lrs_weight *> ws) {
+        uint32_t N[3], n = 0;
+        for (const lrs_weight *w : ws) {
+            const uint32_t one = w->v.n_out;
+            most = std::max(most, gemm_work_bytes(PREFILL_BLOCK, &one, 1, w->v.n_in, w->v.type, 3));
+            N[n++] = one;
+        }
+        most = std::max(most, gemm_work_bytes(PREFILL_BLOCK, N, n, (*ws.begin())->v.n_in, (*ws.begin())->v.type, 3));
+    };
+    for (const DevLayer &L : m->layers) {
+        need({L.gate, L.up});
+        need({L.down});
+        if (L.dn) {
+            need({L.ssm_qkv, L.ssm_gate});
+            need({L.ssm_out});
+        } else {
+            need({L.q, L.k, L.v});
+            need({L.o});
+        }
+    }
+    return std::max<size_t>(most, 256);
+}
+
 static int ensure_prefill(lrs_model *m) {
     if (m->pb_cap) return LRS_OK;
     const lrs_config &c = m->cfg;
@@ -1264,13 +1290,14 @@ static int ensure_prefill(lrs_model *m) {
         (rc = dev_alloc(m, B * qd * 4, (void **)&m->pATT)) ||
         (rc = dev_alloc(m, B * c.n_ff * 4, (void **)&m->pG)) ||
         (rc = dev_alloc(m, B * c.n_ff * 4, (void **)&m->pU)) ||
-        (rc = dev_alloc(m, B * std::max<size_t>(std::max<size_t>(c.n_embd, qd),
-                                                std::max<size_t>(c.n_ff, (size_t)m->hc.dn_v_heads *
-                                                                             m->hc.dn_state)) * 4,
-                        (void **)&m->pA16)) ||
-        // K-sliced GEMMs (few output tiles: o, down, and the narrow k / v):
-        // 8 slices of [rows][n_embd] partials
-        (rc = dev_alloc(m, m->work_bytes = 8 * B * c.n_embd * 4, (void **)&m->pWork)) ||
+        (rc = dev_alloc(m,
+                        gemm_planes_bytes(PREFILL_BLOCK,
+                                          std::max({c.n_embd, (uint32_t)qd, c.n_ff, m->hc.dn_v_heads * m->hc.dn_state}),
+                                          3),
+                        (void **)&m->pA)) ||
+        // K-sliced GEMMs (few output tiles): the most that any projection of a
+        // block of up to B tokens asks for
+        (rc = dev_alloc(m, m->work_bytes = prefill_work_bytes(m), (void **)&m->pWork)) ||
         (rc = dev_alloc(m, B * 4, (void **)&m->ptok)))
         return rc;
     if (m->hybrid) {
@@ -1291,60 +1318,47 @@ static int ensure_prefill(lrs_model *m) {
 }
 
 // one block of nb tokens at positions pos0.. through every layer (the
-// forward of model.rs:99-266 with the matmuls as GEMMs, operands split into
-// bf16 hi + lo); leaves the residual rows in pX
+// forward of model.rs:99-266 with the matmuls as GEMMs of precision 3); leaves the residual rows in pX
 static int prefill_block(lrs_model *m, const uint32_t *tokens, uint32_t nb, uint32_t pos0) {
     const lrs_config &c = m->cfg;
     hipStream_t s = m->ctx->stream;
     const uint32_t qd = c.n_head * c.head_dim, kvd = c.n_head_kv * c.head_dim, E = c.n_embd;
     constexpr int P = 3;
-    // GEMM inputs as bf16 hi / lo planes: hi at pA16, lo right after the
-    // rows x cols hi plane
-    __bf16 *const hi = m->pA16;
-    auto lo = [&](uint32_t rows, uint32_t cols) { return hi + (size_t)rows * cols; };
-    auto split = [&](const float *a, size_t n) { return launch_split_bf16(a, n, hi, hi + n, s); };
-    // y (+)= A W^T over the block, split over K across workgroups when the
-    // weight has too few output tiles to fill the GPU (the slices' partials
-    // must fit the work buffer)
-    auto gemm = [&](const lrs_weight *w, uint32_t K, float *y, uint32_t N, bool accum = false) {
-        float *work = gemm_work_bytes(nb, N, K, P) <= m->work_bytes ? m->pWork : nullptr;
-        return launch_gemm(w->v, hi, lo(nb, K), y, nb, N, P, s, accum, work);
+    uint8_t *const A = m->pA;  // the current GEMM input
+    auto pack = [&](const float *a, uint32_t cols) { return launch_gemm_pack(a, nb, cols, P, A, s); };
+    // y (+)= A W^T over the block
+    auto gemm = [&](const lrs_weight *w, float *y, bool accum = false, uint32_t *ks = nullptr) {
+        const uint32_t N = w->v.n_out;
+        return launch_gemm_segs(&w->v, &y, &N, 1, A, nb, P, s, accum, m->pWork, m->work_bytes, ks);
     };
     // weights over the same normalised rows (q / k / v, gate / up, or the
     // delta net's in-projections): one launch over all their output tiles
-    // when that alone keeps most CUs busy for the whole K (fewer partly
-    // filled rounds of workgroups than one launch each), else one launch
-    // each (split over K)
+    // (fewer partly filled rounds of workgroups than one launch each) where
+    // the types allow it
     auto gemm_group = [&](uint32_t n, const lrs_weight *const *w, float *const *y,
                           const uint32_t *N) -> hipError_t {
         WeightView wv[3];
-        uint32_t tiles = 0;
+        for (uint32_t i = 0; i < n; i++) wv[i] = w[i]->v;
+        if (gemm_segs_supported(wv, n))
+            return launch_gemm_segs(wv, y, N, n, A, nb, P, s, false, m->pWork, m->work_bytes);
         for (uint32_t i = 0; i < n; i++) {
-            wv[i] = w[i]->v;
-            tiles += gemm_out_tiles(nb, N[i], P);
-        }
-        if (tiles >= 192 && gemm_segs_supported(wv, n))
-            return launch_gemm_segs(wv, y, N, n, hi, lo(nb, E), nb, P, s);
-        for (uint32_t i = 0; i < n; i++) {
-            const hipError_t e = gemm(w[i], E, y[i], N[i]);
+            const hipError_t e = gemm(w[i], y[i]);
             if (e != hipSuccess) return e;
         }
         return hipSuccess;
     };
     // pX += A W^T (o, down, the delta net's out-projection), then the
-    // RMSNorm rows of pX times nw as GEMM planes (and in f32 into xn): when
-    // the GEMM splits over K, its slices' reduce and the norm run as one
-    // kernel
-    auto gemm_resid_norm = [&](const lrs_weight *w, uint32_t K, const float *nw,
-                               float *xn) -> hipError_t {
-        float *work = gemm_work_bytes(nb, E, K, P) <= m->work_bytes ? m->pWork : nullptr;
+    // RMSNorm rows of pX times nw as the next GEMM input (and in f32 into
+    // xn): when the GEMM splits over K, its slices' reduce and the norm run
+    // as one kernel
+    auto gemm_resid_norm = [&](const lrs_weight *w, const float *nw, float *xn) -> hipError_t {
         uint32_t ks = 1;
-        const hipError_t e = launch_gemm(w->v, hi, lo(nb, K), m->pX, nb, E, P, s, true, work, &ks);
+        const hipError_t e = gemm(w, m->pX, true, &ks);
         if (e != hipSuccess) return e;
-        return ks > 1 ? launch_reduce_norm_rows(m->pWork, ks, m->pX, nw, c.rms_eps, E, nb, xn, hi, s)
-                      : launch_rmsnorm_rows(m->pX, nw, c.rms_eps, E, nb, xn, s, hi);
+        return ks > 1 ? launch_reduce_norm_rows(m->pWork, ks, m->pX, nw, c.rms_eps, E, nb, xn, A, s)
+                      : launch_rmsnorm_rows(m->pX, nw, c.rms_eps, E, nb, xn, A, s);
     };
-    // the normalised rows as GEMM planes, and in f32 for a delta-net block,
+    // the normalised rows as a GEMM input, and in f32 for a delta-net block,
     // which reads them for its gates
     auto xn_for = [&](const DevLayer &L) { return m->hybrid && L.dn ? m->pXN : nullptr; };
     // the previous layer's down GEMM already normalised the rows for this one
@@ -1360,18 +1374,18 @@ static int prefill_block(lrs_model *m, const uint32_t *tokens, uint32_t nb, uint
             const hipError_t e = gemm_group(2, w, y, N);
             if (e != hipSuccess) return e;
         }
-        const hipError_t e = launch_swiglu_split(m->pG, m->pU, (size_t)nb * c.n_ff, hi, s);
+        const hipError_t e = launch_swiglu_pack(m->pG, m->pU, c.n_ff, nb, A, s);
         if (e != hipSuccess) return e;
-        if (l + 1 == c.n_layer) return gemm(L.down, c.n_ff, m->pX, E, true);
+        if (l + 1 == c.n_layer) return gemm(L.down, m->pX, true);
         const DevLayer &N = m->layers[l + 1];
         normed = true;
-        return gemm_resid_norm(L.down, c.n_ff, N.attn_norm, xn_for(N));
+        return gemm_resid_norm(L.down, N.attn_norm, xn_for(N));
     };
     LRS_HIP(hipMemcpyAsync(m->ptok, tokens, nb * sizeof(uint32_t), hipMemcpyHostToDevice, s));
     LRS_HIP(launch_dequant_rows(m->embd->v, m->ptok, nb, m->pX, s));
     for (uint32_t l = 0; l < c.n_layer; l++) {
         const DevLayer &L = m->layers[l];
-        if (!normed) LRS_HIP(launch_rmsnorm_rows(m->pX, L.attn_norm, c.rms_eps, E, nb, xn_for(L), s, hi));
+        if (!normed) LRS_HIP(launch_rmsnorm_rows(m->pX, L.attn_norm, c.rms_eps, E, nb, xn_for(L), A, s));
         normed = false;
         if (m->hybrid) {
             if (L.dn) {
@@ -1410,8 +1424,8 @@ static int prefill_block(lrs_model *m, const uint32_t *tokens, uint32_t nb, uint
                 da.pos0 = pos0;
                 da.eps = c.rms_eps;
                 LRS_HIP(launch_dn_prefill(da, s));
-                LRS_HIP(split(m->pY, (size_t)nb * VD));
-                LRS_HIP(gemm_resid_norm(L.ssm_out, VD, L.ffn_norm, nullptr));
+                LRS_HIP(pack(m->pY, VD));
+                LRS_HIP(gemm_resid_norm(L.ssm_out, L.ffn_norm, nullptr));
             } else {
                 // gated attention: Q (+ gate), k, v; QK-norm + RoPE; causal
                 // attention over the cache; sigmoid gate; o
@@ -1427,8 +1441,8 @@ static int prefill_block(lrs_model *m, const uint32_t *tokens, uint32_t nb, uint
                 LRS_HIP(launch_attn_prefill(m->pQ, L.kc, L.vc, m->pATT, nb, pos0, c.n_head, c.n_head_kv,
                                             c.head_dim, c.ctx, s));
                 LRS_HIP(launch_gate_rows(m->pATT, m->pQG, nb, qd, c.head_dim, s));
-                LRS_HIP(split(m->pATT, (size_t)nb * qd));
-                LRS_HIP(gemm_resid_norm(L.o, qd, L.ffn_norm, nullptr));
+                LRS_HIP(pack(m->pATT, qd));
+                LRS_HIP(gemm_resid_norm(L.o, L.ffn_norm, nullptr));
             }
             LRS_HIP(ffn(l));
             continue;
@@ -1443,8 +1457,8 @@ static int prefill_block(lrs_model *m, const uint32_t *tokens, uint32_t nb, uint
                                 L.vc, nb, pos0, qd, kvd, c.head_dim, c.rope_dim, c.ctx, s));
         LRS_HIP(launch_attn_prefill(m->pQ, L.kc, L.vc, m->pATT, nb, pos0, c.n_head, c.n_head_kv,
                                     c.head_dim, c.ctx, s));
-        LRS_HIP(split(m->pATT, (size_t)nb * qd));
-        LRS_HIP(gemm_resid_norm(L.o, qd, L.ffn_norm, nullptr));
+        LRS_HIP(pack(m->pATT, qd));
+        LRS_HIP(gemm_resid_norm(L.o, L.ffn_norm, nullptr));
         LRS_HIP(ffn(l));
     }
     return LRS_OK;

@@ -1,33 +1,45 @@
 // prefill.hip — the per-token ops of a batched prompt block (n tokens at
 // positions pos0 .. pos0+n-1) around the matrix-core GEMMs of gemm.hip:
-// RMSNorm per row and SwiGLU (both written straight to the bf16 input
-// planes of the next GEMM), bias + RoPE + f16 KV append after the q/k/v
+// RMSNorm per row and SwiGLU (both written straight as the next GEMM's input,
+// gemm_pack.h), bias + RoPE + f16 KV append after the q/k/v
 // GEMMs, causal GQA attention over the cache.  The formulas of the decode
 // kernels (Model::forward, crates/llama-model/src/model.rs:99-266; ops.rs:
 // 56-66, 952-988; attention.rs:76-166), which is what the reference's
 // prefill_residente (gpu.rs:673-697) drives in blocks of batch_size() tokens;
 // the attention runs on the matrix cores (f16 hi/lo operands, f32
 // accumulation), so its summation order differs from the per-token kernel.
-#include "lrs_internal.h"
+#include "gemm_pack.h"
 
 namespace lrs {
 
-// bf16 hi of v and the bf16 of the remainder (the GEMM input planes)
-__device__ __forceinline__ void split_store(float v, __bf16 *hi, __bf16 *lo) {
-    const __bf16 h = (__bf16)v;
-    *hi = h;
-    *lo = (__bf16)(v - (float)h);
+// (x * scale) * w of eight elements from element i, as a GEMM input and (Y) in f32
+__device__ __forceinline__ void norm_store8(const float *__restrict__ x, const float *__restrict__ w, float scale,
+                                            uint32_t i, uint32_t row, uint32_t E, float *__restrict__ Y,
+                                            uint8_t *__restrict__ planes) {
+    float v[8];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const float4 a = *reinterpret_cast<const float4 *>(x + i + 4 * h);
+        const float4 g = *reinterpret_cast<const float4 *>(w + i + 4 * h);
+        v[4 * h] = (a.x * scale) * g.x;
+        v[4 * h + 1] = (a.y * scale) * g.y;
+        v[4 * h + 2] = (a.z * scale) * g.z;
+        v[4 * h + 3] = (a.w * scale) * g.w;
+        if (Y)
+            *reinterpret_cast<float4 *>(Y + (size_t)row * E + i + 4 * h) =
+                make_float4(v[4 * h], v[4 * h + 1], v[4 * h + 2], v[4 * h + 3]);
+    }
+    gp_store8<3>(v, row, i >> 3, E >> 8, planes);
 }
 
-// Y[r] = (X[r] * scale_r) * w, scale_r = 1 / sqrt(mean(X[r]^2) + eps); with
-// hi, the same values also as bf16 hi / lo planes (lo = hi + gridDim.x * E)
+// the row X[r] * scale_r * w, scale_r = 1 / sqrt(mean(X[r]^2) + eps), as a
+// GEMM input (gemm_pack.h) and, with Y, in f32
 __global__ __launch_bounds__(256) void k_rmsnorm_rows(const float *__restrict__ X,
                                                       const float *__restrict__ w, float eps,
                                                       uint32_t E, float *__restrict__ Y,
-                                                      __bf16 *__restrict__ hi) {
+                                                      uint8_t *__restrict__ planes) {
     __shared__ float red[4];
     const float *x = X + (size_t)blockIdx.x * E;
-    float *y = Y ? Y + (size_t)blockIdx.x * E : nullptr;
     float ss = 0.f;
     for (uint32_t i = 4 * threadIdx.x; i < E; i += 4 * blockDim.x) {
         const float4 v = *reinterpret_cast<const float4 *>(x + i);
@@ -39,12 +51,8 @@ __global__ __launch_bounds__(256) void k_rmsnorm_rows(const float *__restrict__ 
     __syncthreads();
     const float tot = (red[0] + red[1]) + (red[2] + red[3]);
     const float scale = 1.0f / sqrtf(tot / (float)E + eps);
-    const size_t plane = (size_t)gridDim.x * E, r0 = (size_t)blockIdx.x * E;
-    for (uint32_t i = threadIdx.x; i < E; i += blockDim.x) {
-        const float v = (x[i] * scale) * w[i];
-        if (Y) y[i] = v;
-        if (hi) split_store(v, hi + r0 + i, hi + plane + r0 + i);
-    }
+    for (uint32_t i = 8 * threadIdx.x; i < E; i += 8 * blockDim.x)
+        norm_store8(x, w, scale, i, blockIdx.x, E, Y, planes);
 }
 
 // X += the ks K-slice partials part[z][row][E] (summed in slice order, then
@@ -55,7 +63,7 @@ __global__ __launch_bounds__(256) void k_reduce_norm_rows(const float *__restric
                                                           uint32_t ks, float *__restrict__ X,
                                                           const float *__restrict__ w, float eps,
                                                           uint32_t E, float *__restrict__ Y,
-                                                          __bf16 *__restrict__ hi) {
+                                                          uint8_t *__restrict__ planes) {
     __shared__ float red[4];
     const size_t plane = (size_t)gridDim.x * E, r0 = (size_t)blockIdx.x * E;
     float *x = X + r0;
@@ -83,20 +91,9 @@ __global__ __launch_bounds__(256) void k_reduce_norm_rows(const float *__restric
     __syncthreads();
     const float tot = (red[0] + red[1]) + (red[2] + red[3]);
     const float scale = 1.0f / sqrtf(tot / (float)E + eps);
-    // each thread reads back the elements it stored above
-    for (uint32_t i = 4 * threadIdx.x; i < E; i += 4 * blockDim.x) {
-        const float4 v = *reinterpret_cast<const float4 *>(x + i);
-        const float4 g = *reinterpret_cast<const float4 *>(w + i);
-        const float4 o = {(v.x * scale) * g.x, (v.y * scale) * g.y, (v.z * scale) * g.z,
-                          (v.w * scale) * g.w};
-        if (Y) *reinterpret_cast<float4 *>(Y + r0 + i) = o;
-        if (hi) {
-            split_store(o.x, hi + r0 + i, hi + plane + r0 + i);
-            split_store(o.y, hi + r0 + i + 1, hi + plane + r0 + i + 1);
-            split_store(o.z, hi + r0 + i + 2, hi + plane + r0 + i + 2);
-            split_store(o.w, hi + r0 + i + 3, hi + plane + r0 + i + 3);
-        }
-    }
+    __syncthreads();  // the row's stores above are read back by other threads
+    for (uint32_t i = 8 * threadIdx.x; i < E; i += 8 * blockDim.x)
+        norm_store8(x, w, scale, i, blockIdx.x, E, Y, planes);
 }
 
 // q/k/v GEMM outputs -> bias, adjacent-pair RoPE on q and k at position
@@ -410,17 +407,17 @@ __global__ __launch_bounds__(64 * NW) void k_attn_pf_mma(AttnPre a) {
 }
 
 hipError_t launch_rmsnorm_rows(const float *X, const float *w, float eps, uint32_t E, uint32_t n,
-                               float *Y, hipStream_t s, __bf16 *hi) {
-    if (E % 4 || (!Y && !hi)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_rmsnorm_rows, dim3(n), dim3(256), 0, s, X, w, eps, E, Y, hi);
+                               float *Y, uint8_t *planes, hipStream_t s) {
+    if (E % 256 || !planes) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_rmsnorm_rows, dim3(n), dim3(256), 0, s, X, w, eps, E, Y, planes);
     return hipGetLastError();
 }
 
 hipError_t launch_reduce_norm_rows(const float *part, uint32_t ks, float *X, const float *w,
-                                   float eps, uint32_t E, uint32_t n, float *Y, __bf16 *hi,
+                                   float eps, uint32_t E, uint32_t n, float *Y, uint8_t *planes,
                                    hipStream_t s) {
-    if (E % 4 || ks == 0 || (!Y && !hi)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_reduce_norm_rows, dim3(n), dim3(256), 0, s, part, ks, X, w, eps, E, Y, hi);
+    if (E % 256 || ks == 0 || !planes) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_reduce_norm_rows, dim3(n), dim3(256), 0, s, part, ks, X, w, eps, E, Y, planes);
     return hipGetLastError();
 }
 
@@ -469,35 +466,35 @@ hipError_t launch_attn_prefill(const float *q, const _Float16 *kc, const _Float1
     return hipGetLastError();
 }
 
-// silu(G) * U (ops.rs:978-988: g / (1 + e^-g) * u), stored as the bf16 hi / lo
-// planes of the down projection's input
-__global__ __launch_bounds__(256) void k_swiglu_split(const float *__restrict__ G,
-                                                      const float *__restrict__ U, size_t n4,
-                                                      __bf16 *__restrict__ hi,
-                                                      __bf16 *__restrict__ lo) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n4) return;
-    const float4 g = reinterpret_cast<const float4 *>(G)[i];
-    const float4 u = reinterpret_cast<const float4 *>(U)[i];
-    const float y[4] = {(g.x / (1.0f + expf(-g.x))) * u.x, (g.y / (1.0f + expf(-g.y))) * u.y,
-                        (g.z / (1.0f + expf(-g.z))) * u.z, (g.w / (1.0f + expf(-g.w))) * u.w};
-    typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
-    bf16x4 h, l;
+// silu(G) * U (ops.rs:978-988: g / (1 + e^-g) * u) as the down projection's
+// GEMM input; workgroup = 32 rows x one super-block
+__global__ __launch_bounds__(256) void k_swiglu_pack(const float *__restrict__ G,
+                                                     const float *__restrict__ U, uint32_t F, uint32_t n,
+                                                     uint8_t *__restrict__ planes) {
 #pragma unroll
     for (int k = 0; k < 4; k++) {
-        h[k] = (__bf16)y[k];
-        l[k] = (__bf16)(y[k] - (float)h[k]);
+        const uint32_t row = 32 * blockIdx.y + 8 * k + (threadIdx.x >> 5);
+        if (row >= n) return;
+        const uint32_t c = 32 * blockIdx.x + (threadIdx.x & 31);
+        const size_t i = (size_t)row * F + 8 * c;
+        float v[8];
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const float4 g = *reinterpret_cast<const float4 *>(G + i + 4 * h);
+            const float4 u = *reinterpret_cast<const float4 *>(U + i + 4 * h);
+            v[4 * h] = (g.x / (1.0f + expf(-g.x))) * u.x;
+            v[4 * h + 1] = (g.y / (1.0f + expf(-g.y))) * u.y;
+            v[4 * h + 2] = (g.z / (1.0f + expf(-g.z))) * u.z;
+            v[4 * h + 3] = (g.w / (1.0f + expf(-g.w))) * u.w;
+        }
+        gp_store8<3>(v, row, c, F >> 8, planes);
     }
-    reinterpret_cast<bf16x4 *>(hi)[i] = h;
-    reinterpret_cast<bf16x4 *>(lo)[i] = l;
 }
 
-hipError_t launch_swiglu_split(const float *G, const float *U, size_t n, __bf16 *hi,
-                               hipStream_t s) {
-    if (n % 4) return hipErrorInvalidValue;
-    const size_t n4 = n / 4;
-    hipLaunchKernelGGL(k_swiglu_split, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, G, U,
-                       n4, hi, hi + n);
+hipError_t launch_swiglu_pack(const float *G, const float *U, uint32_t F, uint32_t n, uint8_t *planes,
+                              hipStream_t s) {
+    if (F % 256 || n == 0) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_swiglu_pack, dim3(F / 256, (n + 31) / 32), dim3(256), 0, s, G, U, F, n, planes);
     return hipGetLastError();
 }
 

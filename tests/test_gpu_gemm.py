@@ -140,6 +140,37 @@ def quantizer_like(t, n, k, seed):
     return b.reshape(-1)
 
 
+@pytest.mark.parametrize("t", [Q4_K, Q5_K, Q6_K, Q8_0])
+# row tiles of 32 tokens (1, 2 or 4 of them a workgroup) and 256 weight rows,
+# K in whole super-blocks (1: nothing to prefetch; 3: an uneven K split): the
+# sizes at, below and past each edge
+@pytest.mark.parametrize("m,n,k", [(1, 1, 256), (2, 255, 256), (32, 257, 768), (33, 16, 512),
+                                   (64, 272, 1280), (65, 513, 256), (129, 31, 2816)])
+def test_gemm_edges_and_extreme_blocks(lrs, orc, ctx, t, m, n, k):
+    """Tile edges, quantizer-like blocks, and activations whose super-blocks
+    differ by 2^100, are all zero, or hold one outlier of 2^12."""
+    w = quantizer_like(t, n, k, m + n)
+    deq = orc.dequant(t, w).reshape(n, k).astype(np.float64)
+    rng = np.random.default_rng(n)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    a[:, 5] *= 4096.0
+    a[m // 2] *= np.float32(2.0 ** 50)
+    a[m // 3] *= np.float32(2.0 ** -50)
+    a[m - 1, :256] = 0.0
+    W = lrs.Weight.upload(ctx, t, w, k, n)
+    y3, y1 = W.gemm(a, precision=3), W.gemm(a, precision=1)
+    ref3 = a.astype(np.float64) @ deq.T
+    ref1 = bf16(a).astype(np.float64) @ bf16(deq.astype(np.float32)).astype(np.float64).T
+    for r in range(m):
+        # the sum's f32 rounding is relative to its terms, which cancel: the
+        # bounds are the 22-bit activations' and f32 sums' against their size
+        size = np.linalg.norm(np.abs(a[r].astype(np.float64)) @ np.abs(deq).T)
+        assert np.linalg.norm(y3[r] - ref3[r]) <= 2e-6 * size
+        # bf16 of a fused a * q - b may round the other way at a tie: 2^-9 of
+        # a few weights
+        assert np.linalg.norm(y1[r] - ref1[r]) <= 1e-5 * size
+
+
 @pytest.mark.parametrize("t", [Q8_0, Q4_K, Q5_K, Q6_K])
 @pytest.mark.parametrize("n,k,shift", [(1, 256, 0), (17, 768, 0), (5, 512, 1)])
 def test_dequant_into_any_float_address_is_exact(lrs, orc, ctx, t, n, k, shift):
