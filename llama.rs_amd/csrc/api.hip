@@ -424,7 +424,9 @@ int lrs_matvec_f32(lrs_ctx *ctx, const lrs_weight *w, const float *x, float *y, 
 static int gemm_run(lrs_ctx *ctx, const WeightView *wv, float *const *y, const uint32_t *ldy, uint32_t n_w,
                     const float *a_dev, uint32_t m, int precision) {
     const size_t ab = gemm_planes_bytes(m, wv[0].n_in, precision);
-    const size_t wb = gemm_work_bytes(m, ldy, n_w, wv[0].n_in, wv[0].type, precision);
+    uint32_t types[3];
+    for (uint32_t i = 0; i < n_w; i++) types[i] = wv[i].type;
+    const size_t wb = gemm_work_bytes(m, ldy, types, n_w, wv[0].n_in, precision);
     void *buf = nullptr;
     if (int rc_ = ctx_scratch(ctx, ab + wb, &buf)) return rc_;
     LRS_HIP(launch_gemm_pack(a_dev, m, wv[0].n_in, precision, (uint8_t *)buf, ctx->stream));

@@ -601,7 +601,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     const uint32_t ntile = g.nm * g.nn * g.ks, per = (ntile + 7) / 8;
     const uint32_t t0 = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
     if ((blockIdx.x >> 3) >= per || t0 >= ntile) return;
-    const uint32_t mb = t0 % g.nm, t = t0 / g.nm, nt = t % g.nn, kz = t / g.nn;
+    // row tiles of one weight tile run next to each other (they share its bytes
+    // in an XCD's L2); the last segment, of the slower type, starts first
+    const uint32_t mb = t0 % g.nm, t = t0 / g.nm, nt = g.nn - 1 - t % g.nn, kz = t / g.nn;
     uint32_t si = 0;
 #pragma unroll
     for (int i = 1; i < PG_MAX_SEG; i++)
@@ -676,36 +678,47 @@ static uint32_t pg_tiles(uint32_t M, const uint32_t *N, uint32_t nseg, uint32_t 
 }
 
 // us per super-block of n workgroups that share a CU, measured with Q4_K
-// weights at K = 5120: the first workgroups of a CU hide each other's waits
-static double pg_unit(int prec, uint32_t mt, uint32_t n) {
-    static const double p3m1[3] = {2.4, 3.3, 6.2}, p3m2[2] = {3.6, 6.4};
+// weights at K = 5120: the first workgroups of a CU hide each other's waits.
+// `fit`: workgroups that fit a CU at once (by registers)
+static double pg_unit(int prec, uint32_t mt, uint32_t fit, uint32_t n) {
+    static const double p3m1[3] = {2.5, 4.4, 6.6}, p3m2[2] = {3.6, 6.4};
     static const double p1m1[3] = {2.0, 3.0, 4.2}, p1m2[3] = {2.7, 4.8, 6.4}, p1m4[2] = {4.4, 7.8};
     const double *c = prec == 3 ? (mt == 1 ? p3m1 : p3m2) : mt == 1 ? p1m1 : mt == 2 ? p1m2 : p1m4;
-    const uint32_t full = mt == (prec == 3 ? 2u : 4u) ? 2 : 3;
-    return n / full * c[full - 1] + (n % full ? c[n % full - 1] : 0.0);
+    return n / fit * c[fit - 1] + (n % fit ? c[n % fit - 1] : 0.0);
 }
 
 // The shape with the least expected time: the workgroups that a CU gets, and
-// for K slices the partial sums written and read back (at about 8 TB/s, most
+// for K slices the partial sums written and read back (at about 7 TB/s, most
 // of them in the memory-side cache) and the launch that adds them.
 // have_work: K slices may be used
-static PgPlan pg_plan(uint32_t M, const uint32_t *N, uint32_t nseg, uint32_t nsb, uint32_t type, int prec,
+static PgPlan pg_plan(uint32_t M, const uint32_t *N, const uint32_t *type, uint32_t nseg, uint32_t nsb, int prec,
                       bool have_work) {
-    // precision 3: Q6_K and Q8_0 take a third product, Q5_K more unpacking
-    const double rel = prec == 1 || type == T_Q4_K ? 1.0 : type == T_Q5_K ? 1.2 : 1.5;
+    // precision 3: Q6_K and Q8_0 take a third product, Q5_K more unpacking.
+    // While every workgroup runs at once the slowest counts, else the average
     uint32_t ntot = 0;
-    for (uint32_t i = 0; i < nseg; i++) ntot += N[i];
+    double slow = 1.0, mean = 0.0;
+    bool wide = false;  // a type whose operands take more registers
+    for (uint32_t i = 0; i < nseg; i++) {
+        const double rel = prec == 1 || type[i] == T_Q4_K ? 1.0 : type[i] == T_Q5_K ? 1.2 : 1.5;
+        slow = std::max(slow, rel);
+        mean += rel * N[i];
+        ntot += N[i];
+        wide = wide || type[i] == T_Q6_K || type[i] == T_Q5_K;
+    }
+    mean /= ntot;
     PgPlan best = {1, 1};
     double best_cost = 1e30;
     for (uint32_t mt = 1; mt <= (prec == 3 ? 2u : 4u); mt *= 2) {
         if (mt > 1 && M <= 16 * mt) break;
         const uint32_t tiles = pg_tiles(M, N, nseg, mt);
+        const uint32_t fit = mt == (prec == 3 ? 2u : 4u) || (wide && !(prec == 1 && mt == 1)) ? 2 : 3;
         for (uint32_t ks = 1; ks <= nsb && ks <= 32; ks++) {
             if (ks > 1 && (!have_work || tiles >= 2048)) break;
-            const uint32_t len = (nsb + ks - 1) / ks;
-            double cost = (len + 0.5) * rel * pg_unit(prec, mt, (tiles * ks + 255) / 256);
-            if (ks > 1) cost += 4.0 + (2.0 * ks + 1) * M * ntot * 4.0 / 8e6;
-            if (cost < best_cost * 0.999) {
+            const uint32_t len = (nsb + ks - 1) / ks, per = (tiles * ks + 255) / 256;
+            const double rel = per < fit ? slow : per == fit ? 0.5 * (slow + mean) : mean;
+            double cost = (len + 0.5) * rel * pg_unit(prec, mt, fit, per);
+            if (ks > 1) cost += 5.0 + (2.0 * ks + 1) * M * ntot * 4.0 / 7e6;
+            if (cost < best_cost * 0.98) {
                 best_cost = cost;
                 best = {mt, ks};
             }
@@ -717,12 +730,12 @@ static PgPlan pg_plan(uint32_t M, const uint32_t *N, uint32_t nseg, uint32_t nsb
 // scratch of the K-sliced form for any row count up to M (a smaller one may
 // split over more slices): a caller that made its largest call first never
 // needs more
-size_t gemm_work_bytes(uint32_t M, const uint32_t *N, uint32_t nseg, uint32_t K, uint32_t type, int prec) {
+size_t gemm_work_bytes(uint32_t M, const uint32_t *N, const uint32_t *type, uint32_t nseg, uint32_t K, int prec) {
     uint32_t ntot = 0;
     for (uint32_t i = 0; i < nseg; i++) ntot += N[i];
     size_t most = 0;
     for (uint32_t m = M;; m = (m - 1) / 32 * 32) {
-        const uint32_t ks = pg_plan(m, N, nseg, K / 256, type, prec, true).ks;
+        const uint32_t ks = pg_plan(m, N, type, nseg, K / 256, prec, true).ks;
         if (ks > 1) most = std::max(most, (size_t)ks * m * ntot * sizeof(float));
         if (m <= 32) break;
     }
@@ -765,9 +778,9 @@ hipError_t launch_gemm_segs(const WeightView *w, float *const *y, const uint32_t
                             size_t work_bytes, uint32_t *ks_out) {
     if (M == 0 || !planes || !gemm_segs_supported(w, nseg) || w[0].n_in == 0 || w[0].n_in % 256)
         return hipErrorInvalidValue;
-    uint32_t Ns[PG_MAX_SEG];
-    for (uint32_t i = 0; i < nseg; i++) Ns[i] = w[i].n_out;
-    PgPlan p = pg_plan(M, Ns, nseg, w[0].n_in / 256, w[0].type, prec, work != nullptr);
+    uint32_t Ns[PG_MAX_SEG], ts[PG_MAX_SEG];
+    for (uint32_t i = 0; i < nseg; i++) Ns[i] = w[i].n_out, ts[i] = w[i].type;
+    PgPlan p = pg_plan(M, Ns, ts, nseg, w[0].n_in / 256, prec, work != nullptr);
     PgArgs g = {};
     g.a = planes;
     g.nseg = nseg;
@@ -787,7 +800,7 @@ hipError_t launch_gemm_segs(const WeightView *w, float *const *y, const uint32_t
     g.nsb = w[0].n_in / 256;
     g.accum = accum ? 1u : 0u;
     if (p.ks > 1 && (size_t)p.ks * M * ntot * sizeof(float) > work_bytes)
-        p = pg_plan(M, Ns, nseg, g.nsb, w[0].type, prec, false);
+        p = pg_plan(M, Ns, ts, nseg, g.nsb, prec, false);
     g.nm = (M + 32 * p.mt - 1) / (32 * p.mt);
     g.nn = nt;
     g.ntot = ntot;

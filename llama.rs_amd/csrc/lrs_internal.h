@@ -150,7 +150,7 @@ size_t gemm_planes_bytes(uint32_t M, uint32_t K, int prec);
 // ks_out: when given, a K split leaves its ks_out slices of [M][sum of N]
 // partials in work for the caller to reduce (ks_out 1: y written directly)
 bool gemm_segs_supported(const WeightView *w, uint32_t nseg);
-size_t gemm_work_bytes(uint32_t M, const uint32_t *N, uint32_t nseg, uint32_t K, uint32_t type, int prec);
+size_t gemm_work_bytes(uint32_t M, const uint32_t *N, const uint32_t *type, uint32_t nseg, uint32_t K, int prec);
 hipError_t launch_gemm_segs(const WeightView *w, float *const *y, const uint32_t *ldy, uint32_t nseg,
                             const uint8_t *planes, uint32_t M, int prec, hipStream_t s, bool accum = false,
                             float *work = nullptr, size_t work_bytes = 0, uint32_t *ks_out = nullptr);

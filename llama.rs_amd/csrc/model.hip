@@ -1253,13 +1253,14 @@ static bool prefill_capable(const lrs_model *m) {
 static size_t prefill_work_bytes(const lrs_model *m) {
     size_t most = 0;
     auto need = [&](std::initializer_list<const lrs_weight *> ws) {
-        uint32_t N[3], n = 0;
+        uint32_t N[3], t[3], n = 0;
         for (const lrs_weight *w : ws) {
-            const uint32_t one = w->v.n_out;
-            most = std::max(most, gemm_work_bytes(PREFILL_BLOCK, &one, 1, w->v.n_in, w->v.type, 3));
-            N[n++] = one;
+            N[n] = w->v.n_out;
+            t[n] = w->v.type;
+            most = std::max(most, gemm_work_bytes(PREFILL_BLOCK, N + n, t + n, 1, w->v.n_in, 3));
+            n++;
         }
-        most = std::max(most, gemm_work_bytes(PREFILL_BLOCK, N, n, (*ws.begin())->v.n_in, (*ws.begin())->v.type, 3));
+        most = std::max(most, gemm_work_bytes(PREFILL_BLOCK, N, t, n, (*ws.begin())->v.n_in, 3));
     };
     for (const DevLayer &L : m->layers) {
         need({L.gate, L.up});
@@ -1350,10 +1351,12 @@ static int prefill_block(lrs_model *m, const uint32_t *tokens, uint32_t nb, uint
     // pX += A W^T (o, down, the delta net's out-projection), then the
     // RMSNorm rows of pX times nw as the next GEMM input (and in f32 into
     // xn): when the GEMM splits over K, its slices' reduce and the norm run
-    // as one kernel
+    // as one kernel of a workgroup per row.  Few rows are too few workgroups
+    // for the many slices they have (19 rows of 22 slices: 29 us, against
+    // 5 + 4 us as a reduce over all outputs and a norm)
     auto gemm_resid_norm = [&](const lrs_weight *w, const float *nw, float *xn) -> hipError_t {
         uint32_t ks = 1;
-        const hipError_t e = gemm(w, m->pX, true, &ks);
+        const hipError_t e = gemm(w, m->pX, true, nb >= 192 ? &ks : nullptr);
         if (e != hipSuccess) return e;
         return ks > 1 ? launch_reduce_norm_rows(m->pWork, ks, m->pX, nw, c.rms_eps, E, nb, xn, A, s)
                       : launch_rmsnorm_rows(m->pX, nw, c.rms_eps, E, nb, xn, A, s);
