@@ -575,17 +575,6 @@ __global__ __launch_bounds__(HD) void k_qk_prep_rows(const float *__restrict__ q
     }
 }
 
-// att *= sigmoid(gate), gate = second half of each head's Q rows (gate_quant.comp)
-__global__ __launch_bounds__(256) void k_gate_rows(float *__restrict__ att, const float *__restrict__ qg,
-                                                   uint32_t qd, uint32_t hd, size_t n) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const size_t t = i / qd;
-    const uint32_t e = (uint32_t)(i % qd), h = e / hd, dd = e % hd;
-    const float g = qg[t * 2 * qd + (size_t)h * 2 * hd + hd + dd];
-    att[i] = att[i] * (1.0f / (1.0f + expf(-g)));
-}
-
 hipError_t launch_dn_prefill(const DnBlockArgs &a, hipStream_t s) {
     const uint32_t D = a.d_state, KD = a.k_heads * D, VD = a.v_heads * D, CD = 2 * KD + VD;
     if (a.nb == 0 || a.n_embd % 4 || a.d_conv == 0 || a.d_conv > 8 || (D != 64 && D != 128))
@@ -629,13 +618,6 @@ hipError_t launch_qk_prep_rows(const float *qg, const float *kb, const float *vb
         break;
     default: return hipErrorInvalidValue;
     }
-    return hipGetLastError();
-}
-
-hipError_t launch_gate_rows(float *att, const float *qg, uint32_t nb, uint32_t qd, uint32_t hd,
-                            hipStream_t s) {
-    const size_t n = (size_t)nb * qd;
-    hipLaunchKernelGGL(k_gate_rows, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, att, qg, qd, hd, n);
     return hipGetLastError();
 }
 

@@ -170,9 +170,14 @@ hipError_t launch_qkv_post(const float *qt, const float *kt, const float *vt, co
                            _Float16 *kc, _Float16 *vc, uint32_t n, uint32_t pos0, uint32_t qd,
                            uint32_t kvd, uint32_t hd, uint32_t rope_dim, uint32_t ctx,
                            hipStream_t s);
-hipError_t launch_attn_prefill(const float *q, const _Float16 *kc, const _Float16 *vc, float *out,
-                               uint32_t n, uint32_t pos0, uint32_t n_head, uint32_t n_kv,
-                               uint32_t hd, uint32_t ctx, hipStream_t s);
+// causal attention of the block as the o projection's GEMM input (planes,
+// precision 3), over attn_prefill_splits shares of the cache positions: part
+// [splits][n][n_head * hd], ml [splits][n][n_head] scratch.  qg (may be null):
+// [n][n_head][2 hd] rows whose second halves gate the outputs
+uint32_t attn_prefill_splits(uint32_t n, uint32_t pos0, uint32_t n_head, uint32_t n_kv, uint32_t hd);
+hipError_t launch_attn_prefill(const float *q, const _Float16 *kc, const _Float16 *vc, const float *qg, float *part,
+                               float2 *ml, uint32_t n, uint32_t pos0, uint32_t n_head, uint32_t n_kv,
+                               uint32_t hd, uint32_t ctx, uint8_t *planes, hipStream_t s);
 // silu(G) * U [n][F] as a GEMM input of precision 3; F a multiple of 256
 hipError_t launch_swiglu_pack(const float *G, const float *U, uint32_t F, uint32_t n, uint8_t *planes,
                               hipStream_t s);
@@ -231,8 +236,6 @@ hipError_t launch_qk_prep_rows(const float *qg, const float *kb, const float *vb
                                _Float16 *vc, uint32_t nb, uint32_t pos0, uint32_t n_head,
                                uint32_t n_kv, uint32_t head_dim, uint32_t ctx, uint32_t rope_dim,
                                float eps, hipStream_t s);
-hipError_t launch_gate_rows(float *att, const float *qg, uint32_t nb, uint32_t qd, uint32_t hd,
-                            hipStream_t s);
 hipError_t launch_qk_prep(const float *qg, const float *kb, const float *vb, const float *q_norm,
                           const float *k_norm, const float *freq, const uint32_t *step, float *q,
                           _Float16 *kc, _Float16 *vc, uint32_t n_head, uint32_t n_kv,

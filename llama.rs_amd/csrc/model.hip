@@ -169,10 +169,11 @@ struct lrs_model {
     unsigned long long *amax;
     uint32_t head_keys = 0;
     // batched prompt blocks (allocated at the first block): residual,
-    // normalised rows, q/k/v GEMM outputs, q after RoPE, attention output,
-    // gate / up, token ids
+    // normalised rows, q/k/v GEMM outputs, q after RoPE, the attention's
+    // splits and their {max, sum}, gate / up, token ids
     uint32_t pb_cap = 0;
     float *pX = nullptr, *pXN, *pQt, *pKt, *pVt, *pQ, *pATT, *pG, *pU;
+    float2 *pML = nullptr;
     uint8_t *pA = nullptr;  // the current GEMM input (gemm_pack.h)
     // hybrid blocks: Q + gate rows, conv in / out, output gate, rule output,
     // gated norm, per-(token, head) gates
@@ -1281,6 +1282,11 @@ static int ensure_prefill(lrs_model *m) {
     const lrs_config &c = m->cfg;
     const size_t B = PREFILL_BLOCK, qd = (size_t)c.n_head * c.head_dim,
                  kvd = (size_t)c.n_head_kv * c.head_dim;
+    // rows of all the attention's splits, most over the block sizes
+    size_t att_rows = 0;
+    for (uint32_t n = 1; n <= PREFILL_BLOCK; n++)
+        att_rows = std::max<size_t>(att_rows, (size_t)n * attn_prefill_splits(n, c.ctx - std::min(c.ctx, n), c.n_head,
+                                                                              c.n_head_kv, c.head_dim));
     int rc;
     if ((rc = dev_alloc(m, B * c.n_embd * 4, (void **)&m->pX)) ||
         (rc = dev_alloc(m, B * c.n_embd * 4, (void **)&m->pXN)) ||
@@ -1288,7 +1294,8 @@ static int ensure_prefill(lrs_model *m) {
         (rc = dev_alloc(m, B * kvd * 4, (void **)&m->pKt)) ||
         (rc = dev_alloc(m, B * kvd * 4, (void **)&m->pVt)) ||
         (rc = dev_alloc(m, B * qd * 4, (void **)&m->pQ)) ||
-        (rc = dev_alloc(m, B * qd * 4, (void **)&m->pATT)) ||
+        (rc = dev_alloc(m, att_rows * qd * 4, (void **)&m->pATT)) ||
+        (rc = dev_alloc(m, att_rows * c.n_head * sizeof(float2), (void **)&m->pML)) ||
         (rc = dev_alloc(m, B * c.n_ff * 4, (void **)&m->pG)) ||
         (rc = dev_alloc(m, B * c.n_ff * 4, (void **)&m->pU)) ||
         (rc = dev_alloc(m,
@@ -1441,10 +1448,8 @@ static int prefill_block(lrs_model *m, const uint32_t *tokens, uint32_t nb, uint
                 LRS_HIP(launch_qk_prep_rows(m->pQG, m->pKt, m->pVt, L.q_norm, L.k_norm, m->freq, m->pQ,
                                             L.kc, L.vc, nb, pos0, c.n_head, c.n_head_kv, c.head_dim,
                                             c.ctx, c.rope_dim, c.rms_eps, s));
-                LRS_HIP(launch_attn_prefill(m->pQ, L.kc, L.vc, m->pATT, nb, pos0, c.n_head, c.n_head_kv,
-                                            c.head_dim, c.ctx, s));
-                LRS_HIP(launch_gate_rows(m->pATT, m->pQG, nb, qd, c.head_dim, s));
-                LRS_HIP(pack(m->pATT, qd));
+                LRS_HIP(launch_attn_prefill(m->pQ, L.kc, L.vc, m->pQG, m->pATT, m->pML, nb, pos0, c.n_head,
+                                            c.n_head_kv, c.head_dim, c.ctx, A, s));
                 LRS_HIP(gemm_resid_norm(L.o, L.ffn_norm, nullptr));
             }
             LRS_HIP(ffn(l));
@@ -1458,9 +1463,8 @@ static int prefill_block(lrs_model *m, const uint32_t *tokens, uint32_t nb, uint
         }
         LRS_HIP(launch_qkv_post(m->pQt, m->pKt, m->pVt, L.bq, L.bk, L.bv, m->freq, m->pQ, L.kc,
                                 L.vc, nb, pos0, qd, kvd, c.head_dim, c.rope_dim, c.ctx, s));
-        LRS_HIP(launch_attn_prefill(m->pQ, L.kc, L.vc, m->pATT, nb, pos0, c.n_head, c.n_head_kv,
-                                    c.head_dim, c.ctx, s));
-        LRS_HIP(pack(m->pATT, qd));
+        LRS_HIP(launch_attn_prefill(m->pQ, L.kc, L.vc, nullptr, m->pATT, m->pML, nb, pos0, c.n_head,
+                                    c.n_head_kv, c.head_dim, c.ctx, A, s));
         LRS_HIP(gemm_resid_norm(L.o, L.ffn_norm, nullptr));
         LRS_HIP(ffn(l));
     }

@@ -156,8 +156,9 @@ __global__ void k_qkv_post(QkvPost a) {
 struct AttnPre {
     const float *q;                 // [n][n_head * hd]
     const _Float16 *kc, *vc;        // [n_kv][ctx][hd]
-    float *out;                     // [n][n_head * hd]
-    uint32_t n, pos0, n_head, n_kv, ctx;
+    float *out;                     // [S][n][n_head * hd]: each split's sum of e^(s - m) v
+    float2 *ml;                     // [S][n][n_head]: its {m, sum of e^(s - m)}
+    uint32_t n, pos0, n_head, n_kv, ctx, S;
     float scale;
 };
 
@@ -200,7 +201,8 @@ __global__ __launch_bounds__(64 * NW) void k_attn_pf_mma(AttnPre a) {
     __shared__ __attribute__((aligned(16))) _Float16 Vt[2][HD * VLD];
     __shared__ __attribute__((aligned(16))) _Float16 Vraw[VLDS ? 32 * HD : 8];
     const uint32_t rep = a.n_head / a.n_kv, ng = (rep + NW - 1) / NW;
-    const uint32_t qb = blockIdx.x, kh = blockIdx.y / ng;
+    // the last query blocks have the most positions: they start first
+    const uint32_t qb = gridDim.x / a.S - 1 - blockIdx.x / a.S, sp = blockIdx.x % a.S, kh = blockIdx.y / ng;
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, hf = lane >> 5;
     const uint32_t hl = (blockIdx.y % ng) * NW + wave;  // query head within the group
     const bool hact = hl < rep;                         // an idle wavefront stages and stores nothing
@@ -209,7 +211,13 @@ __global__ __launch_bounds__(64 * NW) void k_attn_pf_mma(AttnPre a) {
     const uint32_t qr = qi < a.n ? qi : a.n - 1;  // lanes past the block compute a copy, store nothing
     const uint32_t qpos = a.pos0 + qr;
     const uint32_t kend = a.pos0 + min(q0 + 32, a.n);  // positions 0..kend-1 are attended
-    const uint32_t nch = (kend + 31) / 32;
+    const uint32_t nall = (kend + 31) / 32, share = (nall + a.S - 1) / a.S;
+    const uint32_t c0 = sp * share, nch = min(c0 + share, nall);  // this split's chunks
+    const size_t row = (size_t)sp * a.n + qi;
+    if (c0 >= nall) {  // more splits than chunks: an empty share
+        if (hf == 0 && qi < a.n && hact) a.ml[row * a.n_head + h] = make_float2(-INFINITY, 0.f);
+        return;
+    }
     const _Float16 *kb = a.kc + (size_t)kh * a.ctx * HD;
     const _Float16 *vb = a.vc + (size_t)kh * a.ctx * HD;
 
@@ -306,20 +314,20 @@ __global__ __launch_bounds__(64 * NW) void k_attn_pf_mma(AttnPre a) {
         for (int r = 0; r < 16; r++) o[t][r] = 0.f;
     float m = -INFINITY, l = 0.f;
 
-    stage_k(0, 0);
+    stage_k(c0, 0);
     if constexpr (VLDS) {
-        stage_vraw(0);
+        stage_vraw(c0);
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
         vraw_to_vt(0);
     } else {
-        load_v(0);
+        load_v(c0);
         store_v(0);
     }
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    for (uint32_t c = 0; c < nch; c++) {
-        const uint32_t cur = c & 1;
+    for (uint32_t c = c0; c < nch; c++) {
+        const uint32_t cur = (c - c0) & 1;
         const bool more = c + 1 < nch;
         if (more) {
             stage_k(c + 1, cur ^ 1);
@@ -349,7 +357,9 @@ __global__ __launch_bounds__(64 * NW) void k_attn_pf_mma(AttnPre a) {
             cmax = fmaxf(cmax, sc[r]);
         }
         cmax = fmaxf(cmax, __shfl_xor(cmax, 32, 64));
-        const float mn = fmaxf(m, cmax);  // finite: position 0 is in the first chunk
+        // a query before all of the share's positions so far has only -inf:
+        // any finite maximum then gives zeros
+        const float mn = fmaxf(m, cmax) == -INFINITY ? -1e30f : fmaxf(m, cmax);
         const float alpha = expf(m - mn);
         float ps = 0.f;
         f16x8_t ph[2], pl[2];
@@ -394,16 +404,65 @@ __global__ __launch_bounds__(64 * NW) void k_attn_pf_mma(AttnPre a) {
     }
     // out[token][head][dim]: lane holds dims 32 t + 8 (r/4) + 4 hf + r%4
     if (qi < a.n && hact) {
-        const float inv = 1.0f / l;
-        float *op = a.out + ((size_t)qi * a.n_head + h) * HD;
+        if (hf == 0) a.ml[row * a.n_head + h] = make_float2(m, l);
+        float *op = a.out + (row * a.n_head + h) * HD;
 #pragma unroll
         for (int t = 0; t < OT; t++)
 #pragma unroll
             for (int g = 0; g < 4; g++)
                 *reinterpret_cast<float4 *>(op + 32 * t + 8 * g + 4 * hf) =
-                    make_float4(o[t][4 * g] * inv, o[t][4 * g + 1] * inv, o[t][4 * g + 2] * inv,
-                                o[t][4 * g + 3] * inv);
+                    make_float4(o[t][4 * g], o[t][4 * g + 1], o[t][4 * g + 2], o[t][4 * g + 3]);
     }
+}
+
+// The splits of k_attn_pf_mma merged (softmax over the union of their
+// positions), times sigmoid(gate) for the hybrid (gate_quant.comp; qg holds a
+// head's query, then its gate), as the o projection's GEMM input.  Workgroup =
+// 8 rows x one super-block, eight elements per thread; the splits go by in
+// fours whose loads are in flight together (one at a time the 11 splits of a
+// 19-token turn took 34 us).
+__global__ __launch_bounds__(256) void k_attn_merge(const float *__restrict__ part, const float2 *__restrict__ ml,
+                                                    const float *__restrict__ qg, uint32_t S, uint32_t n,
+                                                    uint32_t n_head, uint32_t hd, uint8_t *__restrict__ planes) {
+    const uint32_t qd = n_head * hd, row = 8 * blockIdx.y + (threadIdx.x >> 5);
+    if (row >= n) return;
+    const uint32_t c = 32 * blockIdx.x + (threadIdx.x & 31), e = 8 * c, h = e / hd;
+    float m = -INFINITY, l = 0.f, v[8] = {};
+    for (uint32_t s0 = 0; s0 < S; s0 += 4) {
+        float2 p[4];
+        float4 a[4], b[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const size_t r = (size_t)min(s0 + i, S - 1) * n + row;
+            p[i] = ml[r * n_head + h];
+            if (s0 + i >= S) p[i] = make_float2(-INFINITY, 0.f);
+            a[i] = *reinterpret_cast<const float4 *>(part + r * qd + e);
+            b[i] = *reinterpret_cast<const float4 *>(part + r * qd + e + 4);
+        }
+        const float mn = fmaxf(fmaxf(fmaxf(p[0].x, p[1].x), fmaxf(p[2].x, p[3].x)), m);
+        const float old = m == -INFINITY ? 0.f : expf(m - mn);
+        l *= old;
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[i] *= old;
+        m = mn;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            if (p[i].y == 0.f) continue;  // an empty share: its sums were not written
+            const float w = expf(p[i].x - m);
+            l = fmaf(p[i].y, w, l);
+            const float x[8] = {a[i].x, a[i].y, a[i].z, a[i].w, b[i].x, b[i].y, b[i].z, b[i].w};
+#pragma unroll
+            for (int k = 0; k < 8; k++) v[k] = fmaf(w, x[k], v[k]);
+        }
+    }
+    const float inv = 1.0f / l;
+    const float *g = qg ? qg + (size_t)row * 2 * qd + (size_t)h * 2 * hd + hd + e % hd : nullptr;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        v[i] *= inv;
+        if (g) v[i] = v[i] * (1.0f / (1.0f + expf(-g[i])));
+    }
+    gp_store8<3>(v, row, c, qd >> 8, planes);
 }
 
 hipError_t launch_rmsnorm_rows(const float *X, const float *w, float eps, uint32_t E, uint32_t n,
@@ -432,11 +491,25 @@ hipError_t launch_qkv_post(const float *qt, const float *kt, const float *vt, co
     return hipGetLastError();
 }
 
-hipError_t launch_attn_prefill(const float *q, const _Float16 *kc, const _Float16 *vc, float *out,
-                               uint32_t n, uint32_t pos0, uint32_t n_head, uint32_t n_kv,
-                               uint32_t hd, uint32_t ctx, hipStream_t s) {
-    if (n == 0 || n_kv == 0 || n_head % n_kv || n_head / n_kv > 8) return hipErrorInvalidValue;
-    AttnPre a = {q, kc, vc, out, n, pos0, n_head, n_kv, ctx, 1.0f / sqrtf((float)hd)};
+// Splits of the cache positions of a block of n tokens: about one workgroup
+// per CU (the five wavefronts of the 32B shape's head groups leave no room for
+// a second), at most one split per chunk of the last query block.  With the
+// merge, 32B shape, us per layer: 512 tokens from position 0 64 -> 47 (four
+// splits a block: 70), 19 tokens behind 333 positions 42 -> 18.
+uint32_t attn_prefill_splits(uint32_t n, uint32_t pos0, uint32_t n_head, uint32_t n_kv, uint32_t hd) {
+    const uint32_t rep = n_head / n_kv, ng = hd == 256 ? (rep + 3) / 4 : 1;
+    const uint32_t wgs = (n + 31) / 32 * n_kv * ng, chunks = (pos0 + n + 31) / 32;
+    const uint32_t want = (256 + wgs - 1) / wgs;
+    return want < chunks ? want : chunks;
+}
+
+hipError_t launch_attn_prefill(const float *q, const _Float16 *kc, const _Float16 *vc, const float *qg, float *part,
+                               float2 *ml, uint32_t n, uint32_t pos0, uint32_t n_head, uint32_t n_kv,
+                               uint32_t hd, uint32_t ctx, uint8_t *planes, hipStream_t s) {
+    if (n == 0 || n_kv == 0 || n_head % n_kv || n_head / n_kv > 8 || (n_head * hd) % 256)
+        return hipErrorInvalidValue;
+    const uint32_t S = attn_prefill_splits(n, pos0, n_head, n_kv, hd);
+    AttnPre a = {q, kc, vc, part, ml, n, pos0, n_head, n_kv, ctx, S, 1.0f / sqrtf((float)hd)};
     const uint32_t rep = n_head / n_kv;
     // wavefronts per workgroup: the whole group, or at head_dim 256 an even
     // share of it in groups of at most 4
@@ -462,7 +535,9 @@ hipError_t launch_attn_prefill(const float *q, const _Float16 *kc, const _Float1
 #undef LRS_PF_NW
     if (!fn) return hipErrorInvalidValue;
     const uint32_t ng = (rep + nw - 1) / nw;
-    hipLaunchKernelGGL(fn, dim3((n + 31) / 32, n_kv * ng), dim3(64 * nw), 0, s, a);
+    hipLaunchKernelGGL(fn, dim3((n + 31) / 32 * S, n_kv * ng), dim3(64 * nw), 0, s, a);
+    hipLaunchKernelGGL(k_attn_merge, dim3(n_head * hd / 256, (n + 7) / 8), dim3(256), 0, s, part, ml, qg, S, n,
+                       n_head, hd, planes);
     return hipGetLastError();
 }
 
