@@ -118,9 +118,10 @@ int lrs_weight_dequant_dev(lrs_ctx *ctx, const lrs_weight *w, float *out_dev);
 int lrs_matvec_f32(lrs_ctx *ctx, const lrs_weight *w, const float *x, float *y,
                    uint32_t cols);
 /* Same on device buffers, enqueued on the context stream (async).  Q8_0
- * weights, several columns and inputs of up to 4096 elements are packed by
- * the matvec launch itself (no scratch); wider single K-quant columns take a
- * pack launch into the context scratch first. */
+ * weights and inputs of up to 4096 elements are packed by the matvec launch
+ * itself (no scratch); wider single K-quant columns take a pack launch into
+ * the context scratch first, and so do several columns where the scratch
+ * holds their packs or may grow (else they are packed by the launch too). */
 int lrs_matvec_dev(lrs_ctx *ctx, const lrs_weight *w, const float *x_dev, float *y_dev,
                    uint32_t cols);
 

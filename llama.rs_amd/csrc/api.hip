@@ -102,6 +102,21 @@ static int ctx_scratch(lrs_ctx *ctx, size_t bytes, void **p) {
     *p = s.p;
     return LRS_OK;
 }
+// the scratch if it can be had without an error: null where growing it is
+// refused (a capture, a live graph), for callers that have another way
+static void *ctx_scratch_or_null(lrs_ctx *ctx, size_t bytes) {
+    {
+        std::lock_guard<std::mutex> lk(g_scratch_mu);
+        const lrs_ctx_scratch &s = g_scratch[ctx];
+        if (s.n >= bytes) return s.p;
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        if (ctx->live_graphs > 0 || hipStreamIsCapturing(ctx->stream, &cs) != hipSuccess ||
+            cs != hipStreamCaptureStatusNone)
+            return nullptr;
+    }
+    void *p = nullptr;
+    return ctx_scratch(ctx, bytes, &p) == LRS_OK ? p : nullptr;
+}
 }  // namespace lrs
 
 // ---- input pack of lrs_matvec_dev_noalloc ---------------------------------
@@ -353,7 +368,8 @@ int lrs_matvec_dev(lrs_ctx *ctx, const lrs_weight *w, const float *x_dev, float 
     if (!matvec_packs_in_kernel(w->v, cols))
         if (int rc_ = ctx_scratch(ctx, xpack_bytes(pack_blocks(w->v.type, w->v.n_in)), &pack))
             return rc_;
-    LRS_HIP(launch_matvec(w->v, x_dev, y_dev, cols, pack, ctx->stream));
+    const size_t cb = matvec_cols_bytes(w->v, cols);
+    LRS_HIP(launch_matvec(w->v, x_dev, y_dev, cols, pack, ctx->stream, cb ? ctx_scratch_or_null(ctx, cb) : nullptr));
     return LRS_OK;
 }
 
@@ -407,13 +423,18 @@ int lrs_matvec_f32(lrs_ctx *ctx, const lrs_weight *w, const float *x, float *y, 
     const size_t pb =
         matvec_packs_in_kernel(w->v, cols) ? 0 : xpack_bytes(pack_blocks(w->v.type, w->v.n_in));
     auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
-    void *buf = nullptr;
-    if (int rc_ = ctx_scratch(ctx, up(xb) + up(yb) + pb, &buf)) return rc_;
+    // several columns' packs where the scratch may hold them too
+    const size_t cb = matvec_cols_bytes(w->v, cols);
+    void *buf = cb ? ctx_scratch_or_null(ctx, up(xb) + up(yb) + cb) : nullptr, *cpack = nullptr;
+    if (buf)
+        cpack = (char *)buf + up(xb) + up(yb);
+    else if (int rc_ = ctx_scratch(ctx, up(xb) + up(yb) + pb, &buf))
+        return rc_;
     float *xd = (float *)buf;
     float *yd = (float *)((char *)buf + up(xb));
     void *pack = pb ? (char *)buf + up(xb) + up(yb) : nullptr;
     LRS_HIP(hipMemcpyAsync(xd, x, xb, hipMemcpyHostToDevice, ctx->stream));
-    LRS_HIP(launch_matvec(w->v, xd, yd, cols, pack, ctx->stream));
+    LRS_HIP(launch_matvec(w->v, xd, yd, cols, pack, ctx->stream, cpack));
     LRS_HIP(hipMemcpyAsync(y, yd, yb, hipMemcpyDeviceToHost, ctx->stream));
     LRS_HIP(hipStreamSynchronize(ctx->stream));
     return LRS_OK;

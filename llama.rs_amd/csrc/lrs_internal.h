@@ -118,11 +118,14 @@ inline uint32_t pack_blocks(uint32_t t, uint32_t n_in) {
 hipError_t launch_argmax_finish(const unsigned long long *keys, uint32_t n, uint32_t *step,
                                 uint32_t *out, uint32_t out_cap, hipStream_t s);
 // y[c] = W x[c] for cols columns: when matvec_packs_in_kernel, up to 8
-// columns per launch share each weight load and every workgroup packs its
-// input columns itself (`pack` unused, may be null); otherwise the staged
-// form below with `pack` (xpack_bytes of the weight)
+// columns per launch share each weight load.  With cols_pack
+// (matvec_cols_bytes; 0: none needed) several columns are packed by a launch
+// before; without it, and for one column, every workgroup packs its input
+// columns itself (`pack` unused, may be null).  Otherwise the staged form
+// below with `pack` (xpack_bytes of the weight)
 hipError_t launch_matvec(WeightView w, const float *x, float *y, uint32_t cols, void *pack,
-                         hipStream_t s);
+                         hipStream_t s, void *cols_pack = nullptr);
+size_t matvec_cols_bytes(WeightView w, uint32_t cols);
 bool matvec_packs_in_kernel(WeightView w, uint32_t cols);
 // the staged form: each column packed into `pack` by its own launch, then one
 // matvec launch per column over that pack (same results)

@@ -99,6 +99,16 @@ __global__ __launch_bounds__(256) void k_xpack(const float *__restrict__ x,
     }
 }
 
+// the x-packs of gridDim.y columns: their digits one after the other, then
+// their meta (as k_mqs stages them)
+__global__ __launch_bounds__(256) void k_xpack_cols(const float *__restrict__ x, uint32_t n, uint32_t nxb, XPack p) {
+    const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x, c = blockIdx.y;
+    if (e >= 32 * nxb) return;  // whole half-waves leave together
+    p.dig += (size_t)c * nxb * 96;
+    p.meta += (size_t)c * nxb * 4;
+    pack_half(e < n ? x[(size_t)c * n + e] : 0.f, e >> 5, p);
+}
+
 hipError_t launch_xpack(const float *x, const float *nw, uint32_t n, uint32_t nxb, XPack p,
                         hipStream_t s, float *xsq) {
     const uint32_t threads = 32 * nxb;
@@ -589,10 +599,10 @@ __device__ __forceinline__ void mq_body(const MqArgs &a, uint32_t si, uint8_t *l
             }
         }
     } else if constexpr (!WT) {
-        const uint32_t bb0 = XSN > 1 ? ub * BPU : 0u;
-        copy_to_lds(reinterpret_cast<const uint8_t *>(a.xin.dig) + (size_t)bb0 * 96, lds, nxl * 96);
+        const uint32_t bb0 = XSN > 1 ? ub * BPU : 0u, nst = NC > 1 ? a.ncols : 1u;  // columns staged
+        copy_to_lds(reinterpret_cast<const uint8_t *>(a.xin.dig) + (size_t)bb0 * 96, lds, nst * nxl * 96);
         copy_to_lds(reinterpret_cast<const uint8_t *>(a.xin.meta + 4 * (size_t)bb0), lds + lp.meta,
-                    nxl * 16);
+                    nst * nxl * 16);
     }
     if (threadIdx.x < 4) reinterpret_cast<uint32_t *>(lds + lp.zero)[threadIdx.x] = 0u;
     // the epilogue's operands of this thread's output (thread i owns output i
@@ -880,7 +890,7 @@ __device__ __forceinline__ void mq_body(const MqArgs &a, uint32_t si, uint8_t *l
             for (int c = 1; c < NC; c++) {
                 float yc = s * partial(grp, tt, ii & 15, c);
                 if (sg.bias) yc = yc + e_bias;
-                sg.out[(size_t)c * a.ostride + row] = yc;
+                if (XF || (uint32_t)c < a.ncols) sg.out[(size_t)c * a.ostride + row] = yc;
             }
         }
     } else if constexpr (EPI == MQ_STORE) {
@@ -1066,6 +1076,22 @@ __attribute__((amdgpu_waves_per_eu(mq_waves_per_eu<TG * KS>()))) void k_mqx(MqAr
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     __shared__ float red[NC * TG * KS * TPW * 16 + TG * KS + 1];
     mq_body<T, TPW, TG, KS, P, MQ_STORE, NC, true>(a, 0, lds, red);
+}
+
+// Matvec of up to NC columns over packs made by an earlier launch (a.xin: the
+// columns' digits one after the other, then their meta).  Packing in the
+// kernel costs every workgroup the pack of every column (about 50 vector
+// operations an element: 8 us of a 4-column launch at K = 5120), which a pack
+// launch does once and the workgroups then copy.  us per call, in-kernel pack
+// -> staged: Q4_K 13824 x 5120 2 / 4 / 8 columns 17.6 / 28.4 / 56.5 ->
+// 12.0 / 15.8 / 29.7, Q8_0 4096 x 4096 8.3 / 13.3 / 23.7 -> 7.9 / 9.4 / 12.1.
+// Eight columns' packs leave room for one workgroup per CU: all its registers.
+template <uint32_t T, int TPW, int TG, int KS, int P, int NC>
+__global__ __launch_bounds__(64 * TG * KS)
+__attribute__((amdgpu_waves_per_eu(NC == 8 ? (TG * KS + 3) / 4 : mq_waves_per_eu<TG * KS>()))) void k_mqs(MqArgs a) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    __shared__ float red[NC * TG * KS * TPW * 16 + TG * KS + 1];
+    mq_body<T, TPW, TG, KS, P, MQ_STORE, NC, false>(a, 0, lds, red);
 }
 
 // ---------------------------------------------------------------------------
@@ -1450,25 +1476,41 @@ static MqFn pick_nc(int nc) {
     }
 }
 
-// the launch shapes store_geom picks (without a tuning override)
-template <uint32_t T>
-static MqFn pick_x_geom(const MqGeom &g, int nc) {
-    if constexpr (T == T_Q8_0) {
-        if (g.tpw == 1 && g.tg == 1 && g.ks == 16 && g.p == 4) return pick_nc<T, 1, 1, 16, 4>(nc);
-    } else {
-        if (g.tpw == 1 && g.tg == 2 && g.ks == 2 && g.p == 2) return pick_nc<T, 1, 2, 2, 2>(nc);
-        if (g.tpw == 1 && g.tg == 2 && g.ks == 4 && g.p == 2) return pick_nc<T, 1, 2, 4, 2>(nc);
-        if (g.tpw == 1 && g.tg == 1 && g.ks == 4 && g.p == 2) return pick_nc<T, 1, 1, 4, 2>(nc);
+// ... and over packs of an earlier launch (k_mqs)
+template <uint32_t T, int TPW, int TG, int KS, int P>
+static MqFn pick_ncs(int nc) {
+    switch (nc) {
+    case 2: return k_mqs<T, TPW, TG, KS, P, 2>;
+    case 4: return k_mqs<T, TPW, TG, KS, P, 4>;
+    case 8: return k_mqs<T, TPW, TG, KS, P, 8>;
+    default: return nullptr;
     }
+}
+
+// the launch shapes store_geom picks (without a tuning override); staged:
+// over packs of an earlier launch
+template <uint32_t T>
+static MqFn pick_x_geom(const MqGeom &g, int nc, bool staged) {
+#define LRS_MQX_CASE(TPW, TG, KS, P)                    \
+    if (g.tpw == TPW && g.tg == TG && g.ks == KS && g.p == P) \
+        return staged ? pick_ncs<T, TPW, TG, KS, P>(nc) : pick_nc<T, TPW, TG, KS, P>(nc);
+    if constexpr (T == T_Q8_0) {
+        LRS_MQX_CASE(1, 1, 16, 4)
+    } else {
+        LRS_MQX_CASE(1, 2, 2, 2)
+        LRS_MQX_CASE(1, 2, 4, 2)
+        LRS_MQX_CASE(1, 1, 4, 2)
+    }
+#undef LRS_MQX_CASE
     return nullptr;
 }
 
-static MqFn pick_x(uint32_t t, const MqGeom &g, int nc) {
+static MqFn pick_x(uint32_t t, const MqGeom &g, int nc, bool staged = false) {
     switch (t) {
-    case T_Q4_K: return pick_x_geom<T_Q4_K>(g, nc);
-    case T_Q5_K: return pick_x_geom<T_Q5_K>(g, nc);
-    case T_Q6_K: return pick_x_geom<T_Q6_K>(g, nc);
-    case T_Q8_0: return pick_x_geom<T_Q8_0>(g, nc);
+    case T_Q4_K: return pick_x_geom<T_Q4_K>(g, nc, staged);
+    case T_Q5_K: return pick_x_geom<T_Q5_K>(g, nc, staged);
+    case T_Q6_K: return pick_x_geom<T_Q6_K>(g, nc, staged);
+    case T_Q8_0: return pick_x_geom<T_Q8_0>(g, nc, staged);
     default: return nullptr;
     }
 }
@@ -1492,37 +1534,73 @@ bool matvec_packs_in_kernel(WeightView w, uint32_t cols) {
     return w.type == T_Q8_0 || cols > 1 || 32 * nxb <= 8 * 64 * (uint32_t)(g.tg * g.ks);
 }
 
-hipError_t launch_matvec(WeightView w, const float *x, float *y, uint32_t cols, void *pack,
-                         hipStream_t s) {
-    if (!is_tiled(w.type)) return hipErrorInvalidValue;
+// columns that one pack launch makes (and the scratch holds) at a time
+static constexpr uint32_t MQS_COLS = 32;
+
+// the matvec launches of columns [0, cols): up to 8 per launch share every
+// weight load.  Each column's arithmetic is the single-column kernel's (same
+// K-slices, same order), so the results do not depend on the grouping.
+// staged: over the packs at `pack` (k_xpack_cols), else packed in the kernel
+// (K-quants then take at most 4 columns)
+static hipError_t launch_columns(WeightView w, const float *x, float *y, uint32_t cols, void *pack, bool staged,
+                                 hipStream_t s) {
     const uint32_t nxb = pack_blocks(w.type, w.n_in);
     const MqGeom g = store_geom(w.type, w.n_in, w.n_out);
-    if (matvec_packs_in_kernel(w, cols)) {
-        // up to 8 columns per launch share every weight load; each column's
-        // arithmetic is the single-column kernel's (same K-slices, same
-        // order), so the results do not depend on the grouping
-        // K-quants: at most 4 columns (8 need more than 128 VGPRs, fewer waves)
-        const int nc_max = w.type == T_Q8_0 ? 8 : 4;
-        for (uint32_t c0 = 0; c0 < cols;) {
-            int nc = nc_max;
-            while (nc > 1 && ((uint32_t)nc > cols - c0 || mqx_lds(nxb, nc) > MQX_LDS_MAX)) nc >>= 1;
-            MqArgs a = {};
-            a.n_seg = a.n_seg0 = 1;
-            a.seg[0].w = w.q;
-            a.seg[0].rows = w.n_out;
-            a.seg[0].out = y + (size_t)c0 * w.n_out;
-            a.seg[0].wg0 = 0;
-            a.n_in = w.n_in;
-            a.nxb = nxb;
+    const uint32_t nc_max = staged || w.type == T_Q8_0 ? 8 : 4;
+    for (uint32_t c0 = 0; c0 < cols;) {
+        uint32_t nc = nc_max;
+        // a staged launch may be short of columns: one of four with three of
+        // them takes less than one of two and one of one
+        while (nc > 1 && ((staged ? nc / 2 : nc - 1) >= cols - c0 || mqx_lds(nxb, (int)nc) > MQX_LDS_MAX)) nc >>= 1;
+        MqArgs a = {};
+        a.n_seg = a.n_seg0 = 1;
+        a.seg[0].w = w.q;
+        a.seg[0].rows = w.n_out;
+        a.seg[0].out = y + (size_t)c0 * w.n_out;
+        a.seg[0].wg0 = 0;
+        a.n_in = w.n_in;
+        a.nxb = nxb;
+        a.ostride = w.n_out;
+        a.ncols = min(nc, cols - c0);
+        const bool over = staged && nc > 1;  // a last single column is packed in the kernel
+        if (over) {
+            a.xin.dig = reinterpret_cast<int8_t *>(pack) + (size_t)c0 * nxb * 96;
+            a.xin.meta = reinterpret_cast<float *>(reinterpret_cast<char *>(pack) + (size_t)cols * nxb * 96) +
+                         (size_t)c0 * nxb * 4;
+        } else {
             a.xf = x + (size_t)c0 * w.n_in;
-            a.ostride = w.n_out;
-            const uint32_t per = (uint32_t)(g.tg * g.tpw);
-            const uint32_t wgs = (ttiles(w.n_out) + per - 1) / per;
-            hipLaunchKernelGGL(pick_x(w.type, g, nc), dim3(wgs), dim3(64 * g.tg * g.ks),
-                               mqx_lds(nxb, nc), s, a);
-            const hipError_t e = hipGetLastError();
+        }
+        const uint32_t per = (uint32_t)(g.tg * g.tpw);
+        hipLaunchKernelGGL(pick_x(w.type, g, (int)nc, over), dim3((ttiles(w.n_out) + per - 1) / per),
+                           dim3(64 * g.tg * g.ks), mqx_lds(nxb, (int)nc), s, a);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        c0 += a.ncols;
+    }
+    return hipSuccess;
+}
+
+size_t matvec_cols_bytes(WeightView w, uint32_t cols) {
+    if (cols < 2 || !matvec_packs_in_kernel(w, cols)) return 0;
+    return (size_t)min(cols, MQS_COLS) * xpack_bytes(pack_blocks(w.type, w.n_in));
+}
+
+hipError_t launch_matvec(WeightView w, const float *x, float *y, uint32_t cols, void *pack,
+                         hipStream_t s, void *cols_pack) {
+    if (!is_tiled(w.type)) return hipErrorInvalidValue;
+    if (matvec_packs_in_kernel(w, cols)) {
+        if (!cols_pack || cols < 2) return launch_columns(w, x, y, cols, nullptr, false, s);
+        const uint32_t nxb = pack_blocks(w.type, w.n_in);
+        for (uint32_t c0 = 0; c0 < cols; c0 += MQS_COLS) {
+            const uint32_t n = min(MQS_COLS, cols - c0);
+            XPack xp;
+            xp.dig = reinterpret_cast<int8_t *>(cols_pack);
+            xp.meta = reinterpret_cast<float *>(reinterpret_cast<char *>(cols_pack) + (size_t)n * nxb * 96);
+            xp.q8 = 0;
+            const float *xc = x + (size_t)c0 * w.n_in;
+            hipLaunchKernelGGL(k_xpack_cols, dim3((32 * nxb + 255) / 256, n), dim3(256), 0, s, xc, w.n_in, nxb, xp);
+            const hipError_t e = launch_columns(w, xc, y + (size_t)c0 * w.n_out, n, cols_pack, true, s);
             if (e != hipSuccess) return e;
-            c0 += (uint32_t)nc;
         }
         return hipSuccess;
     }

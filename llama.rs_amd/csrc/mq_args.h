@@ -89,6 +89,9 @@ struct MqArgs {
     // the input at xf + c * n_in, its outputs at seg[0].out + c * ostride
     const float *xf;
     uint32_t ostride;
+    // columns of a k_mqs launch that exist (at most its NC; the rest compute on
+    // whatever LDS holds and store nothing)
+    uint32_t ncols;
     // MQ_RESID / MQ_SWIGLU split over K across workgroups: xsplit workgroups
     // per 32-output block, each over its own contiguous share of the units;
     // each writes its partial sums to xpart[(block * xsplit + slice) * 32 + i]

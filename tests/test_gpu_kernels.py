@@ -476,3 +476,51 @@ def test_q8_actq_columns_and_errors(lrs, orc, ctx):
         lrs.Weight.upload(ctx, Q4_K, w4, n_in, n_out).matvec_actq(xs[0])
     with pytest.raises(lrs.ModelError):
         lrs.quantize_q8_0(ctx, np.ones(33, np.float32))
+
+
+@pytest.mark.parametrize("t,n_in,n_out", [(Q4_K, 5120, 40), (Q5_K, 1024, 33), (Q6_K, 11264, 17),
+                                          (Q8_0, 2080, 16), (Q4_K, 12288, 5)])
+def test_matvec_columns_staged_packs(lrs, orc, ctx, t, n_in, n_out):
+    """Launches of 2, 4 and 8 columns that are full, short of columns, or held
+    to fewer by the LDS their packs need (11264: 3 fit, 12288: 2), over more than
+    the 32 columns of one pack launch: each column exactly as alone, nothing
+    stored past the last."""
+    w = lrs.Weight.upload(ctx, t, orc.gen_weight(t, 3, n_out, n_in, mode=1), n_in, n_out)
+    x = np.random.default_rng(n_in).standard_normal((37, n_in)).astype(np.float32)
+    xb, yb = ctx.alloc(x.nbytes), ctx.alloc(4 * (37 * n_out + 16))
+    xb.upload(x)
+    alone = np.stack([w.matvec(v) for v in x])
+    for cols in (2, 3, 4, 5, 7, 8, 9, 32, 33, 37):
+        yb.upload(np.full(37 * n_out + 16, 7.0, np.float32))
+        w.matvec_dev(xb, yb, cols)
+        ctx.sync()
+        y = yb.download(np.float32, 37 * n_out + 16)
+        assert np.array_equal(y[:cols * n_out].reshape(cols, n_out), alone[:cols])
+        assert np.all(y[cols * n_out:] == 7.0)
+    assert np.array_equal(w.matvec(x[:5]), alone[:5])
+
+
+def test_matvec_columns_where_the_scratch_may_not_grow(lrs, orc):
+    """Several columns need no scratch: a first call inside a capture (no
+    scratch yet), and calls while a graph lives (none may be made), pack in the
+    kernel with the same results, replays included."""
+    n_in, n_out, cols = 1024, 48, 5
+    with lrs.Context(0) as c:
+        w = lrs.Weight.upload(c, Q4_K, orc.gen_weight(Q4_K, 8, n_out, n_in, mode=1), n_in, n_out)
+        x = np.random.default_rng(1).standard_normal((cols, n_in)).astype(np.float32)
+        xb, yb = c.alloc(x.nbytes), c.alloc(4 * cols * n_out)
+        xb.upload(x)
+        g = c.capture(lambda: w.matvec_dev(xb, yb, cols))
+        w.matvec_dev(xb, yb, cols)
+        c.sync()
+        eager = yb.download(np.float32, cols * n_out)
+        for _ in range(3):
+            yb.upload(np.zeros(cols * n_out, np.float32))
+            g.launch()
+            c.sync()
+            assert np.array_equal(yb.download(np.float32, cols * n_out), eager)
+        g.close()
+        w.matvec_dev(xb, yb, cols)  # now with the scratch
+        c.sync()
+        assert np.array_equal(yb.download(np.float32, cols * n_out), eager)
+        assert np.array_equal(np.stack([w.matvec(v) for v in x]).ravel(), eager)
