@@ -713,7 +713,7 @@ static PgPlan pg_plan(uint32_t M, const uint32_t *N, const uint32_t *type, uint3
         const uint32_t tiles = pg_tiles(M, N, nseg, mt);
         const uint32_t fit = mt == (prec == 3 ? 2u : 4u) || (wide && !(prec == 1 && mt == 1)) ? 2 : 3;
         for (uint32_t ks = 1; ks <= nsb && ks <= 32; ks++) {
-            if (ks > 1 && (!have_work || tiles >= 2048)) break;
+            if (ks > 1 && (!have_work || tiles >= 2048 || M > 65535)) break;  // the reduce's grid has a y row per token
             const uint32_t len = (nsb + ks - 1) / ks, per = (tiles * ks + 255) / 256;
             const double rel = per < fit ? slow : per == fit ? 0.5 * (slow + mean) : mean;
             double cost = (len + 0.5) * rel * pg_unit(prec, mt, fit, per);
