@@ -115,7 +115,9 @@ static void *ctx_scratch_or_null(lrs_ctx *ctx, size_t bytes) {
             return nullptr;
     }
     void *p = nullptr;
-    return ctx_scratch(ctx, bytes, &p) == LRS_OK ? p : nullptr;
+    if (ctx_scratch(ctx, bytes, &p) == LRS_OK) return p;
+    (void)hipGetLastError();  // the caller's launches must not report it
+    return nullptr;
 }
 }  // namespace lrs
 
@@ -441,18 +443,21 @@ int lrs_matvec_f32(lrs_ctx *ctx, const lrs_weight *w, const float *x, float *y, 
 }
 
 // the input packed into context scratch, then the GEMM (its K-slice partials
-// behind the packed input)
+// behind the packed input, where the scratch holds them or may grow: else one
+// slice)
 static int gemm_run(lrs_ctx *ctx, const WeightView *wv, float *const *y, const uint32_t *ldy, uint32_t n_w,
                     const float *a_dev, uint32_t m, int precision) {
     const size_t ab = gemm_planes_bytes(m, wv[0].n_in, precision);
     uint32_t types[3];
     for (uint32_t i = 0; i < n_w; i++) types[i] = wv[i].type;
     const size_t wb = gemm_work_bytes(m, ldy, types, n_w, wv[0].n_in, precision);
-    void *buf = nullptr;
-    if (int rc_ = ctx_scratch(ctx, ab + wb, &buf)) return rc_;
+    void *buf = ctx_scratch_or_null(ctx, ab + wb);
+    const bool work = buf && wb;
+    if (!buf)
+        if (int rc_ = ctx_scratch(ctx, ab, &buf)) return rc_;
     LRS_HIP(launch_gemm_pack(a_dev, m, wv[0].n_in, precision, (uint8_t *)buf, ctx->stream));
     LRS_HIP(launch_gemm_segs(wv, y, ldy, n_w, (const uint8_t *)buf, m, precision, ctx->stream, false,
-                             wb ? (float *)((char *)buf + ab) : nullptr, wb));
+                             work ? (float *)((char *)buf + ab) : nullptr, work ? wb : 0));
     return LRS_OK;
 }
 

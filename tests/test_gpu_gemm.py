@@ -188,3 +188,27 @@ def test_dequant_into_any_float_address_is_exact(lrs, orc, ctx, t, n, k, shift):
     ref = orc.dequant(t, w)
     assert np.array_equal(got[shift:shift + n * k].view(np.uint32), ref.view(np.uint32))
     assert np.all(got[:shift] == 7.0) and np.all(got[shift + n * k:] == 7.0)
+
+
+def test_gemm_whose_partials_do_not_fit_the_scratch_runs_unsplit(lrs, orc):
+    """Inside a capture the scratch may not grow: where it holds the packed
+    input but not the K slices' partial sums the GEMM takes one slice (the same
+    sums in another order: 1e-6)."""
+    n_in, n_out, m = 1280, 2048, 64
+    with lrs.Context(0) as c:
+        small = lrs.Weight.upload(c, Q4_K, orc.gen_weight(Q4_K, 1, 16, n_in), n_in, 16)
+        w = lrs.Weight.upload(c, Q4_K, orc.gen_weight(Q4_K, 2, n_out, n_in, mode=1), n_in, n_out)
+        a = np.random.default_rng(5).standard_normal((m, n_in)).astype(np.float32)
+        small.gemm(a, precision=3)  # the scratch holds this input
+        ab, yb = c.alloc(a.nbytes), c.alloc(4 * m * n_out)
+        ab.upload(a)
+        g = c.capture(lambda: w.gemm_dev(ab, yb, m, 3))
+        got = []
+        for _ in range(2):
+            yb.upload(np.zeros(m * n_out, np.float32))
+            g.launch()
+            c.sync()
+            got.append(yb.download(np.float32, m * n_out).reshape(m, n_out))
+        g.close()
+        assert np.array_equal(got[0], got[1])
+        assert rel_l2(got[0], w.gemm(a, precision=3)) < 1e-6
