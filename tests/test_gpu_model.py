@@ -255,6 +255,28 @@ def test_batched_prompt_matches_oracle(lrs, orc, ctx, name, cfg, mix, n, seed):
     assert gm.generate_greedy(short, 32).tolist() == modelgen.oracle_greedy(om3, short, 32)
 
 
+# KSPLIT: the K slices' reduce is its own launch below 192 rows and fused with
+# the norm from there on.  GQA5: positions split into shares of one chunk with
+# masked and empty ones (19 and 3 rows behind a context that is no multiple of
+# 32), and of several chunks with an uneven last one (321 rows)
+@pytest.mark.parametrize("cfg,pos0,n", [(modelgen.KSPLIT, 0, 191), (modelgen.KSPLIT, 0, 192),
+                                        (modelgen.GQA5, 333, 19), (modelgen.GQA5, 33, 3),
+                                        (modelgen.GQA5, 101, 321)])
+def test_prompt_block_edges_match_oracle(lrs, orc, ctx, cfg, pos0, n):
+    """A prompt block at the edges of its launch rules against Model::forward,
+    and a decode step over the cache that it wrote."""
+    cfg = dict(cfg, ctx=448)
+    w = modelgen.host_model(orc, cfg, seed=21, mode=0, d_lo=1e-3, d_hi=1e-2)
+    gm = modelgen.gpu_model(lrs, ctx, cfg, w)
+    om = orc.Model(cfg, w, kv_f16=True, threads=8, q8_actq=False)
+    toks = np.random.default_rng(n).integers(0, cfg["vocab"], pos0 + n + 1).tolist()
+    if pos0:
+        gm.decode_batch(toks[:pos0], 0)
+    g, o = gm.decode_batch(toks[pos0:-1], pos0), om.forward(toks[:-1])
+    assert rel_l2(g, o) < LOGIT_TOL
+    assert rel_l2(gm.decode(toks[-1], pos0 + n), om.forward(toks[-1:])) < LOGIT_TOL
+
+
 def test_prefill_in_blocks_matches_token_by_token(lrs, orc, ctx):
     """integration.rs:1916-1995: 2 * batch_size() + 3 tokens, whole blocks
     through decode_batch and the rest through decode, against decode() token
