@@ -118,6 +118,9 @@ struct DevLayer {
     bool qkv_q8 = false, o_q8 = false, ffn_q8 = false, down_q8 = false;
 };
 
+// Tokens per block of the batched prompt path (batch_size()).
+static constexpr uint32_t PREFILL_BLOCK = 512;
+
 struct lrs_model {
     lrs_ctx *ctx;
     lrs_config cfg;
@@ -184,7 +187,7 @@ struct lrs_model {
     size_t work_bytes = 0;
     uint32_t *ptok;
     _Float16 *kv;                // all layers' caches
-    uint32_t *step_host;         // pinned
+    uint32_t *words_host;        // pinned: a block's token ids or a result, then the wait-error word
     float *logits_host;          // pinned
     uint32_t *gen_host;          // pinned [gen_cap]: generated tokens on their way out
     hipGraphExec_t g_logits = nullptr, g_greedy = nullptr;
@@ -918,8 +921,7 @@ int finish_model(lrs_model *m, const float *output_norm, const std::vector<float
             if (hipMemset(m->rope_cs, 0, rb) != hipSuccess) return fail(LRS_E_HIP, "memset");
         }
     }
-    // 1024 step slots of 4 words (enqueue_tokens), then the wait-error word
-    if (hipHostMalloc((void **)&m->step_host, (4 * 1024 + 4) * sizeof(uint32_t), hipHostMallocDefault) !=
+    if (hipHostMalloc((void **)&m->words_host, (PREFILL_BLOCK + 4) * sizeof(uint32_t), hipHostMallocDefault) !=
             hipSuccess ||
         hipHostMalloc((void **)&m->logits_host, c.vocab * sizeof(float), hipHostMallocDefault) !=
             hipSuccess ||
@@ -1177,7 +1179,7 @@ void lrs_model_destroy(lrs_model *m) {
     if (m->g_logits) (void)hipGraphExecDestroy(m->g_logits);
     if (m->g_greedy) (void)hipGraphExecDestroy(m->g_greedy);
     for (void *p : m->allocs) (void)hipFree(p);
-    if (m->step_host) (void)hipHostFree(m->step_host);
+    if (m->words_host) (void)hipHostFree(m->words_host);
     if (m->logits_host) (void)hipHostFree(m->logits_host);
     if (m->gen_host) (void)hipHostFree(m->gen_host);
     for (lrs_weight *w : m->owned) lrs_weight_free(w);
@@ -1194,18 +1196,43 @@ static int check_continue(lrs_model *m, uint32_t pos0) {
     return LRS_OK;
 }
 
-// the wait-error word of the combine + o launches (a matvec workgroup that
-// ran out of polls went on without its input): copied out with each call's
-// results, checked after the call's synchronisation
-static constexpr uint32_t AO_ERR_WORD = 4 * 1024;  // past the step slots of step_host
-static hipError_t ao_err_fetch(lrs_model *m, hipStream_t s) {
-    m->step_host[AO_ERR_WORD] = 0;
-    if (!m->ao_sync) return hipSuccess;
-    return hipMemcpyAsync(m->step_host + AO_ERR_WORD, m->ao_sync + 32, sizeof(uint32_t),
-                          hipMemcpyDeviceToHost, s);
+// {token, position, tokens generated so far} of the next forward.  As kernel
+// arguments: a 12-byte copy from pinned memory has the copy engine between two
+// launches.
+__global__ void k_set_step(uint32_t *step, uint32_t token, uint32_t pos) {
+    step[0] = token;
+    step[1] = pos;
+    step[2] = 0;
+}
+static hipError_t set_step(lrs_model *m, uint32_t token, uint32_t pos) {
+    hipLaunchKernelGGL(k_set_step, dim3(1), dim3(1), 0, m->ctx->stream, m->step, token, pos);
+    return hipGetLastError();
+}
+
+// n words into pinned host memory, and the wait-error word of the combine + o
+// launches (err null: none) behind them.  A launch in place of two copies: the
+// bus bounds it either way, the copy engine's start and the wait for it go.
+__global__ __launch_bounds__(256) void k_publish(const uint32_t *__restrict__ src, uint32_t n, uint32_t *__restrict__ host,
+                                                 const uint32_t *err, uint32_t *err_host) {
+    const uint32_t i = 4 * (blockIdx.x * 256 + threadIdx.x);
+    if (i == 0) *err_host = err ? *err : 0u;
+    if (i + 4 <= n)
+        *reinterpret_cast<uint4 *>(host + i) = *reinterpret_cast<const uint4 *>(src + i);
+    else
+        for (uint32_t k = i; k < n; k++) host[k] = src[k];
+}
+
+// the wait-error word (a matvec workgroup that ran out of polls went on
+// without its input): copied out with each call's results, checked after the
+// call's synchronisation
+static constexpr uint32_t AO_ERR_WORD = PREFILL_BLOCK;  // past the token ids in words_host
+static hipError_t publish(lrs_model *m, const uint32_t *src, uint32_t *host, uint32_t n) {
+    hipLaunchKernelGGL(k_publish, dim3((n + 1023) / 1024), dim3(256), 0, m->ctx->stream, src, n, host,
+                       m->ao_sync ? m->ao_sync + 32 : nullptr, m->words_host + AO_ERR_WORD);
+    return hipGetLastError();
 }
 static int ao_err_check(lrs_model *m) {
-    if (m->step_host[AO_ERR_WORD] == 0) return LRS_OK;
+    if (m->words_host[AO_ERR_WORD] == 0) return LRS_OK;
     // the word and the whole flag matrix back to zero: flags a late producer
     // raised after its consumer gave up must not release the next launch's
     (void)hipMemset(m->ao_sync, 0, m->ao_sync_bytes);
@@ -1222,8 +1249,9 @@ static int check_step(lrs_model *m, uint32_t token, uint32_t pos) {
 }
 
 // ---- batched prompt blocks on the matrix cores --------------------------
-// Tokens per block of the batched prompt path (batch_size()).
-static constexpr uint32_t PREFILL_BLOCK = 512;
+__global__ void k_words(const uint32_t *host, uint32_t n, uint32_t *dst) {
+    if (threadIdx.x < n) dst[threadIdx.x] = host[threadIdx.x];
+}
 
 // every matmul weight has a GEMM kernel and the attention shape is supported
 static bool prefill_capable(const lrs_model *m) {
@@ -1391,7 +1419,11 @@ static int prefill_block(lrs_model *m, const uint32_t *tokens, uint32_t nb, uint
         normed = true;
         return gemm_resid_norm(L.down, N.attn_norm, xn_for(N));
     };
-    LRS_HIP(hipMemcpyAsync(m->ptok, tokens, nb * sizeof(uint32_t), hipMemcpyHostToDevice, s));
+    // the token ids through pinned memory, read by a launch (the rows' launch
+    // would read each of them many times)
+    memcpy(m->words_host, tokens, nb * sizeof(uint32_t));
+    hipLaunchKernelGGL(k_words, dim3(1), dim3(PREFILL_BLOCK), 0, s, m->words_host, nb, m->ptok);
+    LRS_HIP(hipGetLastError());
     LRS_HIP(launch_dequant_rows(m->embd->v, m->ptok, nb, m->pX, s));
     for (uint32_t l = 0; l < c.n_layer; l++) {
         const DevLayer &L = m->layers[l];
@@ -1480,9 +1512,8 @@ static int prefill(lrs_model *m, const uint32_t *tokens, uint32_t n, uint32_t po
     uint32_t nb = 0;
     for (uint32_t i = 0; i < n; i += nb) {
         nb = min(m->pb_cap, n - i);
+        LRS_HIP(hipStreamSynchronize(s));  // the block before has read its token ids
         if ((rc = prefill_block(m, tokens + i, nb, pos0 + i))) return rc;
-        // the host token ids of this block must stay valid until it is read
-        LRS_HIP(hipStreamSynchronize(s));
     }
     if (!head) return LRS_OK;
     LRS_HIP(hipMemcpyAsync(m->x, m->pX + (size_t)(nb - 1) * m->cfg.n_embd,
@@ -1493,28 +1524,15 @@ static int prefill(lrs_model *m, const uint32_t *tokens, uint32_t n, uint32_t po
     return LRS_OK;
 }
 
-// enqueues n tokens at pos0.. (logits graph) without waiting; every token's
-// {token, pos} goes through its own pinned slot, and the stream is drained
-// whenever the slots run out
-static constexpr uint32_t STEP_SLOTS = 1024;
-static_assert(4 * STEP_SLOTS <= AO_ERR_WORD, "the wait-error word follows the step slots");
-
+// enqueues n tokens at pos0.. (logits graph) without waiting
 static int enqueue_tokens(lrs_model *m, const uint32_t *tokens, uint32_t n, uint32_t pos0) {
     for (uint32_t i = 0; i < n; i++) {
         int rc = check_step(m, tokens[i], pos0 + i);
         if (rc) return rc;
     }
     LRS_HIP(hipSetDevice(m->ctx->device));
-    hipStream_t s = m->ctx->stream;
-    LRS_HIP(hipStreamSynchronize(s));  // slots of an earlier call are free
     for (uint32_t i = 0; i < n; i++) {
-        const uint32_t slot = i % STEP_SLOTS;
-        if (i > 0 && slot == 0) LRS_HIP(hipStreamSynchronize(s));
-        uint32_t *sh = m->step_host + 4 * slot;
-        sh[0] = tokens[i];
-        sh[1] = pos0 + i;
-        sh[2] = 0;
-        LRS_HIP(hipMemcpyAsync(m->step, sh, 3 * sizeof(uint32_t), hipMemcpyHostToDevice, s));
+        LRS_HIP(set_step(m, tokens[i], pos0 + i));
         LRS_HIP(run_forward(m, false));
     }
     return LRS_OK;
@@ -1526,14 +1544,10 @@ int lrs_decode(lrs_model *m, uint32_t token, uint32_t pos, float *logits) {
     if (rc || (rc = check_continue(m, pos))) return rc;
     LRS_HIP(hipSetDevice(m->ctx->device));
     hipStream_t s = m->ctx->stream;
-    m->step_host[0] = token;
-    m->step_host[1] = pos;
-    m->step_host[2] = 0;
-    LRS_HIP(hipMemcpyAsync(m->step, m->step_host, 3 * sizeof(uint32_t), hipMemcpyHostToDevice, s));
+    LRS_HIP(set_step(m, token, pos));
     LRS_HIP(run_forward(m, false));
-    LRS_HIP(hipMemcpyAsync(m->logits_host, m->logits, m->cfg.vocab * sizeof(float),
-                           hipMemcpyDeviceToHost, s));
-    LRS_HIP(ao_err_fetch(m, s));
+    LRS_HIP(publish(m, reinterpret_cast<const uint32_t *>(m->logits), reinterpret_cast<uint32_t *>(m->logits_host),
+                    m->cfg.vocab));
     LRS_HIP(hipStreamSynchronize(s));
     if (int e = ao_err_check(m)) return e;
     memcpy(logits, m->logits_host, m->cfg.vocab * sizeof(float));
@@ -1557,15 +1571,13 @@ int lrs_decode_batch(lrs_model *m, const uint32_t *tokens, uint32_t n, uint32_t 
         for (uint32_t i = 0; i < n; i++)
             if ((rc = check_step(m, tokens[i], pos0 + i))) return rc;
         LRS_HIP(hipSetDevice(m->ctx->device));
-        LRS_HIP(hipStreamSynchronize(m->ctx->stream));
         if ((rc = prefill(m, tokens, n, pos0, true))) return rc;
     } else if ((rc = enqueue_tokens(m, tokens, n, pos0))) {
         return rc;
     }
     hipStream_t s = m->ctx->stream;
-    LRS_HIP(hipMemcpyAsync(m->logits_host, m->logits, m->cfg.vocab * sizeof(float),
-                           hipMemcpyDeviceToHost, s));
-    LRS_HIP(ao_err_fetch(m, s));
+    LRS_HIP(publish(m, reinterpret_cast<const uint32_t *>(m->logits), reinterpret_cast<uint32_t *>(m->logits_host),
+                    m->cfg.vocab));
     LRS_HIP(hipStreamSynchronize(s));
     if (int e = ao_err_check(m)) return e;
     memcpy(logits, m->logits_host, m->cfg.vocab * sizeof(float));
@@ -1602,16 +1614,12 @@ int lrs_decode_greedy(lrs_model *m, uint32_t token, uint32_t pos, uint32_t *next
     if (rc || (rc = check_continue(m, pos))) return rc;
     LRS_HIP(hipSetDevice(m->ctx->device));
     hipStream_t s = m->ctx->stream;
-    m->step_host[0] = token;
-    m->step_host[1] = pos;
-    m->step_host[2] = 0;
-    LRS_HIP(hipMemcpyAsync(m->step, m->step_host, 3 * sizeof(uint32_t), hipMemcpyHostToDevice, s));
+    LRS_HIP(set_step(m, token, pos));
     LRS_HIP(run_forward(m, true));
-    LRS_HIP(hipMemcpyAsync(m->step_host + 4, m->step, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    LRS_HIP(ao_err_fetch(m, s));
+    LRS_HIP(publish(m, m->step, m->words_host, 1));
     LRS_HIP(hipStreamSynchronize(s));
     if (int e = ao_err_check(m)) return e;
-    *next = m->step_host[4];
+    *next = m->words_host[0];
     m->len = pos + 1;
     return LRS_OK;
 }
@@ -1637,15 +1645,10 @@ int lrs_generate_greedy(lrs_model *m, const uint32_t *prompt, uint32_t n_prompt,
     } else if (n_prompt > 1 && (rc = enqueue_tokens(m, prompt, n_prompt - 1, pos0))) {
         return rc;
     }
-    LRS_HIP(hipStreamSynchronize(s));
-    m->step_host[0] = prompt[n_prompt - 1];
-    m->step_host[1] = pos0 + n_prompt - 1;
-    m->step_host[2] = 0;
-    LRS_HIP(hipMemcpyAsync(m->step, m->step_host, 3 * sizeof(uint32_t), hipMemcpyHostToDevice, s));
+    LRS_HIP(set_step(m, prompt[n_prompt - 1], pos0 + n_prompt - 1));
     for (uint32_t i = 0; i < n_gen; i++) LRS_HIP(run_forward(m, true));
     // through the pinned buffer: the caller's memory is pageable
-    LRS_HIP(hipMemcpyAsync(m->gen_host, m->gen, n_gen * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    LRS_HIP(ao_err_fetch(m, s));
+    LRS_HIP(publish(m, m->gen, m->gen_host, n_gen));
     LRS_HIP(hipStreamSynchronize(s));
     if (int e = ao_err_check(m)) return e;
     memcpy(out_tokens, m->gen_host, n_gen * sizeof(uint32_t));
@@ -1738,10 +1741,7 @@ int lrs_model_profile(lrs_model *m, uint32_t op, uint32_t iters, float *avg_us, 
         b = wbytes(m->output) + 2 * E4 + (size_t)c.vocab * 4;
     }
     // the step buffer must hold a valid position: the last decoded one
-    m->step_host[0] = 0;
-    m->step_host[1] = L - 1;
-    m->step_host[2] = 0;
-    LRS_HIP(hipMemcpyAsync(m->step, m->step_host, 3 * sizeof(uint32_t), hipMemcpyHostToDevice, s));
+    LRS_HIP(set_step(m, 0, L - 1));
     auto one = [&](uint32_t i) -> hipError_t {
         const uint32_t l = ls[i % ls.size()];
         switch (op) {
@@ -1766,7 +1766,7 @@ int lrs_model_profile(lrs_model *m, uint32_t op, uint32_t iters, float *avg_us, 
     LRS_HIP(hipEventRecord(m->ctx->ev0, s));
     for (uint32_t i = 0; i < iters; i++) LRS_HIP(one(i));
     LRS_HIP(hipEventRecord(m->ctx->ev1, s));
-    LRS_HIP(ao_err_fetch(m, s));
+    LRS_HIP(publish(m, m->step, m->words_host, 1));  // for the wait-error word
     LRS_HIP(hipEventSynchronize(m->ctx->ev1));
     LRS_HIP(hipStreamSynchronize(s));
     if (int e = ao_err_check(m)) return e;
