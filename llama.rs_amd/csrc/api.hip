@@ -68,6 +68,7 @@ using namespace lrs;
 struct lrs_ctx_scratch {
     void *p = nullptr;
     size_t n = 0;
+    void *host = nullptr;  // pinned, HOST_STAGE bytes once a host-buffer call asked for it
 };
 static std::mutex g_scratch_mu;
 static std::unordered_map<lrs_ctx *, lrs_ctx_scratch> g_scratch;
@@ -118,6 +119,20 @@ static void *ctx_scratch_or_null(lrs_ctx *ctx, size_t bytes) {
     if (ctx_scratch(ctx, bytes, &p) == LRS_OK) return p;
     (void)hipGetLastError();  // the caller's launches must not report it
     return nullptr;
+}
+// pinned memory for the vectors of a host-buffer call, null where there is none
+// (a capture, an allocation that failed)
+static constexpr size_t HOST_STAGE = 512u << 10;
+static void *ctx_host_stage(lrs_ctx *ctx) {
+    std::lock_guard<std::mutex> lk(g_scratch_mu);
+    lrs_ctx_scratch &s = g_scratch[ctx];
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return nullptr;
+    if (!s.host && hipHostMalloc(&s.host, HOST_STAGE, hipHostMallocDefault) != hipSuccess) {
+        s.host = nullptr;
+        (void)hipGetLastError();
+    }
+    return s.host;
 }
 }  // namespace lrs
 
@@ -212,6 +227,7 @@ void lrs_ctx_destroy(lrs_ctx *ctx) {
         auto it = g_scratch.find(ctx);
         if (it != g_scratch.end()) {
             if (it->second.p) (void)hipFree(it->second.p);
+            if (it->second.host) (void)hipHostFree(it->second.host);
             g_scratch.erase(it);
         }
     }
@@ -435,6 +451,23 @@ int lrs_matvec_f32(lrs_ctx *ctx, const lrs_weight *w, const float *x, float *y, 
     float *xd = (float *)buf;
     float *yd = (float *)((char *)buf + up(xb));
     void *pack = pb ? (char *)buf + up(xb) + up(yb) : nullptr;
+    // Vectors of up to HOST_STAGE bytes go through pinned memory that the
+    // kernels read and write themselves: a copy of pageable memory costs 10 us
+    // and more each way whatever its size.  The pack launch reads x once; where
+    // the workgroups pack, each of them reads all of x, so a launch brings it
+    // into device memory.  Every output is written once.  us per call, copies ->
+    // this: Q6_K 1024 x 5120 38 -> 23, Q4_K 100000 x 5120 92 -> 77 (400 KB out),
+    // Q8_0 4096 x 4096 at 8 columns 61 -> 37 (with the launch that packs them).
+    char *const hx = up(xb) + yb <= HOST_STAGE ? (char *)ctx_host_stage(ctx) : nullptr;
+    if (hx) {
+        float *const hy = (float *)(hx + up(xb));
+        memcpy(hx, x, xb);
+        if (!pack) LRS_HIP(launch_copy_words(hx, xb / 4, xd, ctx->stream));
+        LRS_HIP(launch_matvec(w->v, pack ? (const float *)hx : xd, hy, cols, pack, ctx->stream, cpack));
+        LRS_HIP(hipStreamSynchronize(ctx->stream));
+        memcpy(y, hy, yb);
+        return LRS_OK;
+    }
     LRS_HIP(hipMemcpyAsync(xd, x, xb, hipMemcpyHostToDevice, ctx->stream));
     LRS_HIP(launch_matvec(w->v, xd, yd, cols, pack, ctx->stream, cpack));
     LRS_HIP(hipMemcpyAsync(y, yd, yb, hipMemcpyDeviceToHost, ctx->stream));

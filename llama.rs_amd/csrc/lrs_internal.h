@@ -126,6 +126,8 @@ hipError_t launch_argmax_finish(const unsigned long long *keys, uint32_t n, uint
 hipError_t launch_matvec(WeightView w, const float *x, float *y, uint32_t cols, void *pack,
                          hipStream_t s, void *cols_pack = nullptr);
 size_t matvec_cols_bytes(WeightView w, uint32_t cols);
+// n words from (pinned host) src, 16-byte aligned as dst
+hipError_t launch_copy_words(const void *src, size_t n, void *dst, hipStream_t s);
 bool matvec_packs_in_kernel(WeightView w, uint32_t cols);
 // the staged form: each column packed into `pack` by its own launch, then one
 // matvec launch per column over that pack (same results)

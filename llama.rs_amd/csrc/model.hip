@@ -1249,10 +1249,6 @@ static int check_step(lrs_model *m, uint32_t token, uint32_t pos) {
 }
 
 // ---- batched prompt blocks on the matrix cores --------------------------
-__global__ void k_words(const uint32_t *host, uint32_t n, uint32_t *dst) {
-    if (threadIdx.x < n) dst[threadIdx.x] = host[threadIdx.x];
-}
-
 // every matmul weight has a GEMM kernel and the attention shape is supported
 static bool prefill_capable(const lrs_model *m) {
     // with the reference's Q8_0 input rounding on, Q8_0 weights stay on the
@@ -1422,8 +1418,7 @@ static int prefill_block(lrs_model *m, const uint32_t *tokens, uint32_t nb, uint
     // the token ids through pinned memory, read by a launch (the rows' launch
     // would read each of them many times)
     memcpy(m->words_host, tokens, nb * sizeof(uint32_t));
-    hipLaunchKernelGGL(k_words, dim3(1), dim3(PREFILL_BLOCK), 0, s, m->words_host, nb, m->ptok);
-    LRS_HIP(hipGetLastError());
+    LRS_HIP(launch_copy_words(m->words_host, nb, m->ptok, s));
     LRS_HIP(launch_dequant_rows(m->embd->v, m->ptok, nb, m->pX, s));
     for (uint32_t l = 0; l < c.n_layer; l++) {
         const DevLayer &L = m->layers[l];

@@ -109,6 +109,21 @@ __global__ __launch_bounds__(256) void k_xpack_cols(const float *__restrict__ x,
     pack_half(e < n ? x[(size_t)c * n + e] : 0.f, e >> 5, p);
 }
 
+__global__ __launch_bounds__(256) void k_copy_words(const uint32_t *__restrict__ src, uint32_t n,
+                                                    uint32_t *__restrict__ dst) {
+    const uint32_t i = 4 * (blockIdx.x * 256 + threadIdx.x);
+    if (i + 4 <= n)
+        *reinterpret_cast<uint4 *>(dst + i) = *reinterpret_cast<const uint4 *>(src + i);
+    else
+        for (uint32_t k = i; k < n; k++) dst[k] = src[k];
+}
+
+hipError_t launch_copy_words(const void *src, size_t n, void *dst, hipStream_t s) {
+    hipLaunchKernelGGL(k_copy_words, dim3((unsigned)((n + 1023) / 1024)), dim3(256), 0, s, (const uint32_t *)src,
+                       (uint32_t)n, (uint32_t *)dst);
+    return hipGetLastError();
+}
+
 hipError_t launch_xpack(const float *x, const float *nw, uint32_t n, uint32_t nxb, XPack p,
                         hipStream_t s, float *xsq) {
     const uint32_t threads = 32 * nxb;

@@ -524,3 +524,26 @@ def test_matvec_columns_where_the_scratch_may_not_grow(lrs, orc):
         c.sync()
         assert np.array_equal(yb.download(np.float32, cols * n_out), eager)
         assert np.array_equal(np.stack([w.matvec(v) for v in x]).ravel(), eager)
+
+
+# vectors through pinned memory up to 512 KiB together, copied beyond; packed by
+# the workgroups (256, Q8_0), by a launch that reads the host vector (5120), or
+# as several columns
+@pytest.mark.parametrize("t,n_in,n_out,cols", [(Q4_K, 256, 130816, 1), (Q4_K, 256, 130817, 1), (Q6_K, 5120, 33, 1),
+                                               (Q8_0, 2080, 17, 1), (Q5_K, 5120, 40, 5), (Q4_K, 1024, 3, 130)])
+def test_matvec_of_host_vectors_equals_the_device_call(lrs, orc, t, n_in, n_out, cols):
+    """The same bits as lrs_matvec_dev, also from the second call on (the
+    pinned memory holds the first one's values) and from unaligned vectors."""
+    with lrs.Context(0) as c:
+        w = lrs.Weight.upload(c, t, orc.gen_weight(t, 5, n_out, n_in, mode=1), n_in, n_out)
+        xb, yb = c.alloc(4 * cols * n_in), c.alloc(4 * cols * n_out)
+        for seed in (1, 2):
+            x = np.random.default_rng(seed).standard_normal(cols * n_in + 1).astype(np.float32)
+            for v in (x[:-1], x[1:]):
+                xb.upload(np.ascontiguousarray(v))
+                w.matvec_dev(xb, yb, cols)
+                c.sync()
+                y = np.full(cols * n_out + 1, 7.0, np.float32)
+                lrs.check(lrs.lib.lrs_matvec_f32(c.h, w.h, v.ctypes.data, y.ctypes.data, cols))
+                assert np.array_equal(y[:-1], yb.download(np.float32, cols * n_out))
+                assert y[-1] == 7.0
