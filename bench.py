@@ -28,10 +28,11 @@ Workloads:
           and the prompt replayed before the timed tokens).
   prefill config 5 through the full model: a prompt of M tokens (--m: 128 /
           512 / 2048) consumed by the 32B-shaped model of config 3 in blocks of
-          512 tokens (bf16 hi/lo matrix-core GEMMs for every projection,
+          512 tokens (f32-grade matrix-core GEMMs for every projection,
           batched norm / RoPE / causal attention); a step is one whole prompt.
           Reports prompt tok/s and the algorithmic matmul TFLOP/s (2 x M x
-          weight elements; the hi/lo split issues three bf16 products each).
+          weight elements; the f16 hi/lo activations take two products each,
+          three with Q6_K).
   pmc     profiling helper for the rocprofv3 counter passes: a plain copy
           kernel of known size (calibration) and the dominant decode kernel
           on a 4-layer model of the 32B shape.
@@ -868,7 +869,7 @@ def line_gemm(lrs, ctx, a, threads, m, precision):
     return {"metric": "prefill dequant-GEMM TFLOP/s (config 5 FFN set, MFMA)",
             **common(a, round(r["tflops"], 2), "TFLOP/s", round(r["us"] / 1e3, 5)),
             "dtype": "bf16 operands, f32 accumulate" if precision == 1 else
-                     "bf16 hi/lo split operands (3 products), f32 accumulate",
+                     "f16 whole-number weights x f16 hi/lo activations (2 products, Q6_K 3), f32 accumulate",
             "data": "synthetic (seeded GGUF blocks, x ~ N(0,1))",
             "config": {"workload": "config5-prefill-gemm-ffn", "m": m,
                        "weights": "gate/up Q4_K 13824x5120, down Q6_K 5120x13824",
@@ -885,7 +886,7 @@ def prefill_line(a, m_tok, r):
     peak = 2500.0  # MI355X dense bf16 MFMA
     return {"metric": "prefill tok/s through the 32B-shaped Q4_K_M model (config 5)",
             **common(a, round(r["tok_s"], 1), "tok/s", round(r["s"] * 1e3, 3)),
-            "dtype": "bf16 hi/lo split operands (3 products), f32 accumulate",
+            "dtype": "f16 whole-number weights x f16 hi/lo activations (2 products, Q6_K 3), f32 accumulate",
             "data": "synthetic (random-init Q4_K_M GGUF blocks generated on the GPU; "
                     "prompt ids uniform random, seed 4321)",
             "config": {"workload": "config5-prefill-32b-model", "m": m_tok,
@@ -984,7 +985,7 @@ def main():
     ap.add_argument("--m", type=int, default=512,
                     help="gemm / prefill: prompt tokens (config 5: 128/512/2048)")
     ap.add_argument("--precision", type=int, default=1, choices=[1, 3],
-                    help="gemm: 1 = bf16 operands, 3 = bf16 hi/lo split")
+                    help="gemm: 1 = bf16 operands, 3 = f32 grade, f16 hi/lo activations")
     ap.add_argument("--no-cpu", action="store_true", help="skip the CPU baselines")
     ap.add_argument("--no-sub", action="store_true",
                     help="decode: skip the labelled lines of configs 1, 2, 4 and 5")

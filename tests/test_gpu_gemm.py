@@ -3,9 +3,8 @@ CPU oracle's dequant (bit-exact dequant.rs restatement) and float64 products.
 
 precision 1 (bf16 operands, f32 accumulation) is checked
 against the exact product of the same bf16-rounded operands (tolerance 1e-5
-relative L2: only the f32 summation order differs); precision 3 (bf16 hi/lo
-split) against the f32 operands themselves (tolerance 1e-4, the north-star
-GEMM bar).
+relative L2: only the f32 summation order differs); precision 3 (f16 hi/lo
+activations) against the f32 operands themselves (tolerance 1e-4).
 """
 import numpy as np
 import pytest
@@ -57,7 +56,7 @@ def test_gemm_matches_oracle(lrs, orc, ctx, t, m, n, k):
 
 def test_gemm_row_of_one_hot_activations_is_a_weight_column(lrs, orc, ctx):
     """a = identity rows: y[i] = column i of W (exact for values that bf16
-    represents, which the hi/lo split reaches to 2^-16)."""
+    represents, which the hi/lo activations reach to 2^-22)."""
     k, n = 256, 64
     w = orc.gen_weight(Q4_K, 5, n, k, mode=1)
     deq = orc.dequant(Q4_K, w).reshape(n, k)

@@ -174,7 +174,7 @@ def test_q8_0_rounding_mode_follows_the_reference_int8_path(lrs, orc, ctx, name,
 
 def test_decode_batch_matches_token_loop_and_reset_is_deterministic(lrs, orc, ctx):
     """decode_batch runs the prompt through the matrix-core GEMMs (operands
-    split into bf16 hi + lo) instead of the matvecs.  The two differ by f32
+    split into f16 hi + lo) instead of the matvecs.  The two differ by f32
     summation order, which the f16 K/V cache turns into an occasional 1-ulp
     f16 difference (2^-11 relative): both stay within the oracle bar, with the
     same argmax."""
