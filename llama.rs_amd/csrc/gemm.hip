@@ -810,7 +810,7 @@ hipError_t launch_gemm_segs(const WeightView *w, float *const *y, const uint32_t
     const uint32_t grid = 8 * ((g.nm * g.nn * g.ks + 7) / 8);
     hipLaunchKernelGGL(fn, dim3(grid), dim3(64 * PG_WAVES), 0, s, g);
     if (ks_out) {
-        *ks_out = g.ks;  // the caller reduces the slices (launch_reduce_norm_rows)
+        *ks_out = g.ks;  // the caller reduces the slices (launch_norm_rows)
     } else if (g.ks > 1) {
         if (v4)
             hipLaunchKernelGGL((k_reduce_ks<4>), dim3((nmax + 1023) / 1024, M, nseg), dim3(256), 0, s, g);

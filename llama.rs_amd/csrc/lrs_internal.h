@@ -160,16 +160,11 @@ hipError_t launch_gemm_segs(const WeightView *w, float *const *y, const uint32_t
                             const uint8_t *planes, uint32_t M, int prec, hipStream_t s, bool accum = false,
                             float *work = nullptr, size_t work_bytes = 0, uint32_t *ks_out = nullptr);
 // batched prompt block (prefill.hip)
-// RMSNorm rows of X times w as a GEMM input of precision 3 (planes), and in
-// f32 when Y is given; E a multiple of 256
-hipError_t launch_rmsnorm_rows(const float *X, const float *w, float eps, uint32_t E, uint32_t n,
-                               float *Y, uint8_t *planes, hipStream_t s);
-// X += the ks K-slice partials part[z][n][E] (slices in order, as
-// k_reduce_ks), then the RMSNorm rows of the new X times w as
-// launch_rmsnorm_rows writes them
-hipError_t launch_reduce_norm_rows(const float *part, uint32_t ks, float *X, const float *w,
-                                   float eps, uint32_t E, uint32_t n, float *Y, uint8_t *planes,
-                                   hipStream_t s);
+// X += the ks K-slice partials part[z][n][E] (slices in order, as k_reduce_ks;
+// ks 0: none), then the RMSNorm rows of X times w as a GEMM input of precision 3
+// (planes), and in f32 when Y is given; E a multiple of 256
+hipError_t launch_norm_rows(const float *part, uint32_t ks, float *X, const float *w, float eps, uint32_t E,
+                            uint32_t n, float *Y, uint8_t *planes, hipStream_t s);
 hipError_t launch_qkv_post(const float *qt, const float *kt, const float *vt, const float *bq,
                            const float *bk, const float *bv, const float *freq, float *q,
                            _Float16 *kc, _Float16 *vc, uint32_t n, uint32_t pos0, uint32_t qd,

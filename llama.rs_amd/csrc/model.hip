@@ -1382,15 +1382,12 @@ static int prefill_block(lrs_model *m, const uint32_t *tokens, uint32_t nb, uint
     // pX += A W^T (o, down, the delta net's out-projection), then the
     // RMSNorm rows of pX times nw as the next GEMM input (and in f32 into
     // xn): when the GEMM splits over K, its slices' reduce and the norm run
-    // as one kernel of a workgroup per row.  Few rows are too few workgroups
-    // for the many slices they have (19 rows of 22 slices: 29 us, against
-    // 5 + 4 us as a reduce over all outputs and a norm)
+    // as one kernel of a workgroup per row
     auto gemm_resid_norm = [&](const lrs_weight *w, const float *nw, float *xn) -> hipError_t {
         uint32_t ks = 1;
-        const hipError_t e = gemm(w, m->pX, true, nb >= 192 ? &ks : nullptr);
+        const hipError_t e = gemm(w, m->pX, true, &ks);
         if (e != hipSuccess) return e;
-        return ks > 1 ? launch_reduce_norm_rows(m->pWork, ks, m->pX, nw, c.rms_eps, E, nb, xn, A, s)
-                      : launch_rmsnorm_rows(m->pX, nw, c.rms_eps, E, nb, xn, A, s);
+        return launch_norm_rows(m->pWork, ks > 1 ? ks : 0, m->pX, nw, c.rms_eps, E, nb, xn, A, s);
     };
     // the normalised rows as a GEMM input, and in f32 for a delta-net block,
     // which reads them for its gates
@@ -1422,7 +1419,7 @@ static int prefill_block(lrs_model *m, const uint32_t *tokens, uint32_t nb, uint
     LRS_HIP(launch_dequant_rows(m->embd->v, m->ptok, nb, m->pX, s));
     for (uint32_t l = 0; l < c.n_layer; l++) {
         const DevLayer &L = m->layers[l];
-        if (!normed) LRS_HIP(launch_rmsnorm_rows(m->pX, L.attn_norm, c.rms_eps, E, nb, xn_for(L), A, s));
+        if (!normed) LRS_HIP(launch_norm_rows(nullptr, 0, m->pX, L.attn_norm, c.rms_eps, E, nb, xn_for(L), A, s));
         normed = false;
         if (m->hybrid) {
             if (L.dn) {

@@ -12,88 +12,78 @@
 
 namespace lrs {
 
-// (x * scale) * w of eight elements from element i, as a GEMM input and (Y) in f32
-__device__ __forceinline__ void norm_store8(const float *__restrict__ x, const float *__restrict__ w, float scale,
-                                            uint32_t i, uint32_t row, uint32_t E, float *__restrict__ Y,
-                                            uint8_t *__restrict__ planes) {
-    float v[8];
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-        const float4 a = *reinterpret_cast<const float4 *>(x + i + 4 * h);
-        const float4 g = *reinterpret_cast<const float4 *>(w + i + 4 * h);
-        v[4 * h] = (a.x * scale) * g.x;
-        v[4 * h + 1] = (a.y * scale) * g.y;
-        v[4 * h + 2] = (a.z * scale) * g.z;
-        v[4 * h + 3] = (a.w * scale) * g.w;
-        if (Y)
-            *reinterpret_cast<float4 *>(Y + (size_t)row * E + i + 4 * h) =
-                make_float4(v[4 * h], v[4 * h + 1], v[4 * h + 2], v[4 * h + 3]);
-    }
-    gp_store8<3>(v, row, i >> 3, E >> 8, planes);
-}
-
-// the row X[r] * scale_r * w, scale_r = 1 / sqrt(mean(X[r]^2) + eps), as a
-// GEMM input (gemm_pack.h) and, with Y, in f32
-__global__ __launch_bounds__(256) void k_rmsnorm_rows(const float *__restrict__ X,
-                                                      const float *__restrict__ w, float eps,
-                                                      uint32_t E, float *__restrict__ Y,
-                                                      uint8_t *__restrict__ planes) {
-    __shared__ float red[4];
-    const float *x = X + (size_t)blockIdx.x * E;
-    float ss = 0.f;
-    for (uint32_t i = 4 * threadIdx.x; i < E; i += 4 * blockDim.x) {
-        const float4 v = *reinterpret_cast<const float4 *>(x + i);
-        ss += (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w);
-    }
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) ss += __shfl_xor(ss, o, 64);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
-    __syncthreads();
-    const float tot = (red[0] + red[1]) + (red[2] + red[3]);
-    const float scale = 1.0f / sqrtf(tot / (float)E + eps);
-    for (uint32_t i = 8 * threadIdx.x; i < E; i += 8 * blockDim.x)
-        norm_store8(x, w, scale, i, blockIdx.x, E, Y, planes);
-}
-
-// X += the ks K-slice partials part[z][row][E] (summed in slice order, then
-// added to X, as k_reduce_ks does), then k_rmsnorm_rows over the new rows
-// (same sum-of-squares order, so the same scale): the residual add of a
-// K-split o / down GEMM and the norm after it in one pass over the rows
-__global__ __launch_bounds__(256) void k_reduce_norm_rows(const float *__restrict__ part,
-                                                          uint32_t ks, float *__restrict__ X,
-                                                          const float *__restrict__ w, float eps,
-                                                          uint32_t E, float *__restrict__ Y,
-                                                          uint8_t *__restrict__ planes) {
-    __shared__ float red[4];
+// X += the ks K-slice partials part[z][row][E] of a split o / down GEMM (summed
+// in slice order, then added to X, as k_reduce_ks does; ks 0: none), then the
+// row X[r] * scale_r * w, scale_r = 1 / sqrt(mean(X[r]^2) + eps), as a GEMM
+// input (gemm_pack.h) and, with Y, in f32.  Workgroup = a row.  Load latency
+// bounds it, so a thread has all of its eight elements' loads in flight (a
+// wider row takes more passes, whose elements are read back for the second
+// half).  us at E = 5120, 256 threads that went over the row four elements at a
+// time and read it back -> this: 512 rows norm alone 15.9 -> 11.0, with the
+// slices of o and down 20.3 -> 17.5; 19 rows of 11 to 22 slices 11.6 (a reduce
+// launch of its own and a norm) -> 7.6.
+__global__ __launch_bounds__(1024) void k_norm_rows(const float *__restrict__ part, uint32_t ks, float *X,
+                                                    const float *__restrict__ w, float eps, uint32_t E,
+                                                    float *__restrict__ Y, uint8_t *__restrict__ planes) {
+    __shared__ float red[16];
     const size_t plane = (size_t)gridDim.x * E, r0 = (size_t)blockIdx.x * E;
-    float *x = X + r0;
+    float *const x = X + r0;
+    const uint32_t i0 = 8 * threadIdx.x, step = 8 * blockDim.x;
+    float v0[8], g0[8];  // the first pass's elements and weights
+    auto load8 = [](const float *p, float (&v)[8]) __attribute__((always_inline)) {
+        const float4 a = *reinterpret_cast<const float4 *>(p), b = *reinterpret_cast<const float4 *>(p + 4);
+        v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
+    };
+    auto store8 = [](float *p, const float (&v)[8]) __attribute__((always_inline)) {
+        *reinterpret_cast<float4 *>(p) = make_float4(v[0], v[1], v[2], v[3]);
+        *reinterpret_cast<float4 *>(p + 4) = make_float4(v[4], v[5], v[6], v[7]);
+    };
+    if (i0 < E) load8(w + i0, g0);
     float ss = 0.f;
-    for (uint32_t i = 4 * threadIdx.x; i < E; i += 4 * blockDim.x) {
-        float4 p = *reinterpret_cast<const float4 *>(part + r0 + i);
-        for (uint32_t z = 1; z < ks; z++) {
-            const float4 q = *reinterpret_cast<const float4 *>(part + z * plane + r0 + i);
-            p.x += q.x;
-            p.y += q.y;
-            p.z += q.z;
-            p.w += q.w;
+    for (uint32_t i = i0; i < E; i += step) {
+        float v[8];
+        load8(x + i, v);
+        if (ks) {
+            float p[8];
+            load8(part + r0 + i, p);
+#pragma unroll 4
+            for (uint32_t z = 1; z < ks; z++) {
+                float q[8];
+                load8(part + z * plane + r0 + i, q);
+#pragma unroll
+                for (int k = 0; k < 8; k++) p[k] += q[k];
+            }
+#pragma unroll
+            for (int k = 0; k < 8; k++) v[k] += p[k];
+            store8(x + i, v);
         }
-        float4 v = *reinterpret_cast<const float4 *>(x + i);
-        v.x += p.x;
-        v.y += p.y;
-        v.z += p.z;
-        v.w += p.w;
-        *reinterpret_cast<float4 *>(x + i) = v;
-        ss += (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w);
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            ss = fmaf(v[k], v[k], ss);
+            if (i == i0) v0[k] = v[k];
+        }
     }
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) ss += __shfl_xor(ss, o, 64);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
     __syncthreads();
-    const float tot = (red[0] + red[1]) + (red[2] + red[3]);
+    float tot = 0.f;
+    for (uint32_t i = 0; i < blockDim.x / 64; i++) tot += red[i];
     const float scale = 1.0f / sqrtf(tot / (float)E + eps);
-    __syncthreads();  // the row's stores above are read back by other threads
-    for (uint32_t i = 8 * threadIdx.x; i < E; i += 8 * blockDim.x)
-        norm_store8(x, w, scale, i, blockIdx.x, E, Y, planes);
+    for (uint32_t i = i0; i < E; i += step) {
+        float v[8], g[8];
+        if (i == i0) {
+#pragma unroll
+            for (int k = 0; k < 8; k++) v[k] = v0[k], g[k] = g0[k];
+        } else {
+            load8(x + i, v);
+            load8(w + i, g);
+        }
+#pragma unroll
+        for (int k = 0; k < 8; k++) v[k] = (v[k] * scale) * g[k];
+        if (Y) store8(Y + r0 + i, v);
+        gp_store8<3>(v, blockIdx.x, i >> 3, E >> 8, planes);
+    }
 }
 
 // q/k/v GEMM outputs -> bias, adjacent-pair RoPE on q and k at position
@@ -465,18 +455,11 @@ __global__ __launch_bounds__(256) void k_attn_merge(const float *__restrict__ pa
     gp_store8<3>(v, row, c, qd >> 8, planes);
 }
 
-hipError_t launch_rmsnorm_rows(const float *X, const float *w, float eps, uint32_t E, uint32_t n,
-                               float *Y, uint8_t *planes, hipStream_t s) {
-    if (E % 256 || !planes) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_rmsnorm_rows, dim3(n), dim3(256), 0, s, X, w, eps, E, Y, planes);
-    return hipGetLastError();
-}
-
-hipError_t launch_reduce_norm_rows(const float *part, uint32_t ks, float *X, const float *w,
-                                   float eps, uint32_t E, uint32_t n, float *Y, uint8_t *planes,
-                                   hipStream_t s) {
-    if (E % 256 || ks == 0 || !planes) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_reduce_norm_rows, dim3(n), dim3(256), 0, s, part, ks, X, w, eps, E, Y, planes);
+hipError_t launch_norm_rows(const float *part, uint32_t ks, float *X, const float *w, float eps, uint32_t E,
+                            uint32_t n, float *Y, uint8_t *planes, hipStream_t s) {
+    if (E == 0 || E % 256 || !planes) return hipErrorInvalidValue;
+    const uint32_t threads = min(1024u, (E / 8 + 63) / 64 * 64);
+    hipLaunchKernelGGL(k_norm_rows, dim3(n), dim3(threads), 0, s, part, ks, X, w, eps, E, Y, planes);
     return hipGetLastError();
 }
 
