@@ -877,8 +877,7 @@ def line_gemm(lrs, ctx, a, threads, m, precision):
                        "op_us": {k: round(v["us"], 2) for k, v in r["per"].items()}},
             "roofline": {"bound": "mfma", "achieved": round(r["tflops"], 1), "peak": peak,
                          "unit": "TFLOP/s", "frac": round(r["tflops"] / peak, 4),
-                         "traffic": read_traffic("gemm_set") if (m, precision) == (512, 1)
-                         else None},
+                         "traffic": None},
             "cpu_baseline": None if a.no_cpu else cpu_baseline_gemm(threads, m)}
 
 
@@ -893,7 +892,9 @@ def prefill_line(a, m_tok, r):
                        "block": 512, "matmul_flop_per_prompt": r["flop"]},
             "roofline": {"bound": "mfma", "achieved": round(r["tflops"], 1), "peak": peak,
                          "unit": "TFLOP/s", "frac": round(r["tflops"] / peak, 4),
-                         "traffic": None, "mfma_work_per_flop": 3}}
+                         "traffic": None,
+                         # two products a weight, three for v and down (Q6_K: 30 % of them)
+                         "mfma_work_per_flop": 2.3}}
 
 
 STREAM_SIZES = {  # algorithmic bytes of the decode launches (config 3, then configs 1, 2, 4)
