@@ -693,23 +693,27 @@ static double pg_unit(int prec, uint32_t mt, uint32_t fit, uint32_t n) {
 // have_work: K slices may be used
 static PgPlan pg_plan(uint32_t M, const uint32_t *N, const uint32_t *type, uint32_t nseg, uint32_t nsb, int prec,
                       bool have_work) {
-    // precision 3: Q6_K and Q8_0 take a third product, Q5_K more unpacking.
+    // precision 3: Q6_K and Q8_0 take a third product, Q5_K more unpacking;
+    // precision 1: their unpacking shows where a workgroup has few row tiles.
     // While every workgroup runs at once the slowest counts, else the average
     uint32_t ntot = 0;
-    double slow = 1.0, mean = 0.0;
     bool wide = false;  // a type whose operands take more registers
     for (uint32_t i = 0; i < nseg; i++) {
-        const double rel = prec == 1 || type[i] == T_Q4_K ? 1.0 : type[i] == T_Q5_K ? 1.2 : 1.5;
-        slow = std::max(slow, rel);
-        mean += rel * N[i];
         ntot += N[i];
         wide = wide || type[i] == T_Q6_K || type[i] == T_Q5_K;
     }
-    mean /= ntot;
     PgPlan best = {1, 1};
     double best_cost = 1e30;
     for (uint32_t mt = 1; mt <= (prec == 3 ? 2u : 4u); mt *= 2) {
         if (mt > 1 && M <= 16 * mt) break;
+        double slow = 1.0, mean = 0.0;
+        for (uint32_t i = 0; i < nseg; i++) {
+            const double rel = type[i] == T_Q4_K ? 1.0
+                               : prec == 1       ? (mt == 4 ? 1.05 : 1.25)
+                                                 : type[i] == T_Q5_K ? 1.2 : 1.5;
+            slow = std::max(slow, rel);
+            mean += rel * N[i] / ntot;
+        }
         const uint32_t tiles = pg_tiles(M, N, nseg, mt);
         const uint32_t fit = mt == (prec == 3 ? 2u : 4u) || (wide && !(prec == 1 && mt == 1)) ? 2 : 3;
         for (uint32_t ks = 1; ks <= nsb && ks <= 32; ks++) {
