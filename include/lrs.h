@@ -161,8 +161,10 @@ int lrs_matvec_q8_0_actq_dev(lrs_ctx *ctx, const lrs_weight *w, const float *x_d
  * (crates/llama-vulkan/src/matmul.rs:433-465), which quantizes a to int8:
  * here both operands keep more bits, with f32 accumulation on the matrix cores.
  * precision 1: each operand rounded to bf16 once; precision 3: the weights as
- * exact f16 whole numbers and the activations as f16 hi + lo (22 bits), for
- * prefill that must match the f32 forward (observed 2e-7 to 5e-7 relative L2).
+ * exact f16 whole numbers and the activations as f16 hi + lo, for prefill that
+ * must match the f32 forward (observed 2e-7 to 5e-7 relative L2).  An
+ * activation has 22 bits down to 2^-17 of the largest of its 256 columns and an
+ * absolute 2^-40 of that largest below.
  * Weights: Q4_K, Q5_K, Q6_K, Q8_0; n_in a multiple of 256. */
 int lrs_gemm_dev(lrs_ctx *ctx, const lrs_weight *w, const float *a_dev, float *y_dev, uint32_t m,
                  int precision);

@@ -1,5 +1,5 @@
 // Input layout of the prompt GEMM (gemm.hip), written by the kernels that
-// produce its rows (prefill.hip, dn.hip) or by launch_gemm_pack.
+// produce its rows (prefill.hip) or by launch_gemm_pack.
 //
 // The rows come in tiles of 32 and the row length K in super-blocks of 256.
 // The bytes of one (row tile, super-block) are contiguous and in the order in
@@ -11,10 +11,16 @@
 // of row m: the order in which the weights' nibbles unpack two at a time from
 // 32-bit words (elements i and i + 2 of a word's four bytes sit 16 bits apart).
 //   precision 3: per K-step 1 KB of f16 hi, then 1 KB of f16 lo (hi + lo = 22
-//     bits of x * 2^-e, |x * 2^-e| < 1024 with e the super-block's own), after
-//     the 16 steps 1 KB of sub-block sums (lane m: the f16 hi of the eight
-//     32-element sums of row m, lane m + 32: their lo) for the K-quant minima,
-//     then the 32 rows' 2^e in f32 (padded to 1 KB)
+//     bits of x * 2^-e, or 2^-25 in absolute terms where that is coarser; e the
+//     super-block's own), after the 16 steps 1 KB of sub-block sums (lane m: the
+//     f16 hi of the eight 32-element sums of row m, lane m + 32: their lo) for
+//     the K-quant minima, then the 32 rows' 2^e in f32 (padded to 1 KB).
+//     e is the least for which every element and every sub-block sum is below
+//     2^15 times 2^e: an element keeps its 22 bits down to 2^-17 of the largest
+//     of its super-block, 16 bits (a bf16 hi + lo pair's) down to 2^-21, and an
+//     absolute 2^-40 of the largest below.  (With e fixed by 32 times the largest
+//     element, which no sum can exceed, it was 2^-35: beside one element of 2^20
+//     the error of N(0, 1) elements was 3.5e-5, now 1.1e-6; bf16 pairs have 2.5e-6.)
 //   precision 1: per K-step 1 KB of bf16
 #pragma once
 
@@ -45,30 +51,30 @@ __device__ __forceinline__ void gp_store8(const float (&v)[8], uint32_t row, uin
         *reinterpret_cast<bf16x8_p *>(b + 1024 * t + lane16) = h;
     } else {
         typedef __attribute__((ext_vector_type(8))) _Float16 f16x8_p;
-        float mx = 0.f;
+        // sub-block sums (four lanes) of x / 32, which the largest |x| bounds
+        float mx = 0.f, s = 0.f;
 #pragma unroll
-        for (int i = 0; i < 8; i++) mx = fmaxf(mx, fabsf(v[i]));
+        for (int i = 0; i < 8; i++) mx = fmaxf(mx, fabsf(v[i])), s += v[i] * 0.03125f;
+        s += __shfl_xor(s, 1, 64);
+        s += __shfl_xor(s, 2, 64);
+        mx = fmaxf(mx * 0.03125f, fabsf(s));
 #pragma unroll
         for (int o = 16; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
         int ex;
-        (void)frexpf(mx, &ex);  // mx < 2^ex
+        (void)frexpf(mx, &ex);  // mx < 2^ex: elements and sums below 2^(ex + 5)
         ex = mx > 0.f ? (ex < -100 ? -100 : ex) : 0;
         f16x8_p h, l;
-        float s = 0.f;
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             const float x = ldexpf(v[i], 10 - ex);
             const _Float16 xh = (_Float16)x;
             h[gp_slot(i)] = xh;
             l[gp_slot(i)] = (_Float16)(x - (float)xh);
-            s += x;
         }
         *reinterpret_cast<f16x8_p *>(b + 2048 * t + lane16) = h;
         *reinterpret_cast<f16x8_p *>(b + 2048 * t + 1024 + lane16) = l;
-        // the 32-element sub-block's sum: four lanes
-        s += __shfl_xor(s, 1, 64);
-        s += __shfl_xor(s, 2, 64);
         if ((c8 & 3) == 0) {
+            s = ldexpf(s, 15 - ex);
             const _Float16 sh = (_Float16)s;
             _Float16 *sp = reinterpret_cast<_Float16 *>(b + GP_SUMS + 16 * (row & 31)) + gp_slot(c8 >> 2);
             sp[0] = sh;

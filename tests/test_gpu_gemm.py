@@ -170,6 +170,65 @@ def test_gemm_edges_and_extreme_blocks(lrs, orc, ctx, t, m, n, k):
         assert np.linalg.norm(y1[r] - ref1[r]) <= 1e-5 * size
 
 
+def zero_column_5(t, w):
+    """Quantizer-like blocks whose weight 5 of every 256 is zero: beside an
+    activation of any size there, the others' contributions show."""
+    bb = {Q8_0: 34 * 8, Q4_K: 144, Q5_K: 176, Q6_K: 210}[t]
+    b = w.reshape(-1, bb).copy()
+    if t == Q8_0:
+        b[:, 2 + 5] = 0
+    elif t == Q6_K:
+        b[:, 5] &= 0xF0
+        b[:, 128 + 5] = (b[:, 128 + 5] & 0xFC) | 2
+    else:
+        b[:, 8] &= 0xC0  # the first sub-block's minimum
+        b[:, {Q4_K: 16, Q5_K: 48}[t] + 5] &= 0xF0
+        if t == Q5_K:
+            b[:, 16 + 5] &= 0xFE
+    return b.reshape(-1)
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q5_K, Q6_K, Q8_0])
+def test_gemm_activations_beside_a_large_one(lrs, orc, ctx, t):
+    """One activation of 2^20 in every 256 (of either sign, its weights zero):
+    the rest keep what a bf16 hi + lo pair would (2^-17 of themselves).  An
+    element's error is at most 2^-40 of the largest's next power of two, 2^-19;
+    the f32 sums add 2^-22 of the terms."""
+    m, n, k = 33, 48, 768
+    w = zero_column_5(t, quantizer_like(t, n, k, 3))
+    deq = orc.dequant(t, w).reshape(n, k).astype(np.float64)
+    assert not deq[:, 5::256].any()
+    rng = np.random.default_rng(8)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    a[:, 5::256] = np.float32(2.0 ** 20) * rng.choice([-1, 1], (m, k // 256))
+    y = lrs.Weight.upload(ctx, t, w, k, n).gemm(a, precision=3)
+    a[:, 5::256] = 0
+    ref = a.astype(np.float64) @ deq.T
+    # independent roundings: their 2-norm, eight times (a K-quant's two terms,
+    # scale times quant and the minimum, are each up to about twice the weight)
+    tol = 8 * 2.0 ** -19 / np.sqrt(3) * np.linalg.norm(deq, axis=1) + 2.0 ** -22 * (np.abs(a) @ np.abs(deq).T)
+    assert np.all(np.abs(y - ref) <= tol)
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q5_K, Q6_K, Q8_0])
+def test_gemm_super_blocks_of_different_size(lrs, orc, ctx, t):
+    """Inside a row, 256-column blocks scaled by 2^20 and 2^-20 in turn: the
+    small blocks alone (the others zero) as exact as any, and their scale taken
+    into a sum with the large ones."""
+    m, n, k = 5, 40, 1024
+    w = quantizer_like(t, n, k, 4)
+    deq = orc.dequant(t, w).reshape(n, k).astype(np.float64)
+    a = np.random.default_rng(9).standard_normal((m, k)).astype(np.float32)
+    s = np.repeat([2.0 ** 20, 2.0 ** -20, 2.0 ** 20, 2.0 ** -20], 256).astype(np.float32)
+    W = lrs.Weight.upload(ctx, t, w, k, n)
+    for keep in (s > 1, s < 1, s > 0):
+        x = a * s * keep
+        ref = x.astype(np.float64) @ deq.T
+        y = W.gemm(x, precision=3)
+        size = np.linalg.norm(np.abs(x.astype(np.float64)) @ np.abs(deq).T)
+        assert np.linalg.norm(y - ref) <= 2e-6 * size
+
+
 @pytest.mark.parametrize("t", [Q8_0, Q4_K, Q5_K, Q6_K])
 @pytest.mark.parametrize("n,k,shift", [(1, 256, 0), (17, 768, 0), (5, 512, 1)])
 def test_dequant_into_any_float_address_is_exact(lrs, orc, ctx, t, n, k, shift):
