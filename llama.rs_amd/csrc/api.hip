@@ -1,4 +1,5 @@
 // api.hip — the extern "C" boundary of liblrs.so (declared in include/lrs.h).
+#include "gemm_plan.h"
 #include "lrs_internal.h"
 
 #include <cstdio>

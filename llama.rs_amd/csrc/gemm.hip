@@ -38,9 +38,8 @@
 // gate / up launch, whose 1.1 PFLOP/s of products compare with 1.27 (bf16) and
 // 1.37 (f16) of a large library product.
 #include "gemm_pack.h"
+#include "gemm_plan.h"
 #include "quant_dev.h"
-
-#include <algorithm>
 
 namespace lrs {
 
@@ -53,7 +52,6 @@ typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
 typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
 typedef __attribute__((address_space(3))) void lds_void;
 
-constexpr int PG_WAVES = 4;
 constexpr int PG_MAX_SEG = 3;
 struct PgSeg {
     const uint8_t *q;  // weight, tiled layout (tiled.h)
@@ -662,88 +660,6 @@ hipError_t launch_gemm_pack(const float *a, uint32_t M, uint32_t K, int prec, ui
 
 size_t gemm_planes_bytes(uint32_t M, uint32_t K, int prec) {
     return (size_t)((M + 31) / 32) * (K / 256) * gemm_block_bytes(prec);
-}
-
-constexpr uint32_t PG_ROWS = 64 * PG_WAVES;  // weight rows of a workgroup
-
-// Launch shape of a GEMM: row tiles of 32 tokens per workgroup, K slices.
-struct PgPlan {
-    uint32_t mt, ks;
-};
-
-static uint32_t pg_tiles(uint32_t M, const uint32_t *N, uint32_t nseg, uint32_t mt) {
-    uint32_t nn = 0;
-    for (uint32_t i = 0; i < nseg; i++) nn += (N[i] + PG_ROWS - 1) / PG_ROWS;
-    return (M + 32 * mt - 1) / (32 * mt) * nn;
-}
-
-// us per super-block of n workgroups that share a CU, measured with Q4_K
-// weights at K = 5120: the first workgroups of a CU hide each other's waits.
-// `fit`: workgroups that fit a CU at once (by registers)
-static double pg_unit(int prec, uint32_t mt, uint32_t fit, uint32_t n) {
-    static const double p3m1[3] = {2.5, 4.4, 6.6}, p3m2[2] = {3.6, 6.4};
-    static const double p1m1[3] = {2.0, 3.0, 4.2}, p1m2[3] = {2.7, 4.8, 6.4}, p1m4[2] = {4.4, 7.8};
-    const double *c = prec == 3 ? (mt == 1 ? p3m1 : p3m2) : mt == 1 ? p1m1 : mt == 2 ? p1m2 : p1m4;
-    return n / fit * c[fit - 1] + (n % fit ? c[n % fit - 1] : 0.0);
-}
-
-// The shape with the least expected time: the workgroups that a CU gets, and
-// for K slices the partial sums written and read back (at about 7 TB/s, most
-// of them in the memory-side cache) and the launch that adds them.
-// have_work: K slices may be used
-static PgPlan pg_plan(uint32_t M, const uint32_t *N, const uint32_t *type, uint32_t nseg, uint32_t nsb, int prec,
-                      bool have_work) {
-    // precision 3: Q6_K and Q8_0 take a third product, Q5_K more unpacking;
-    // precision 1: their unpacking shows where a workgroup has few row tiles.
-    // While every workgroup runs at once the slowest counts, else the average
-    uint32_t ntot = 0;
-    bool wide = false;  // a type whose operands take more registers
-    for (uint32_t i = 0; i < nseg; i++) {
-        ntot += N[i];
-        wide = wide || type[i] == T_Q6_K || type[i] == T_Q5_K;
-    }
-    PgPlan best = {1, 1};
-    double best_cost = 1e30;
-    for (uint32_t mt = 1; mt <= (prec == 3 ? 2u : 4u); mt *= 2) {
-        if (mt > 1 && M <= 16 * mt) break;
-        double slow = 1.0, mean = 0.0;
-        for (uint32_t i = 0; i < nseg; i++) {
-            const double rel = type[i] == T_Q4_K ? 1.0
-                               : prec == 1       ? (mt == 4 ? 1.05 : 1.25)
-                                                 : type[i] == T_Q5_K ? 1.2 : 1.5;
-            slow = std::max(slow, rel);
-            mean += rel * N[i] / ntot;
-        }
-        const uint32_t tiles = pg_tiles(M, N, nseg, mt);
-        const uint32_t fit = mt == (prec == 3 ? 2u : 4u) || (wide && !(prec == 1 && mt == 1)) ? 2 : 3;
-        for (uint32_t ks = 1; ks <= nsb && ks <= 32; ks++) {
-            if (ks > 1 && (!have_work || tiles >= 2048 || M > 65535)) break;  // the reduce's grid has a y row per token
-            const uint32_t len = (nsb + ks - 1) / ks, per = (tiles * ks + 255) / 256;
-            const double rel = per < fit ? slow : per == fit ? 0.5 * (slow + mean) : mean;
-            double cost = (len + 0.5) * rel * pg_unit(prec, mt, fit, per);
-            if (ks > 1) cost += 5.0 + (2.0 * ks + 1) * M * ntot * 4.0 / 7e6;
-            if (cost < best_cost * 0.98) {
-                best_cost = cost;
-                best = {mt, ks};
-            }
-        }
-    }
-    return best;
-}
-
-// scratch of the K-sliced form for any row count up to M (a smaller one may
-// split over more slices): a caller that made its largest call first never
-// needs more
-size_t gemm_work_bytes(uint32_t M, const uint32_t *N, const uint32_t *type, uint32_t nseg, uint32_t K, int prec) {
-    uint32_t ntot = 0;
-    for (uint32_t i = 0; i < nseg; i++) ntot += N[i];
-    size_t most = 0;
-    for (uint32_t m = M;; m = (m - 1) / 32 * 32) {
-        const uint32_t ks = pg_plan(m, N, type, nseg, K / 256, prec, true).ks;
-        if (ks > 1) most = std::max(most, (size_t)ks * m * ntot * sizeof(float));
-        if (m <= 32) break;
-    }
-    return most;
 }
 
 using GemmFn = void (*)(PgArgs);

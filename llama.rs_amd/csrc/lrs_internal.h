@@ -151,11 +151,10 @@ size_t gemm_planes_bytes(uint32_t M, uint32_t K, int prec);
 // one launch (their output tiles side by side): the same n_in, at most two
 // types with the first type's weights first and only the pairs the kernel is
 // built for (one type; Q4_K or Q5_K then Q6_K).
-// work (gemm_work_bytes): scratch of the K-sliced form (null or too small: one slice)
+// work (gemm_work_bytes, gemm_plan.h): scratch of the K-sliced form (null or too small: one slice)
 // ks_out: when given, a K split leaves its ks_out slices of [M][sum of N]
 // partials in work for the caller to reduce (ks_out 1: y written directly)
 bool gemm_segs_supported(const WeightView *w, uint32_t nseg);
-size_t gemm_work_bytes(uint32_t M, const uint32_t *N, const uint32_t *type, uint32_t nseg, uint32_t K, int prec);
 hipError_t launch_gemm_segs(const WeightView *w, float *const *y, const uint32_t *ldy, uint32_t nseg,
                             const uint8_t *planes, uint32_t M, int prec, hipStream_t s, bool accum = false,
                             float *work = nullptr, size_t work_bytes = 0, uint32_t *ks_out = nullptr);

@@ -27,6 +27,7 @@
 // replayed for every token; a greedy generation loop runs as back-to-back
 // graph launches with no host round trip.
 #include "dn_dev.h"
+#include "gemm_plan.h"
 #include "lrs_internal.h"
 #include "pack_dev.h"
 #include "quant_dev.h"
@@ -36,6 +37,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <set>
 #include <string>
 #include <strings.h>
 #include <vector>
@@ -1274,18 +1276,17 @@ static bool prefill_capable(const lrs_model *m) {
     return true;
 }
 
-// scratch of the K-sliced GEMMs of a prompt block
+// scratch of the K-sliced GEMMs of a prompt block: of any number of tokens, for
+// each set of weights that the block may launch together or alone
 static size_t prefill_work_bytes(const lrs_model *m) {
-    size_t most = 0;
+    std::set<std::vector<uint32_t>> sets;  // {n_in, rows and type of each}
     auto need = [&](std::initializer_list<const lrs_weight *> ws) {
-        uint32_t N[3], t[3], n = 0;
+        std::vector<uint32_t> all = {(*ws.begin())->v.n_in};
         for (const lrs_weight *w : ws) {
-            N[n] = w->v.n_out;
-            t[n] = w->v.type;
-            most = std::max(most, gemm_work_bytes(PREFILL_BLOCK, N + n, t + n, 1, w->v.n_in, 3));
-            n++;
+            all.insert(all.end(), {w->v.n_out, w->v.type});
+            sets.insert({w->v.n_in, w->v.n_out, w->v.type});
         }
-        most = std::max(most, gemm_work_bytes(PREFILL_BLOCK, N, t, n, (*ws.begin())->v.n_in, 3));
+        sets.insert(all);
     };
     for (const DevLayer &L : m->layers) {
         need({L.gate, L.up});
@@ -1298,7 +1299,13 @@ static size_t prefill_work_bytes(const lrs_model *m) {
             need({L.o});
         }
     }
-    return std::max<size_t>(most, 256);
+    size_t most = 256;
+    for (const std::vector<uint32_t> &s : sets) {
+        uint32_t N[3], t[3], n = 0;
+        for (size_t i = 1; i < s.size(); i += 2, n++) N[n] = s[i], t[n] = s[i + 1];
+        most = std::max(most, gemm_work_most(PREFILL_BLOCK, N, t, n, s[0], 3));
+    }
+    return most;
 }
 
 static int ensure_prefill(lrs_model *m) {
