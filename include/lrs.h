@@ -165,6 +165,7 @@ int lrs_matvec_q8_0_actq_dev(lrs_ctx *ctx, const lrs_weight *w, const float *x_d
  * must match the f32 forward (observed 2e-7 to 5e-7 relative L2).  An
  * activation has 22 bits down to 2^-17 of the largest of its 256 columns and an
  * absolute 2^-40 of that largest below.
+ * A call's sums, and so its bits, depend on its sizes and types alone.
  * Weights: Q4_K, Q5_K, Q6_K, Q8_0; n_in a multiple of 256. */
 int lrs_gemm_dev(lrs_ctx *ctx, const lrs_weight *w, const float *a_dev, float *y_dev, uint32_t m,
                  int precision);

@@ -75,7 +75,7 @@ static std::mutex g_scratch_mu;
 static std::unordered_map<lrs_ctx *, lrs_ctx_scratch> g_scratch;
 
 namespace lrs {
-static int ctx_scratch(lrs_ctx *ctx, size_t bytes, void **p) {
+static int ctx_scratch(lrs_ctx *ctx, size_t bytes, void **p, size_t *have = nullptr) {
     std::lock_guard<std::mutex> lk(g_scratch_mu);
     lrs_ctx_scratch &s = g_scratch[ctx];
     if (s.n < bytes) {
@@ -102,6 +102,7 @@ static int ctx_scratch(lrs_ctx *ctx, size_t bytes, void **p) {
         s.n = n;
     }
     *p = s.p;
+    if (have) *have = s.n;
     return LRS_OK;
 }
 // the scratch if it can be had without an error: null where growing it is
@@ -476,9 +477,9 @@ int lrs_matvec_f32(lrs_ctx *ctx, const lrs_weight *w, const float *x, float *y, 
     return LRS_OK;
 }
 
-// the input packed into context scratch, then the GEMM (its K-slice partials
-// behind the packed input, where the scratch holds them or may grow: else one
-// slice)
+// the input packed into context scratch, then the GEMM with its K slices'
+// partial sums behind it: all of them where the scratch holds that or may grow,
+// else as many as there is room for
 static int gemm_run(lrs_ctx *ctx, const WeightView *wv, float *const *y, const uint32_t *ldy, uint32_t n_w,
                     const float *a_dev, uint32_t m, int precision) {
     const size_t ab = gemm_planes_bytes(m, wv[0].n_in, precision);
@@ -486,12 +487,12 @@ static int gemm_run(lrs_ctx *ctx, const WeightView *wv, float *const *y, const u
     for (uint32_t i = 0; i < n_w; i++) types[i] = wv[i].type;
     const size_t wb = gemm_work_bytes(m, ldy, types, n_w, wv[0].n_in, precision);
     void *buf = ctx_scratch_or_null(ctx, ab + wb);
-    const bool work = buf && wb;
+    size_t have = ab + wb;
     if (!buf)
-        if (int rc_ = ctx_scratch(ctx, ab, &buf)) return rc_;
+        if (int rc_ = ctx_scratch(ctx, ab, &buf, &have)) return rc_;
     LRS_HIP(launch_gemm_pack(a_dev, m, wv[0].n_in, precision, (uint8_t *)buf, ctx->stream));
     LRS_HIP(launch_gemm_segs(wv, y, ldy, n_w, (const uint8_t *)buf, m, precision, ctx->stream, false,
-                             work ? (float *)((char *)buf + ab) : nullptr, work ? wb : 0));
+                             (float *)((char *)buf + ab), have - ab));
     return LRS_OK;
 }
 

@@ -62,6 +62,8 @@ struct PgArgs {
     const uint8_t *a;  // planes (gemm_pack.h)
     PgSeg seg[PG_MAX_SEG];
     uint32_t nseg, nseg0, M, nsb, accum, nm, nn, ks, ntot;
+    uint32_t kz0, kn;  // the launch's slices of the ks
+    uint32_t cont;     // k_reduce_ks: y holds the sum of the slices before kz0
     float *part;
 };
 
@@ -577,8 +579,8 @@ static __device__ __forceinline__ void run(const PgArgs &g, const PgSeg &sg, uin
             for (int e = 0; e < 16; e++) {
                 const uint32_t m = 32 * (mb * MT + i) + 8 * (e >> 2) + 4 * hf + (e & 3);
                 if (m < g.M) {
-                    if (g.ks > 1) {
-                        g.part[((size_t)kz * g.M + m) * g.ntot + sg.noff + n] = tot[i][j][e];
+                    if (g.kn > 1) {
+                        g.part[((size_t)(kz - g.kz0) * g.M + m) * g.ntot + sg.noff + n] = tot[i][j][e];
                     } else {
                         float *o = sg.y + (size_t)m * sg.ldy + n;
                         *o = g.accum ? *o + tot[i][j][e] : tot[i][j][e];
@@ -596,12 +598,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     __shared__ __attribute__((aligned(16))) uint8_t As0[L::STAGE];
     __shared__ __attribute__((aligned(16))) uint8_t As1[L::STAGE];
     __shared__ __attribute__((aligned(16))) uint8_t Ss[2 * L::SUMS];
-    const uint32_t ntile = g.nm * g.nn * g.ks, per = (ntile + 7) / 8;
+    const uint32_t ntile = g.nm * g.nn * g.kn, per = (ntile + 7) / 8;
     const uint32_t t0 = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
     if ((blockIdx.x >> 3) >= per || t0 >= ntile) return;
     // row tiles of one weight tile run next to each other (they share its bytes
     // in an XCD's L2); the last segment, of the slower type, starts first
-    const uint32_t mb = t0 % g.nm, t = t0 / g.nm, nt = g.nn - 1 - t % g.nn, kz = t / g.nn;
+    const uint32_t mb = t0 % g.nm, t = t0 / g.nm, nt = g.nn - 1 - t % g.nn, kz = g.kz0 + t / g.nn;
     uint32_t si = 0;
 #pragma unroll
     for (int i = 1; i < PG_MAX_SEG; i++)
@@ -626,9 +628,10 @@ __global__ __launch_bounds__(256) void k_reduce_ks(PgArgs g) {
     typedef __attribute__((ext_vector_type(V))) float fv;
     const float *p = g.part + (size_t)m * g.ntot + sg.noff + n;
     const size_t st = (size_t)g.M * g.ntot;
-    fv v = *reinterpret_cast<const fv *>(p);
-    for (uint32_t z = 1; z < g.ks; z++) v += *reinterpret_cast<const fv *>(p + z * st);
     fv *o = reinterpret_cast<fv *>(sg.y + (size_t)m * sg.ldy + n);
+    fv v = *reinterpret_cast<const fv *>(p);
+    if (g.cont) v = *o + v;
+    for (uint32_t z = 1; z < g.kn; z++) v += *reinterpret_cast<const fv *>(p + z * st);
     *o = g.accum ? *o + v : v;
 }
 
@@ -700,7 +703,7 @@ hipError_t launch_gemm_segs(const WeightView *w, float *const *y, const uint32_t
         return hipErrorInvalidValue;
     uint32_t Ns[PG_MAX_SEG], ts[PG_MAX_SEG];
     for (uint32_t i = 0; i < nseg; i++) Ns[i] = w[i].n_out, ts[i] = w[i].type;
-    PgPlan p = pg_plan(M, Ns, ts, nseg, w[0].n_in / 256, prec, work != nullptr);
+    const PgPlan p = pg_plan(M, Ns, ts, nseg, w[0].n_in / 256, prec);
     PgArgs g = {};
     g.a = planes;
     g.nseg = nseg;
@@ -718,26 +721,39 @@ hipError_t launch_gemm_segs(const WeightView *w, float *const *y, const uint32_t
     }
     g.M = M;
     g.nsb = w[0].n_in / 256;
-    g.accum = accum ? 1u : 0u;
-    if (p.ks > 1 && (size_t)p.ks * M * ntot * sizeof(float) > work_bytes)
-        p = pg_plan(M, Ns, ts, nseg, g.nsb, prec, false);
+    // Where the scratch holds fewer partial sums than there are slices, the
+    // slices go by in rounds of as many as it holds (one: straight to y), added
+    // in the same order: a call's bits depend on its sizes and types alone.  A
+    // sum that starts from y, or that the caller reduces, has its scratch.
+    uint32_t fit = p.ks;
+    if (pg_bytes(p, M, Ns, nseg) > work_bytes) {
+        if (accum || ks_out) return hipErrorInvalidValue;
+        fit = (uint32_t)std::max<size_t>(1, work_bytes / ((size_t)M * ntot * sizeof(float)));
+    }
     g.nm = (M + 32 * p.mt - 1) / (32 * p.mt);
     g.nn = nt;
     g.ntot = ntot;
     g.ks = p.ks;
     g.part = work;
     const GemmFn fn = pick_gemm(w[0].type, w[nseg - 1].type, prec, p.mt);
-    const uint32_t grid = 8 * ((g.nm * g.nn * g.ks + 7) / 8);
-    hipLaunchKernelGGL(fn, dim3(grid), dim3(64 * PG_WAVES), 0, s, g);
-    if (ks_out) {
-        *ks_out = g.ks;  // the caller reduces the slices (launch_norm_rows)
-    } else if (g.ks > 1) {
-        if (v4)
-            hipLaunchKernelGGL((k_reduce_ks<4>), dim3((nmax + 1023) / 1024, M, nseg), dim3(256), 0, s, g);
-        else
-            hipLaunchKernelGGL((k_reduce_ks<1>), dim3((nmax + 255) / 256, M, nseg), dim3(256), 0, s, g);
+    for (; g.kz0 < g.ks; g.kz0 += g.kn) {
+        g.kn = std::min(fit, g.ks - g.kz0);
+        g.cont = g.kz0 ? 1u : 0u;
+        g.accum = accum || (g.kn == 1 && g.cont) ? 1u : 0u;
+        const uint32_t grid = 8 * ((g.nm * g.nn * g.kn + 7) / 8);
+        hipLaunchKernelGGL(fn, dim3(grid), dim3(64 * PG_WAVES), 0, s, g);
+        if (ks_out) {
+            *ks_out = g.ks;  // the caller reduces the slices (launch_norm_rows)
+        } else if (g.kn > 1) {
+            if (v4)
+                hipLaunchKernelGGL((k_reduce_ks<4>), dim3((nmax + 1023) / 1024, M, nseg), dim3(256), 0, s, g);
+            else
+                hipLaunchKernelGGL((k_reduce_ks<1>), dim3((nmax + 255) / 256, M, nseg), dim3(256), 0, s, g);
+        }
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
     }
-    return hipGetLastError();
+    return hipSuccess;
 }
 
 }  // namespace lrs

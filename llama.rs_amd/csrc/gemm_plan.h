@@ -37,9 +37,7 @@ inline double pg_unit(int prec, uint32_t mt, uint32_t fit, uint32_t n) {
 // The shape with the least expected time: the workgroups that a CU gets, and
 // for K slices the partial sums written and read back (at about 7 TB/s, most
 // of them in the memory-side cache) and the launch that adds them.
-// have_work: K slices may be used
-inline PgPlan pg_plan(uint32_t M, const uint32_t *N, const uint32_t *type, uint32_t nseg, uint32_t nsb, int prec,
-                      bool have_work) {
+inline PgPlan pg_plan(uint32_t M, const uint32_t *N, const uint32_t *type, uint32_t nseg, uint32_t nsb, int prec) {
     // precision 3: Q6_K and Q8_0 take a third product, Q5_K more unpacking;
     // precision 1: their unpacking shows where a workgroup has few row tiles.
     // While every workgroup runs at once the slowest counts, else the average
@@ -64,7 +62,7 @@ inline PgPlan pg_plan(uint32_t M, const uint32_t *N, const uint32_t *type, uint3
         const uint32_t tiles = pg_tiles(M, N, nseg, mt);
         const uint32_t fit = mt == (prec == 3 ? 2u : 4u) || (wide && !(prec == 1 && mt == 1)) ? 2 : 3;
         for (uint32_t ks = 1; ks <= nsb && ks <= 32; ks++) {
-            if (ks > 1 && (!have_work || tiles >= 2048 || M > 65535)) break;  // the reduce's grid has a y row per token
+            if (ks > 1 && (tiles >= 2048 || M > 65535)) break;  // the reduce's grid has a y row per token
             const uint32_t len = (nsb + ks - 1) / ks, per = (tiles * ks + 255) / 256;
             const double rel = per < fit ? slow : per == fit ? 0.5 * (slow + mean) : mean;
             double cost = (len + 0.5) * rel * pg_unit(prec, mt, fit, per);
@@ -88,7 +86,7 @@ inline size_t pg_bytes(const PgPlan &p, uint32_t M, const uint32_t *N, uint32_t 
 // scratch of the K-sliced form of one call
 inline size_t gemm_work_bytes(uint32_t M, const uint32_t *N, const uint32_t *type, uint32_t nseg, uint32_t K,
                               int prec) {
-    return pg_bytes(pg_plan(M, N, type, nseg, K / 256, prec, true), M, N, nseg);
+    return pg_bytes(pg_plan(M, N, type, nseg, K / 256, prec), M, N, nseg);
 }
 
 // ... of any call of up to M rows.  Fewer rows can take so many more slices

@@ -151,7 +151,8 @@ size_t gemm_planes_bytes(uint32_t M, uint32_t K, int prec);
 // one launch (their output tiles side by side): the same n_in, at most two
 // types with the first type's weights first and only the pairs the kernel is
 // built for (one type; Q4_K or Q5_K then Q6_K).
-// work (gemm_work_bytes, gemm_plan.h): scratch of the K-sliced form (null or too small: one slice)
+// work (gemm_work_bytes, gemm_plan.h): scratch of the K-sliced form; where it is
+// smaller, or null, the slices go by in rounds (an error with accum or ks_out)
 // ks_out: when given, a K split leaves its ks_out slices of [M][sum of N]
 // partials in work for the caller to reduce (ks_out 1: y written directly)
 bool gemm_segs_supported(const WeightView *w, uint32_t nseg);

@@ -6,6 +6,8 @@ against the exact product of the same bf16-rounded operands (tolerance 1e-5
 relative L2: only the f32 summation order differs); precision 3 (f16 hi/lo
 activations) against the f32 operands themselves (tolerance 1e-4).
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -248,25 +250,39 @@ def test_dequant_into_any_float_address_is_exact(lrs, orc, ctx, t, n, k, shift):
     assert np.all(got[:shift] == 7.0) and np.all(got[shift + n * k:] == 7.0)
 
 
-def test_gemm_whose_partials_do_not_fit_the_scratch_runs_unsplit(lrs, orc):
-    """Inside a capture the scratch may not grow: where it holds the packed
-    input but not the K slices' partial sums the GEMM takes one slice (the same
-    sums in another order: 1e-6)."""
-    n_in, n_out, m = 1280, 2048, 64
-    with lrs.Context(0) as c:
-        small = lrs.Weight.upload(c, Q4_K, orc.gen_weight(Q4_K, 1, 16, n_in), n_in, 16)
-        w = lrs.Weight.upload(c, Q4_K, orc.gen_weight(Q4_K, 2, n_out, n_in, mode=1), n_in, n_out)
-        a = np.random.default_rng(5).standard_normal((m, n_in)).astype(np.float32)
-        small.gemm(a, precision=3)  # the scratch holds this input
-        ab, yb = c.alloc(a.nbytes), c.alloc(4 * m * n_out)
+@pytest.mark.parametrize("t", [Q4_K, Q8_0])
+@pytest.mark.parametrize("prec,rows", [(1, 512), (1, 1024), (3, 512), (3, 768)])
+def test_gemm_whose_partials_do_not_fit_the_scratch_gives_the_same_bits(lrs, orc, t, prec, rows):
+    """Inside a capture the scratch may not grow. Where it holds the packed
+    input (made by a call of `rows` tokens) but not the K slices' partial sums
+    (2 MB each, at least four), the slices go by in rounds: of one, straight to y
+    (512), or of the two that fit.  The same bits as a call whose partials fit,
+    single and grouped."""
+    n_in, n_out, m = 5120, 1024, 512
+    a = np.random.default_rng(5).standard_normal((rows, n_in)).astype(np.float32)
+    with lrs.Context(0) as c, lrs.Context(0) as free:
+        host = [orc.gen_weight(t, 2 + i, n, n_in, mode=1) for i, n in enumerate((n_out, 256))]
+        up = lambda x: [lrs.Weight.upload(x, t, h, n_in, n) for h, n in zip(host, (n_out, 256))]
+        ws, wf = up(c), up(free)
+        small = lrs.Weight.upload(c, t, orc.gen_weight(t, 1, 16, n_in), n_in, 16)
+        small.gemm(a, precision=prec)  # the scratch holds this input
+        ab = c.alloc(a.nbytes)
         ab.upload(a)
-        g = c.capture(lambda: w.gemm_dev(ab, yb, m, 3))
-        got = []
-        for _ in range(2):
-            yb.upload(np.zeros(m * n_out, np.float32))
+        ys = [c.alloc(4 * m * n_out), c.alloc(4 * m * n_out), c.alloc(4 * m * 256)]
+        wa = (C.c_void_p * 2)(*[w.h for w in ws])
+        ya = (C.c_void_p * 2)(ys[1].ptr, ys[2].ptr)
+
+        def calls():
+            ws[0].gemm_dev(ab, ys[0], m, prec)
+            lrs.check(lrs.lib.lrs_gemm_group_dev(c.h, wa, 2, ab.ptr, ya, m, prec))
+
+        g = c.capture(calls)
+        ref = [wf[0].gemm(a[:m], precision=prec)] + lrs.gemm_group(free, wf, a[:m], precision=prec)
+        for _ in range(3):
+            for y in ys:
+                y.upload(np.full(y.nbytes // 4, 7.0, np.float32))
             g.launch()
             c.sync()
-            got.append(yb.download(np.float32, m * n_out).reshape(m, n_out))
+            for y, r in zip(ys, ref):
+                assert np.array_equal(y.download(np.float32, r.size).reshape(r.shape), r)
         g.close()
-        assert np.array_equal(got[0], got[1])
-        assert rel_l2(got[0], w.gemm(a, precision=3)) < 1e-6
