@@ -120,8 +120,9 @@ int lrs_matvec_f32(lrs_ctx *ctx, const lrs_weight *w, const float *x, float *y,
 /* Same on device buffers, enqueued on the context stream (async).  Q8_0
  * weights and inputs of up to 4096 elements are packed by the matvec launch
  * itself (no scratch); wider single K-quant columns take a pack launch into
- * the context scratch first, and so do several columns where the scratch
- * holds their packs or may grow (else they are packed by the launch too). */
+ * the context scratch first, and so do several columns (its first size holds
+ * their packs, so they never make it grow; where there is none yet and a
+ * capture or a live graph forbids one, the launch packs them too). */
 int lrs_matvec_dev(lrs_ctx *ctx, const lrs_weight *w, const float *x_dev, float *y_dev,
                    uint32_t cols);
 

@@ -66,6 +66,12 @@ using namespace lrs;
 // (input pack, host-buffer staging, GEMM operand planes).  Graphs captured on
 // the context record its address, so while any of them is alive the buffer
 // must not move: growth is refused instead (lrs_ctx::live_graphs).
+// The first use allocates SCRATCH_MIN: the packed input of a short GEMM (32 rows
+// at precision 3: 136 bytes per 8 columns of a row, 3.8 MB at n_in 27648), which a
+// call inside a capture may be the first to need, and the packs of as many
+// matvec columns as a launch makes (at most 2.5 MB), so that those never make an
+// asynchronous call wait for a larger buffer.
+static constexpr size_t SCRATCH_MIN = 8u << 20;
 struct lrs_ctx_scratch {
     void *p = nullptr;
     size_t n = 0;
@@ -96,7 +102,7 @@ static int ctx_scratch(lrs_ctx *ctx, size_t bytes, void **p, size_t *have = null
             s.p = nullptr;
             s.n = 0;
         }
-        size_t n = bytes < (1u << 20) ? (1u << 20) : bytes;
+        size_t n = bytes < SCRATCH_MIN ? SCRATCH_MIN : bytes;
         hipError_t e = hipMalloc(&s.p, n);
         if (e != hipSuccess) return hip_fail(e, "hipMalloc(scratch)");
         s.n = n;

@@ -286,3 +286,25 @@ def test_gemm_whose_partials_do_not_fit_the_scratch_gives_the_same_bits(lrs, orc
             for y, r in zip(ys, ref):
                 assert np.array_equal(y.download(np.float32, r.size).reshape(r.shape), r)
         g.close()
+
+
+@pytest.mark.parametrize("prec", [1, 3])
+@pytest.mark.parametrize("m", [1, 3, 33])
+def test_short_gemm_first_made_inside_a_capture(lrs, orc, m, prec):
+    """Whatever call made the scratch, its first size holds a short GEMM's packed
+    input (whole tiles of 32 rows: 3.8 MB for 33 x 13824 at precision 3), so that
+    a capture needs no such call before it; the bits of an eager call."""
+    n_in, n_out = 13824, 256
+    a = np.random.default_rng(m).standard_normal((m, n_in)).astype(np.float32)
+    host = orc.gen_weight(Q4_K, 3, n_out, n_in, mode=1)
+    with lrs.Context(0) as c:
+        w = lrs.Weight.upload(c, Q4_K, host, n_in, n_out)
+        w.matvec(a[0])
+        ab, yb = c.alloc(a.nbytes), c.alloc(4 * m * n_out)
+        ab.upload(a)
+        g = c.capture(lambda: w.gemm_dev(ab, yb, m, prec))
+        g.launch()
+        c.sync()
+        got = yb.download(np.float32, m * n_out).reshape(m, n_out)
+        g.close()
+        assert np.array_equal(got, w.gemm(a, precision=prec))
