@@ -119,7 +119,7 @@ hipError_t launch_argmax_finish(const unsigned long long *keys, uint32_t n, uint
                                 uint32_t *out, uint32_t out_cap, hipStream_t s);
 // y[c] = W x[c] for cols columns: when matvec_packs_in_kernel, up to 8
 // columns per launch share each weight load.  With cols_pack
-// (matvec_cols_bytes; 0: none needed) several columns are packed by a launch
+// (matvec_cols_bytes; 0: it would not pay) several columns are packed by a launch
 // before; without it, and for one column, every workgroup packs its input
 // columns itself (`pack` unused, may be null).  Otherwise the staged form
 // below with `pack` (xpack_bytes of the weight)

@@ -1595,9 +1595,23 @@ static hipError_t launch_columns(WeightView w, const float *x, float *y, uint32_
     return hipSuccess;
 }
 
+// The packs' launch costs about 2 us; it does not pay where no launch can take
+// two packed columns (n_in 27648, 2 columns of a Q8_0 weight 38 us, with packs
+// that nothing read 41), and for two or four columns of few elements that one
+// launch of not many workgroups packs itself: Q4_K 1024 rows, in the kernel /
+// packed before, 2 columns of 256 4.4 / 6.5 us, of 1280 5.8 / 6.4, of 2048 7.1 /
+// 6.6; 4 columns of 256 6.4 / 6.6, of 512 7.1 / 7.0.  Three columns take the
+// kernel two launches (256: 7.6 / 6.8), 864 workgroups more than one round
+// (Q8_0 13824 x 256, 2 columns 14.0 / 10.7), and 432 workgroups pay for 1024
+// elements (Q4_K 13824 x 1024 6.8 / 6.5; of 512 6.2 / 6.4).
 size_t matvec_cols_bytes(WeightView w, uint32_t cols) {
-    if (cols < 2 || !matvec_packs_in_kernel(w, cols)) return 0;
-    return (size_t)min(cols, MQS_COLS) * xpack_bytes(pack_blocks(w.type, w.n_in));
+    const uint32_t nxb = pack_blocks(w.type, w.n_in);
+    if (cols < 2 || mqx_lds(nxb, 2) > MQX_LDS_MAX || !matvec_packs_in_kernel(w, cols)) return 0;
+    const MqGeom g = store_geom(w.type, w.n_in, w.n_out);
+    const uint32_t per = (uint32_t)(g.tg * g.tpw);
+    const uint32_t wgs = (ttiles(w.n_out) + per - 1) / per;
+    if (wgs <= 512 && (cols == 2 ? w.n_in * wgs <= 1536 * 256 && w.n_in <= 1536 : cols == 4 && w.n_in <= 256)) return 0;
+    return (size_t)min(cols, MQS_COLS) * xpack_bytes(nxb);
 }
 
 hipError_t launch_matvec(WeightView w, const float *x, float *y, uint32_t cols, void *pack,

@@ -479,12 +479,15 @@ def test_q8_actq_columns_and_errors(lrs, orc, ctx):
 
 
 @pytest.mark.parametrize("t,n_in,n_out", [(Q4_K, 5120, 40), (Q5_K, 1024, 33), (Q6_K, 11264, 17),
-                                          (Q8_0, 2080, 16), (Q4_K, 12288, 5)])
+                                          (Q8_0, 2080, 16), (Q4_K, 12288, 5), (Q8_0, 22176, 18),
+                                          (Q8_0, 22240, 18), (Q6_K, 27648, 5), (Q5_K, 256, 1040),
+                                          (Q8_0, 1536, 4096), (Q8_0, 1568, 33), (Q8_0, 768, 8224)])
 def test_matvec_columns_staged_packs(lrs, orc, ctx, t, n_in, n_out):
     """Launches of 2, 4 and 8 columns that are full, short of columns, or held
-    to fewer by the LDS their packs need (11264: 3 fit, 12288: 2), over more than
-    the 32 columns of one pack launch: each column exactly as alone, nothing
-    stored past the last."""
+    to fewer by the LDS their packs need (11264 to 22176: 2, 22240 and 27648: one,
+    packed in the kernel as are 2 columns of up to 1536 and 4 of 256 elements in
+    few workgroups), over more than the 32 columns of one pack launch: each
+    column exactly as alone, nothing stored past the last."""
     w = lrs.Weight.upload(ctx, t, orc.gen_weight(t, 3, n_out, n_in, mode=1), n_in, n_out)
     x = np.random.default_rng(n_in).standard_normal((37, n_in)).astype(np.float32)
     xb, yb = ctx.alloc(x.nbytes), ctx.alloc(4 * (37 * n_out + 16))
