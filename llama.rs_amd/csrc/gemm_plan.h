@@ -24,50 +24,65 @@ inline uint32_t pg_tiles(uint32_t M, const uint32_t *N, uint32_t nseg, uint32_t 
     return (M + 32 * mt - 1) / (32 * mt) * nn;
 }
 
-// us per super-block of n workgroups that share a CU, measured with Q4_K
-// weights at K = 5120: the first workgroups of a CU hide each other's waits.
-// `fit`: workgroups that fit a CU at once (by registers)
-inline double pg_unit(int prec, uint32_t mt, uint32_t fit, uint32_t n) {
-    static const double p3m1[3] = {2.5, 4.4, 6.6}, p3m2[2] = {3.6, 6.4};
-    static const double p1m1[3] = {2.0, 3.0, 4.2}, p1m2[3] = {2.7, 4.8, 6.4}, p1m4[2] = {4.4, 7.8};
-    const double *c = prec == 3 ? (mt == 1 ? p3m1 : p3m2) : mt == 1 ? p1m1 : mt == 2 ? p1m2 : p1m4;
-    return n / fit * c[fit - 1] + (n % fit ? c[n % fit - 1] : 0.0);
+// us per super-block of 1, 2, ... workgroups that share a CU (the first ones hide
+// each other's waits), as many as fit it by registers.  The bf16 form's, and
+// Q8_0's, are fitted to launches of every shape forced in turn on random weights:
+// matrices and groups from 2048 x 2048 to 2 x 27648 x 5120, 2 to 2048 rows, up to
+// 32 slices, weights from memory and from the cache, 38 000 launches.  Over them
+// the shape chosen in bf16 takes 1.0 % longer than the best (geometric mean; at
+// most 22 %), and with Q8_0 at precision 3 1.2 % (12 %).  Costs of Q4_K times a
+// factor per type took 3.7 % (51 %: Q4_K in bf16, 384 x 13824 x 5120 as one row
+// tile 116 us, as four 79) and 3.1 % (32 %).  The K-quants' at precision 3 (2 %)
+// are those factors: fitted costs took 0.5 % over these calls, but a prompt block
+// of 12 to 32 tokens, where the launch that adds the slices costs 5 us, was up to
+// 6 % slower.
+struct PgCost {
+    uint32_t fit;
+    double us[4];
+};
+inline PgCost pg_cost(int prec, uint32_t mt, uint32_t type) {
+    const int t = type == LRS_TYPE_Q4_K ? 0 : type == LRS_TYPE_Q5_K ? 1 : type == LRS_TYPE_Q6_K ? 2 : 3;
+    static const PgCost p3[2][4] = {
+        {{3, {2.5, 4.4, 6.6}}, {2, {3.0, 5.28}}, {2, {3.75, 6.6}}, {3, {3.8, 5.6, 9.4}}},
+        {{2, {3.6, 6.4}}, {2, {4.32, 7.68}}, {2, {5.4, 9.6}}, {2, {5.4, 8.8}}}};
+    static const PgCost p1[3][4] = {
+        {{4, {2.0, 3.3, 4.6, 6.5}}, {3, {2.4, 3.7, 5.3}}, {3, {2.4, 4.1, 6.0}}, {4, {2.8, 3.6, 5.2, 7.0}}},
+        {{3, {2.7, 4.5, 6.4}}, {2, {3.5, 5.0}}, {2, {3.4, 5.6}}, {3, {3.4, 4.8, 6.4}}},
+        {{2, {4.3, 6.5}}, {2, {4.6, 8.0}}, {2, {4.6, 8.1}}, {2, {4.7, 6.8}}}};
+    return prec == 3 ? p3[mt / 2][t] : p1[mt / 2][t];
 }
 
-// The shape with the least expected time: the workgroups that a CU gets, and
-// for K slices the partial sums written and read back (at about 7 TB/s, most
-// of them in the memory-side cache) and the launch that adds them.
+// The shape with the least expected time: the super-blocks of a workgroup (and
+// part of one to start it), times what they cost with the workgroups that a CU
+// gets; for K slices the partial sums written and read back (most of them in the
+// memory-side cache) and the launch that adds them.
 inline PgPlan pg_plan(uint32_t M, const uint32_t *N, const uint32_t *type, uint32_t nseg, uint32_t nsb, int prec) {
-    // precision 3: Q6_K and Q8_0 take a third product, Q5_K more unpacking;
-    // precision 1: their unpacking shows where a workgroup has few row tiles.
-    // While every workgroup runs at once the slowest counts, else the average
-    uint32_t ntot = 0;
-    bool wide = false;  // a type whose operands take more registers
-    for (uint32_t i = 0; i < nseg; i++) {
-        ntot += N[i];
-        wide = wide || type[i] == LRS_TYPE_Q6_K || type[i] == LRS_TYPE_Q5_K;
-    }
+    double ntot = 0;
+    for (uint32_t i = 0; i < nseg; i++) ntot += N[i];
     PgPlan best = {1, 1};
     double best_cost = 1e30;
     for (uint32_t mt = 1; mt <= (prec == 3 ? 2u : 4u); mt *= 2) {
         if (mt > 1 && M <= 16 * mt) break;
-        double slow = 1.0, mean = 0.0;
-        for (uint32_t i = 0; i < nseg; i++) {
-            const double rel = type[i] == LRS_TYPE_Q4_K ? 1.0
-                               : prec == 1       ? (mt == 4 ? 1.05 : 1.25)
-                                                 : type[i] == LRS_TYPE_Q5_K ? 1.2 : 1.5;
-            slow = std::max(slow, rel);
-            mean += rel * N[i] / ntot;
-        }
         const uint32_t tiles = pg_tiles(M, N, nseg, mt);
-        const uint32_t fit = mt == (prec == 3 ? 2u : 4u) || (wide && !(prec == 1 && mt == 1)) ? 2 : 3;
+        // a launch of two types is compiled for the larger's registers
+        uint32_t fit = 4;
+        for (uint32_t i = 0; i < nseg; i++) fit = std::min(fit, pg_cost(prec, mt, type[i]).fit);
         for (uint32_t ks = 1; ks <= nsb && ks <= 32; ks++) {
             if (ks > 1 && (tiles >= 2048 || M > 65535)) break;  // the reduce's grid has a y row per token
             const uint32_t len = (nsb + ks - 1) / ks, per = (tiles * ks + 255) / 256;
-            const double rel = per < fit ? slow : per == fit ? 0.5 * (slow + mean) : mean;
-            double cost = (len + 0.5) * rel * pg_unit(prec, mt, fit, per);
-            if (ks > 1) cost += 5.0 + (2.0 * ks + 1) * M * ntot * 4.0 / 7e6;
-            if (cost < best_cost * 0.98) {
+            // while every workgroup runs at once the slowest type counts, else the average
+            double slow = 0.0, mean = 0.0;
+            for (uint32_t i = 0; i < nseg; i++) {
+                const PgCost c = pg_cost(prec, mt, type[i]);
+                const double u = per / fit * c.us[fit - 1] + (per % fit ? c.us[per % fit - 1] : 0.0);
+                slow = std::max(slow, u);
+                mean += u * N[i] / ntot;
+            }
+            const double u = per < fit ? slow : per == fit ? 0.5 * (slow + mean) : mean;
+            const double moved = (2.0 * ks + 1) * M * ntot * 4.0;
+            double cost = (len + (prec == 3 ? 0.5 : 0.3)) * u;
+            if (ks > 1) cost += prec == 3 ? 5.0 + moved / 7e6 : 1.0 + 0.2 * ks + moved / 8e6;
+            if (cost < best_cost * 0.98) {  // fewer row tiles and slices where it is close
                 best_cost = cost;
                 best = {mt, ks};
             }

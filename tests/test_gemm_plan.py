@@ -16,6 +16,10 @@ using namespace lrs;
 extern "C" size_t work(uint32_t M, const uint32_t *N, const uint32_t *t, uint32_t n, uint32_t K, int prec) {
     return gemm_work_bytes(M, N, t, n, K, prec);
 }
+extern "C" uint32_t shape(uint32_t M, const uint32_t *N, const uint32_t *t, uint32_t n, uint32_t K, int prec) {
+    const PgPlan p = pg_plan(M, N, t, n, K / 256, prec);
+    return p.mt << 16 | p.ks;
+}
 extern "C" size_t most(uint32_t M, const uint32_t *N, const uint32_t *t, uint32_t n, uint32_t K, int prec) {
     return gemm_work_most(M, N, t, n, K, prec);
 }
@@ -32,6 +36,7 @@ def plan(tmp_path_factory):
     lib = C.CDLL(str(so))
     for f in (lib.work, lib.most):
         f.restype = C.c_size_t
+    for f in (lib.work, lib.most, lib.shape):
         f.argtypes = [C.c_uint32, C.c_void_p, C.c_void_p, C.c_uint32, C.c_uint32, C.c_int]
     return lib
 
@@ -58,3 +63,24 @@ def test_scratch_of_a_block_covers_every_shorter_one(plan, k, ns, ts, prec):
     n, t, c = args(ns, ts)
     most = plan.most(BLOCK, n, t, c, k, prec)
     assert all(plan.work(m, n, t, c, k, prec) <= most for m in range(1, BLOCK + 1))
+
+
+# bf16 Q4_K over 13824 x 5120: one row tile without a split takes 116 us at 384
+# rows and 118 at 448, where four take 79 and 91
+@pytest.mark.parametrize("m", [289, 320, 352, 378, 384, 385, 400, 416, 448, 512, 1024, 2048])
+def test_bf16_q4_k_takes_several_row_tiles(plan, m):
+    n, t, c = args((13824,), (Q4_K,))
+    assert plan.shape(m, n, t, c, 5120, 1) >> 16 > 1
+
+
+@pytest.mark.parametrize("k,ns,ts", SETS)
+@pytest.mark.parametrize("prec", [1, 3])
+@pytest.mark.parametrize("m", [1, 31, 32, 33, 64, 65, 512, 4096, 65535, 65536, 1 << 20])
+def test_shapes_are_launchable(plan, k, ns, ts, prec, m):
+    """Row tiles that the kernel is built for, not more slices than super-blocks,
+    and none past the reduce's grid."""
+    n, t, c = args(ns, ts)
+    s = plan.shape(m, n, t, c, k, prec)
+    mt, ks = s >> 16, s & 0xFFFF
+    assert mt in ((1, 2) if prec == 3 else (1, 2, 4)) and 1 <= ks <= min(32, k // 256)
+    assert m <= 65535 or ks == 1
