@@ -59,12 +59,14 @@ struct PgSeg {
     uint32_t N, ldy, nt0, noff;
 };
 struct PgArgs {
+    // what a workgroup needs to find its tile, in one 64-byte line (spread over
+    // two, a short launch starts 0.3 us later)
     const uint8_t *a;  // planes (gemm_pack.h)
-    PgSeg seg[PG_MAX_SEG];
-    uint32_t nseg, nseg0, M, nsb, accum, nm, nn, ks, ntot;
-    uint32_t kz0, kn;  // the launch's slices of the ks
-    uint32_t cont;     // k_reduce_ks: y holds the sum of the slices before kz0
     float *part;
+    uint32_t nm, nn, ks, kz0, kn;  // kz0, kn: the launch's slices of the ks
+    uint32_t nseg, nseg0, nsb, M, ntot;
+    uint32_t accum, cont;  // cont: k_reduce_ks: y holds the sum of the slices before kz0
+    PgSeg seg[PG_MAX_SEG];
 };
 
 __device__ __forceinline__ f16x2 as_h2(uint32_t v) { return __builtin_bit_cast(f16x2, v); }
