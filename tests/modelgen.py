@@ -18,6 +18,11 @@ HD256R8 = dict(n_layer=2, n_embd=512, n_head=8, n_head_kv=1, head_dim=256, n_ff=
 KSPLIT = dict(n_layer=2, n_embd=512, n_head=16, n_head_kv=2, head_dim=128, n_ff=2048,
               vocab=1000, rope_dim=128, ctx=160, rms_eps=1e-6, freq_base=1e6)
 
+# a residual of more than 8192 elements, no multiple of it: the prompt block's row
+# norms take two passes a thread, with K slices of down to add or without
+WIDE = dict(n_layer=2, n_embd=8448, n_head=4, n_head_kv=1, head_dim=128, n_ff=2048, vocab=512,
+            rope_dim=128, ctx=256, rms_eps=1e-6, freq_base=1e6)
+
 Q4_K_M = dict(attn_q=Q4_K, attn_k=Q4_K, attn_v=Q6_K, attn_output=Q4_K, ffn_gate=Q4_K,
               ffn_up=Q4_K, ffn_down=Q6_K, output=Q6_K, token_embd=Q4_K)
 ALL_Q8_0 = {k: Q8_0 for k in Q4_K_M}

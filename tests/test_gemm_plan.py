@@ -84,3 +84,10 @@ def test_shapes_are_launchable(plan, k, ns, ts, prec, m):
     mt, ks = s >> 16, s & 0xFFFF
     assert mt in ((1, 2) if prec == 3 else (1, 2, 4)) and 1 <= ks <= min(32, k // 256)
     assert m <= 65535 or ks == 1
+
+
+# the edge that the prompt block tests on the GPU stand on either side of
+@pytest.mark.parametrize("k,ns,ts,m", [(2048, (8448,), (Q6_K,), 128)])
+def test_split_ends_where_the_block_tests_stand(plan, k, ns, ts, m):
+    n, t, c = args(ns, ts)
+    assert plan.shape(m, n, t, c, k, 3) & 0xFFFF > 1 and plan.shape(m + 1, n, t, c, k, 3) & 0xFFFF == 1

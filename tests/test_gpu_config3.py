@@ -1,5 +1,5 @@
-"""GPU parity at the benchmark's own shape (the
-Qwen2.5-32B-shaped Q4_K_M model) cut to two layers, against the CPU oracle's
+"""GPU parity at the benchmark's own shape (the Qwen2.5-32B-shaped Q4_K_M
+model) cut to two layers, against the CPU oracle's
 Model::forward (model.rs:99-266) on identical seeded weights.
 
 Every decode kernel instance the benchmark times runs here at its real
@@ -10,7 +10,7 @@ tiles x 6 K-slices, and the full 152064-row Q6_K head with the on-device
 greedy argmax; the batched prompt runs the full-width GEMMs.  The weights
 follow the benchmark distributions (f16 scales uniform in [1e-3, 1e-2]).
 
-Bars (BASELINE north star): logits within 1e-3 relative L2 of the oracle,
+Bars: logits within 1e-3 relative L2 of the oracle,
 identical greedy tokens for 32 steps, the head matvec within 1e-4."""
 import os
 

@@ -1,4 +1,4 @@
-"""GPU parity at the hybrid benchmark's own width (BASELINE config 4, the
+"""GPU parity at the hybrid benchmark's own width (the
 27B-scale qwen35-shaped Q4_K_M model) cut to one block of four layers
 (three gated delta-net layers, then one gated full-attention layer, as
 full_attn_interval 4 puts them), against the CPU oracle's hybrid forward on
@@ -16,7 +16,7 @@ block runs every full-width GEMM and the block delta-net kernels.  The
 output head of 248320 Q6_K rows runs as a plain matvec.  The weights follow
 the benchmark distributions (f16 scales uniform in [1e-3, 1e-2]).
 
-Bars (BASELINE north star): logits within 1e-3 relative L2 of the oracle,
+Bars: logits within 1e-3 relative L2 of the oracle,
 identical greedy tokens for 32 steps, the head matvec within 1e-4."""
 import os
 

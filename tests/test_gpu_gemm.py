@@ -1,7 +1,7 @@
 """GPU parity of the batched-prefill dequant-GEMM (lrs_gemm_dev) against the
 CPU oracle's dequant (bit-exact dequant.rs restatement) and float64 products.
 
-precision 1 (BASELINE config 5: bf16 operands, f32 accumulation) is checked
+precision 1 (bf16 operands, f32 accumulation) is checked
 against the exact product of the same bf16-rounded operands (tolerance 1e-5
 relative L2: only the f32 summation order differs); precision 3 (f16 hi/lo
 activations) against the f32 operands themselves (tolerance 1e-4).
@@ -255,7 +255,7 @@ def test_dequant_into_any_float_address_is_exact(lrs, orc, ctx, t, n, k, shift):
 def test_gemm_whose_partials_do_not_fit_the_scratch_gives_the_same_bits(lrs, orc, t, prec, rows):
     """Inside a capture the scratch may not grow. Where it holds the packed
     input (made by a call of `rows` tokens) but not the K slices' partial sums
-    (2 MB each, at least four), the slices go by in rounds: of one, straight to y
+    (2 MB each, at least three), the slices go by in rounds: of one, straight to y
     (512), or of the two that fit.  The same bits as a call whose partials fit,
     single and grouped."""
     n_in, n_out, m = 5120, 1024, 512

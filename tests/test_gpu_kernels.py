@@ -1,6 +1,6 @@
 """GPU parity of the kernel-level C ABI against the CPU oracle.
 
-Bars (BASELINE north star): dequant bit-exact; matvec within 1e-4 relative
+Bars: dequant bit-exact; matvec within 1e-4 relative
 L2 of dequant + sequential f32 dot (measured values are ~1e-7).
 """
 import json
@@ -316,7 +316,7 @@ def test_matvec_rejects_unsupported(lrs, ctx):
         w2.matvec(np.zeros(255, np.float32))
 
 
-# BASELINE configs 1 and 2 at full size, BASELINE distributions
+# the Q8_0 4096 x 4096 matvec and the 14B layer set at full size, with the benchmark distributions
 CFG1 = [("q8_0", Q8_0, 4096, 4096)]
 CFG2 = [("attn_q", Q4_K, 5120, 5120), ("attn_k", Q4_K, 5120, 1024),
         ("attn_v", Q6_K, 5120, 1024), ("attn_output", Q4_K, 5120, 5120),

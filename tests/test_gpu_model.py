@@ -1,7 +1,7 @@
 """GPU parity of the resident decode (GpuResidentDecode) against the CPU
 oracle's Model::forward on identical seeded weights.
 
-Bars (BASELINE north star): logits within 1e-3 relative L2 and an identical
+Bars: logits within 1e-3 relative L2 and an identical
 greedy argmax for 32 steps.  The oracle keeps K/V in f16 like the GPU cache
 (integration.rs:872-893 does the same); a second check compares against the
 pure f32-cache reference.  Q8_0 weights go through the int8-activation path
@@ -202,7 +202,7 @@ def test_decode_batch_matches_token_loop_and_reset_is_deterministic(lrs, orc, ct
 # Random-init models with the wide "mode 1" block scales amplify f16 K/V
 # rounding: for some seeds and lengths even the oracle with an f16 cache and
 # the oracle with an f32 cache differ by more than 1e-3.  The batched-prompt
-# cases therefore use the BASELINE weight distributions (mode 0), where the
+# cases therefore use the benchmark weight distributions (mode 0), where the
 # logits track the oracle to ~1e-5 and a 1e-3 miss would be a real defect.
 PREFILL_CASES = [
     # crosses the 512-token block boundary
@@ -255,11 +255,13 @@ def test_batched_prompt_matches_oracle(lrs, orc, ctx, name, cfg, mix, n, seed):
     assert gm.generate_greedy(short, 32).tolist() == modelgen.oracle_greedy(om3, short, 32)
 
 
-# KSPLIT: the K slices' reduce is its own launch below 192 rows and fused with
-# the norm from there on.  GQA5: positions split into shares of one chunk with
-# masked and empty ones (19 and 3 rows behind a context that is no multiple of
-# 32), and of several chunks with an uneven last one (321 rows)
-@pytest.mark.parametrize("cfg,pos0,n", [(modelgen.KSPLIT, 0, 191), (modelgen.KSPLIT, 0, 192),
+# KSPLIT: o and down leave eight K slices to the norm that follows.  WIDE: down
+# leaves three up to 128 rows, none from 129; o none.  GQA5: positions split into
+# shares of one chunk with masked and empty ones (19 and 3 rows behind a context
+# that is no multiple of 32), and of several chunks with an uneven last one (321
+# rows)
+@pytest.mark.parametrize("cfg,pos0,n", [(modelgen.KSPLIT, 0, 33), (modelgen.WIDE, 0, 128),
+                                        (modelgen.WIDE, 0, 129),
                                         (modelgen.GQA5, 333, 19), (modelgen.GQA5, 33, 3),
                                         (modelgen.GQA5, 101, 321)])
 def test_prompt_block_edges_match_oracle(lrs, orc, ctx, cfg, pos0, n):
