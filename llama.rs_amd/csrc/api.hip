@@ -67,8 +67,8 @@ using namespace lrs;
 // the context record its address, so while any of them is alive the buffer
 // must not move: growth is refused instead (lrs_ctx::live_graphs).
 // The first use allocates SCRATCH_MIN: the packed input of a short GEMM (32 rows
-// at precision 3: 136 bytes per 8 columns of a row, 3.8 MB at n_in 27648), which a
-// call inside a capture may be the first to need, and the packs of as many
+// at precision 3: 136 bytes a column, 3.8 MB at n_in 27648), which a call inside a
+// capture may be the first to need, and the packs of as many
 // matvec columns as a launch makes (at most 2.5 MB), so that those never make an
 // asynchronous call wait for a larger buffer.
 static constexpr size_t SCRATCH_MIN = 8u << 20;

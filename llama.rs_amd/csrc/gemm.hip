@@ -31,12 +31,15 @@
 // fill each other's waits (one workgroup of eight wavefronts in lockstep took
 // 98 against 63 us at 512 x 5120 x 5120).
 //
-// What bounds it: the matrix pipe and the vector pipe both near full (132
-// matrix operations of 32 clocks and about 610 vector operations of 4.8 clocks
-// per wavefront and super-block; up to four vector operations hide behind a
-// matrix one), and at 512 tokens the card's power: 1.85-1.95 GHz during the
-// gate / up launch, whose 1.1 PFLOP/s of products compare with 1.27 (bf16) and
-// 1.37 (f16) of a large library product.
+// What bounds it.  Where a CU has two workgroups at precision 3, the matrix and the
+// vector pipe together (132 matrix operations of 32 clocks and about 610 vector
+// operations of 4.8 clocks per wavefront and super-block; up to four vector
+// operations hide behind a matrix one) and the card's power: 32B gate / up of 512
+// tokens has the one busy for 60 % of the time and the other for 43 %, at 1.8 to
+// 1.9 GHz, and its 1.1 PFLOP/s of products compare with 1.27 (bf16) and 1.37 (f16)
+// of a large library product; down 57 and 52 %.  Fewer workgroups leave waits that
+// no pipe fills: the bf16 512 x 13824 x 5120 is 216 workgroups of four row tiles
+// on 256 CUs, 31 and 31 % busy at 2.2 GHz; the same at precision 3 48 and 35 %.
 #include "gemm_pack.h"
 #include "gemm_plan.h"
 #include "quant_dev.h"

@@ -106,7 +106,7 @@ inline size_t gemm_work_bytes(uint32_t M, const uint32_t *N, const uint32_t *typ
 
 // ... of any call of up to M rows.  Fewer rows can take so many more slices
 // that they need more (13824 x 4096 Q4_K, precision 3: 290 rows 64.1 MB, 512
-// rows 42.5), at no particular row counts, so each is looked at: 0.2 ms for 512.
+// rows none), at no particular row counts, so each is looked at: 0.2 ms for 512.
 inline size_t gemm_work_most(uint32_t M, const uint32_t *N, const uint32_t *type, uint32_t nseg, uint32_t K,
                              int prec) {
     size_t most = 0;
