@@ -148,8 +148,8 @@ def quantizer_like(t, n, k, seed):
 @pytest.mark.parametrize("m,n,k", [(1, 1, 256), (2, 255, 256), (32, 257, 768), (33, 16, 512),
                                    (64, 272, 1280), (65, 513, 256), (129, 31, 2816)])
 def test_gemm_edges_and_extreme_blocks(lrs, orc, ctx, t, m, n, k):
-    """Tile edges, quantizer-like blocks, and activations whose super-blocks
-    differ by 2^100, are all zero, or hold one outlier of 2^12."""
+    """Tile edges, quantizer-like blocks, and activations whose rows differ by
+    2^100, with a super-block of zeros and outliers of 2^12."""
     w = quantizer_like(t, n, k, m + n)
     deq = orc.dequant(t, w).reshape(n, k).astype(np.float64)
     rng = np.random.default_rng(n)
